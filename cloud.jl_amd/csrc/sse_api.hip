@@ -25,7 +25,8 @@
 
 namespace sse {
 hipError_t launch_generic_dispatch(const DevParams& p, const double* u, double* dudt, const RKStage& rk,
-                                   hipStream_t s, int which);
+                                   hipStream_t s, int which, const ErkTail& tail);
+size_t lds_time_derivative_ec(const DevParams& p);
 size_t lds_nodal_values_generic(const DevParams& p);
 size_t lds_nodal_values_mfma(const DevParams& p);
 size_t lds_time_derivative_generic(const DevParams& p);
@@ -793,7 +794,104 @@ int build_struct(sse_handle* h, const sse_desc* D) {
     return 0;
 }
 
-int launch(sse_handle* h, const double* u, double* dudt, const RKStage& rk, int which) {
+// Tables of the general entropy-conservative time derivative (k_time_derivative_ec).
+int build_pairs(sse_handle* h, const sse_desc* D) {
+    DevParams& P = h->P;
+    const int d = D->d, N_q = D->N_q, N_f = D->N_f, N_p = D->N_p;
+    auto S = [&](int i, int j, int m) { return D->S[i + (size_t)N_q * (j + (size_t)N_q * m)]; };
+    struct Entry {
+        int j;
+        double v[3];
+    };
+    // Volume pairs i < j of the union sparsity, by S_m[i, j] (the upper triangle). Node i's
+    // row subtracts the term and node j's adds it: in the list of j the entry is -S_m[i, j] (halved
+    // in the table: the flux contracts with half the vector).
+    // Pairs go by cyclic offset between their nodes, each to the node with the shorter list so
+    // far (on a tie, to the one at the start of the shorter cyclic way): the lists of a dense
+    // operator then have one offset per entry, and the atomic adds of neighbouring threads go
+    // to different rows.
+    std::vector<std::array<int, 3>> order;  // offset, start node, other node
+    for (int i = 0; i < N_q; ++i)
+        for (int j = i + 1; j < N_q; ++j) {
+            bool nz = false;
+            for (int m = 0; m < d; ++m) nz |= S(i, j, m) != 0.0;
+            if (!nz) continue;
+            if (2 * (j - i) <= N_q) order.push_back({j - i, i, j});
+            else order.push_back({N_q - (j - i), j, i});
+        }
+    std::sort(order.begin(), order.end());
+    std::vector<std::vector<Entry>> vol(N_q), fac(N_q), col(N_f);
+    auto entry = [&](int a, int b) {  // of node a's list, partner b
+        Entry e{b, {0.0, 0.0, 0.0}};
+        for (int m = 0; m < d; ++m) e.v[m] = 0.5 * (a < b ? S(a, b, m) : -S(b, a, m));
+        return e;
+    };
+    for (const auto& o : order) {
+        const int a = o[1], b = o[2];
+        if (P.det || vol[a].size() <= vol[b].size()) vol[a].push_back(entry(a, b));
+        else vol[b].push_back(entry(b, a));
+        if (P.det) vol[b].push_back(entry(b, a));
+    }
+    if (D->C_kind != SSE_C_NONE)
+        for (int i = 0; i < N_q; ++i)
+            for (int t = 0; t < N_f; ++t) {
+                const int j = (i + t) % N_f;  // neighbouring nodes' entries go to different facet nodes
+                const double c = D->C[i + (size_t)N_q * j];
+                if (c == 0.0) continue;
+                fac[i].push_back({j, {0.25 * c, 0.0, 0.0}});
+                if (P.det) col[j].push_back({i, {0.25 * c, 0.0, 0.0}});
+            }
+    auto table = [&](const std::vector<std::vector<Entry>>& lists, int nv, int& width, const int** idx,
+                     const double** val) {
+        width = 0;
+        for (const auto& l : lists) width = std::max(width, (int)l.size());
+        const size_t n = lists.size();
+        std::vector<int> ti((size_t)width * n, -1);
+        std::vector<double> tv((size_t)width * nv * n, 0.0);
+        for (size_t o = 0; o < n; ++o)
+            for (size_t w = 0; w < lists[o].size(); ++w) {
+                ti[w * n + o] = lists[o][w].j;
+                for (int m = 0; m < nv; ++m) tv[(w * nv + m) * n + o] = lists[o][w].v[m];
+            }
+        int r;
+        if ((r = upload(h, ti, idx)) || (r = upload(h, tv, val))) return r;
+        return 0;
+    };
+    int rc;
+    sse::PairLists& L = P.pairs;
+    if ((rc = table(vol, d, L.vol_w, &L.vol_j, &L.vol_s)) || (rc = table(fac, 1, L.fac_w, &L.fac_j, &L.fac_c)) ||
+        (rc = table(col, 1, L.col_w, &L.col_i, &L.col_c)))
+        return rc;
+    if (P.has_V) {  // [V; -R V]': column i < N_q is row i of V, column N_q + j is -(row j of R V)
+        std::vector<double> Q((size_t)N_p * (N_q + N_f), 0.0);
+        for (int c = 0; c < N_p; ++c) {
+            for (int i = 0; i < N_q; ++i) Q[c + (size_t)N_p * i] = D->V[i + (size_t)N_q * c];
+            for (int j = 0; j < N_f; ++j) {
+                double s = 0.0;
+                if (D->R_selection) {
+                    s = D->V[D->R_selection[j] - 1 + (size_t)N_q * c];
+                } else {
+                    for (int i = 0; i < N_q; ++i) s += D->R[j + (size_t)N_f * i] * D->V[i + (size_t)N_q * c];
+                }
+                Q[c + (size_t)N_p * (N_q + j)] = -s;
+            }
+        }
+        if ((rc = upload(h, Q, &P.Q))) return rc;
+    }
+    if (D->R_selection) {
+        std::vector<int> sel(N_f);
+        for (int j = 0; j < N_f; ++j) sel[j] = (int)(D->R_selection[j] - 1);
+        if ((rc = upload(h, sel, &P.sel))) return rc;
+    }
+    if (sse::lds_time_derivative_ec(P) > 160 * 1024) {
+        h->err = "element too large for the LDS-staged kernels";
+        return SSE_ERR_UNSUPPORTED;
+    }
+    return 0;
+}
+
+int launch(sse_handle* h, const double* u, double* dudt, const RKStage& rk, int which,
+           const sse::ErkTail& tail = sse::ErkTail{}) {
     if (h->use_struct) {
         hipError_t e = hipSuccess;
         if (which & 1) e = sse::launch_tensor(h->TP, u, dudt, rk, h->stream, 1);
@@ -805,11 +903,11 @@ int launch(sse_handle* h, const double* u, double* dudt, const RKStage& rk, int 
     if (h->use_std_tensor) {
         e = sse::launch_std_tensor(h->TP, 1, nullptr, 0, u, dudt, rk, h->stream, which);
     } else if (h->P.standard) {  // phase 1 without entropy projection, then the StandardForm kernels
-        e = (which & 1) ? sse::launch_generic_dispatch(h->P, u, dudt, rk, h->stream, 1) : hipSuccess;
+        e = (which & 1) ? sse::launch_generic_dispatch(h->P, u, dudt, rk, h->stream, 1, tail) : hipSuccess;
         if (e == hipSuccess) e = sse::launch_standard(h->P, dudt, rk, h->stream, which);
     } else {
         e = h->use_tensor ? sse::launch_tensor(h->TP, u, dudt, rk, h->stream, which)
-                          : sse::launch_generic_dispatch(h->P, u, dudt, rk, h->stream, which);
+                          : sse::launch_generic_dispatch(h->P, u, dudt, rk, h->stream, which, tail);
     }
     if (e != hipSuccess) return fail(h, SSE_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
     return 0;
@@ -968,11 +1066,15 @@ int create_handle(const sse_desc* D, int members, sse_handle** out) {
     } else if ((rc = union_rows(D->S, false, true, &P.S_ptr, &P.S_idx, &P.S_val))) {
         return cleanup_fail(rc);
     }
-    if (!P.standard) {  // flux work items: volume pairs i < j, then the nonzeros of C
+    P.ec = !P.standard && D->law == SSE_EULER && D->two_point_flux == SSE_TWO_POINT_EC;
+    P.det = !P.standard && D->deterministic ? 1 : 0;
+    if (!P.standard) {
         if (N_q >= 32768 || N_f >= 32768) {  // item_ij packs i | j << 16 into an int
             h->err = "too many nodes per element";
             return cleanup_fail(SSE_ERR_UNSUPPORTED);
         }
+    }
+    if (!P.standard && !P.ec) {  // flux work items: volume pairs i < j, then the nonzeros of C
         std::vector<int> ij;
         std::vector<double> val;
         for (int i = 0; i < N_q; ++i)
@@ -1020,7 +1122,6 @@ int create_handle(const sse_desc* D, int members, sse_handle** out) {
         if (!ij.empty() && ((rc = upload(h, ij, &P.item_ij)) || (rc = upload(h, val, &P.item_val))))
             return cleanup_fail(rc);
         // deterministic mode: each node's items, in item order (volume nodes, then facet nodes)
-        P.det = D->deterministic ? 1 : 0;
         if (P.det) {
             std::vector<std::vector<int>> own((size_t)N_q + N_f);
             for (int c = 0; c < (int)ij.size(); ++c) {
@@ -1088,9 +1189,10 @@ int create_handle(const sse_desc* D, int members, sse_handle** out) {
     }
     if (kenv && !strcmp(kenv, "generic")) h->use_tensor = h->use_std_tensor = false;
     if (!h->use_tensor) h->use_struct = false;
-    // the tensor kernels' weight-adjusted mass solve with a kept matrix per element
-    // (N_p^2 doubles each; up to 16 GiB) in place of V, W/J and V' (SSE_MASS_MATRICES=0: off)
-    if (h->use_tensor && P.has_V && (size_t)N_p * N_p * N_e * sizeof(double) <= ((size_t)16 << 30)) {
+    // the weight-adjusted mass solve with a kept matrix per element (N_p^2 doubles each; up to
+    // 16 GiB) in place of V, W/J and V' (SSE_MASS_MATRICES=0: off): tensor kernels and the
+    // general entropy-conservative time derivative
+    if ((h->use_tensor || P.ec) && P.has_V && (size_t)N_p * N_p * N_e * sizeof(double) <= ((size_t)16 << 30)) {
         const char* menv = getenv("SSE_MASS_MATRICES");
         if (!(menv && menv[0] == '0')) {
             double* Mw = nullptr;
@@ -1101,9 +1203,11 @@ int create_handle(const sse_desc* D, int members, sse_handle** out) {
                 h->err = std::string("weight-adjusted inverse: ") + hipGetErrorString(e);
                 return cleanup_fail(SSE_ERR_HIP);
             }
-            h->TP.Mw = Mw;
+            if (h->use_tensor) h->TP.Mw = Mw;
+            else P.Mw = Mw;
         }
     }
+    if (P.ec && !h->use_tensor && (rc = build_pairs(h, D))) return cleanup_fail(rc);
     if (members > 1 && !h->use_std_tensor) {
         h->err = "an ensemble of problems needs the compiled StandardForm shapes of scalar laws";
         return cleanup_fail(SSE_ERR_UNSUPPORTED);
@@ -1691,14 +1795,10 @@ int sse_rk_steps(sse_handle* h, double* u, double t0, double dt, int32_t nsteps,
 
 namespace {
 
-// out = base + sum_q c[q] K[idx[q]] over n entries (a Runge-Kutta stage combination;
-// out may alias base). The nonzero coefficients only, at most SSE_ERK_MAX_STAGES.
-struct ErkTerms {
-    int count;
-    int idx[SSE_ERK_MAX_STAGES];
-    double c[SSE_ERK_MAX_STAGES];
-};
+using sse::ErkTerms;
+static_assert(sizeof(ErkTerms::idx) / sizeof(int) == SSE_ERK_MAX_STAGES, "stage combination size");
 
+// out = base + sum_q c[q] K[idx[q]] over n entries (out may alias base)
 __global__ void __launch_bounds__(256) k_erk_combine(size_t n, const double* base, const double* __restrict__ K,
                                                      ErkTerms terms, double* out) {
     for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (size_t)gridDim.x * blockDim.x) {
@@ -1735,12 +1835,13 @@ int sse_erk_steps(sse_handle* h, double* u, double t0, double dt, int32_t nsteps
                 return fail(h, SSE_ERR_INVALID_ARGUMENT, "A must be strictly lower triangular (an explicit method)");
     const size_t n = state_size(h);
     int rc;
-    if (h->erk_stages < stages) {  // stage derivatives and the stage state (kept for later calls)
-        if ((rc = alloc(h, (size_t)(stages + 1) * n, &h->erk_k))) return rc;
+    if (h->erk_stages < stages) {  // stage derivatives and two stage states (kept for later calls)
+        if ((rc = alloc(h, (size_t)(stages + 2) * n, &h->erk_k))) return rc;
         h->erk_stages = stages;
     }
     double* K = h->erk_k;
     double* y = h->erk_k + (size_t)h->erk_stages * n;
+    double* y2 = y + n;
     double* ud = u;
     if (where == SSE_HOST) {
         if (!h->stage_u && ((rc = alloc(h, n, &h->stage_u)) || (rc = alloc(h, n, &h->stage_dudt)))) return rc;
@@ -1753,14 +1854,33 @@ int sse_erk_steps(sse_handle* h, double* u, double t0, double dt, int32_t nsteps
             fin.idx[fin.count] = i;
             fin.c[fin.count++] = dt * b[i];
         }
+    auto row = [&](int i) {  // the combination before stage i
+        ErkTerms st{};
+        for (int j = 0; j < i; ++j)
+            if (A[i * stages + j] != 0.0) {
+                st.idx[st.count] = j;
+                st.c[st.count++] = dt * A[i * stages + j];
+            }
+        return st;
+    };
+    // Nodal diagonal-E schemes (one kernel per residual, which reads its state directly): each
+    // residual also forms the next stage's state, in its epilogue. Two stage states take turns,
+    // because other workgroups still read the current one; a single-stage method would update
+    // u while it is read.
+    const bool fused = h->P.ec && !h->use_tensor && h->P.sel && !h->P.has_V && stages > 1;
     for (int step = 0; step < nsteps; ++step) {
+        if (fused) {
+            for (int i = 0; i < stages; ++i) {
+                const bool last = i + 1 == stages;
+                const double* yi = i == 0 ? ud : (i & 1 ? y : y2);
+                double* yo = last ? ud : (i & 1 ? y2 : y);
+                const sse::ErkTail tail{last ? fin : row(i + 1), i, n, ud, K, yo};
+                if ((rc = launch(h, yi, K + (size_t)i * n, RKStage{}, 3, tail))) return rc;
+            }
+            continue;
+        }
         for (int i = 0; i < stages; ++i) {
-            ErkTerms st{};
-            for (int j = 0; j < i; ++j)
-                if (A[i * stages + j] != 0.0) {
-                    st.idx[st.count] = j;
-                    st.c[st.count++] = dt * A[i * stages + j];
-                }
+            const ErkTerms st = row(i);
             const double* yi = ud;
             if (st.count) {
                 if ((rc = erk_combine(h, n, ud, K, st, y))) return rc;

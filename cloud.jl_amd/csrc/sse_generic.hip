@@ -10,7 +10,9 @@
 //   time_derivative  src/Solvers/flux_differencing_form.jl:294-347
 //   mass solve (WA)  src/Solvers/mass_matrix.jl:185-196
 //
-// The time derivative evaluates every two-point flux once: the interface fluxes,
+// The time derivative here serves linear advection and the conservative two-point flux; Euler
+// with the entropy-conservative flux runs k_time_derivative_ec (sse_generic_ec.hip). It
+// evaluates every two-point flux once: the interface fluxes,
 // the volume pairs i < j of the Hadamard sum and the facet-correction pairs form
 // one flat list of work items shared evenly by the workgroup's threads (dense
 // multidimensional operators have N_q (N_q - 1) / 2 volume and N_q N_f facet
@@ -410,12 +412,20 @@ size_t lds_time_derivative_generic(const DevParams& p) {
 }
 
 hipError_t launch_nodal_values_mfma(const DevParams& p, const double* u, hipStream_t s);
+hipError_t launch_time_derivative_ec(const DevParams& p, const double* u, double* dudt, const RKStage& rk,
+                                     const ErkTail& tail, hipStream_t s);
 
 template <int D, int LAW>
 hipError_t launch_generic(const DevParams& p, const double* u, double* dudt, const RKStage& rk, hipStream_t s,
-                          int which /* bit 0: phase 1, bit 1: phase 2 */) {
+                          int which /* bit 0: phase 1, bit 1: phase 2 */, const ErkTail& tail) {
     dim3 grid(p.N_e), block(256);
-    if ((which & 1) && p.mfma) {
+    // nodal diagonal-E schemes: u_q = u and u_f selects from it, so a whole residual reads u
+    // directly and needs no phase 1. Not inside an RK stage, whose epilogue updates u while
+    // other workgroups still read their neighbours' states.
+    const bool direct = which == 3 && !rk.active && p.ec && p.sel && !p.has_V;
+    if (direct) {
+        which = 2;
+    } else if ((which & 1) && p.mfma) {
         hipError_t err = launch_nodal_values_mfma(p, u, s);
         if (err != hipSuccess) return err;
     } else if (which & 1) {
@@ -424,6 +434,7 @@ hipError_t launch_generic(const DevParams& p, const double* u, double* dudt, con
         if (err != hipSuccess) return err;
     }
     if (which & 2) {
+        if (p.ec) return launch_time_derivative_ec(p, direct ? u : nullptr, dudt, rk, tail, s);
         if (p.det)
             hipLaunchKernelGGL((k_time_derivative_generic<D, LAW, true>), grid, block, lds_time_derivative_generic(p),
                                s, p, dudt, rk);
@@ -436,15 +447,15 @@ hipError_t launch_generic(const DevParams& p, const double* u, double* dudt, con
 }
 
 hipError_t launch_generic_dispatch(const DevParams& p, const double* u, double* dudt, const RKStage& rk,
-                                   hipStream_t s, int which) {
+                                   hipStream_t s, int which, const ErkTail& tail) {
     const bool euler = (p.N_c != 1);
     switch (p.d) {
-        case 1: return euler ? launch_generic<1, LAW_EULER>(p, u, dudt, rk, s, which)
-                             : launch_generic<1, LAW_ADVECTION>(p, u, dudt, rk, s, which);
-        case 2: return euler ? launch_generic<2, LAW_EULER>(p, u, dudt, rk, s, which)
-                             : launch_generic<2, LAW_ADVECTION>(p, u, dudt, rk, s, which);
-        case 3: return euler ? launch_generic<3, LAW_EULER>(p, u, dudt, rk, s, which)
-                             : launch_generic<3, LAW_ADVECTION>(p, u, dudt, rk, s, which);
+        case 1: return euler ? launch_generic<1, LAW_EULER>(p, u, dudt, rk, s, which, tail)
+                             : launch_generic<1, LAW_ADVECTION>(p, u, dudt, rk, s, which, tail);
+        case 2: return euler ? launch_generic<2, LAW_EULER>(p, u, dudt, rk, s, which, tail)
+                             : launch_generic<2, LAW_ADVECTION>(p, u, dudt, rk, s, which, tail);
+        case 3: return euler ? launch_generic<3, LAW_EULER>(p, u, dudt, rk, s, which, tail)
+                             : launch_generic<3, LAW_ADVECTION>(p, u, dudt, rk, s, which, tail);
         default: return hipErrorInvalidValue;
     }
 }

@@ -7,6 +7,17 @@
 
 namespace sse {
 
+// Work lists of the general entropy-conservative time derivative (Euler), one column of each
+// table per node (-1 pads). Volume lists: partner node and S_m / 2, m < d; a pair sits in the list
+// of one of its nodes (in both lists in deterministic mode). Facet lists: the rows of C
+// (facet node, C_ij / 4); columns of C (volume node, C_ij / 4) in deterministic mode only.
+struct PairLists {
+    int vol_w, fac_w, col_w;                   // longest lists
+    const int* vol_j; const double* vol_s;     // vol_w x N_q, vol_w x d x N_q
+    const int* fac_j; const double* fac_c;     // fac_w x N_q
+    const int* col_i; const double* col_c;     // col_w x N_f
+};
+
 // Everything a residual kernel reads, as device pointers. Operator tables are
 // compressed-row lists built once on the host from the dense reference
 // operators (nonzero entries only).
@@ -33,6 +44,14 @@ struct DevParams {
     // C rows: volume node i -> (facet node j, C_ij); C columns: facet node j -> (volume node i, C_ij)
     const int* Cr_ptr; const int* Cr_idx; const double* Cr_val;
     const int* Cc_ptr; const int* Cc_idx; const double* Cc_val;
+    // Euler with the entropy-conservative two-point flux, general kernel: its work lists, the
+    // stacked operator [V; -R V]' (N_p x (N_q + N_f) column-major), each element's kept
+    // V' diag(W / J_k) V (or null) and the volume node of each facet node (diagonal E, else null)
+    int ec;
+    PairLists pairs;
+    const double* Q;
+    const double* Mw;
+    const int* sel;
     // flux work items of the general time-derivative kernel: volume pairs i < j
     // (item_val = S_m[i,j], m < d) then facet-correction pairs (item_val[0] = C_ij);
     // item_ij = i | j << 16
@@ -108,6 +127,25 @@ struct RKStage {
     const double* dt_e;  // per-element time step (batched independent problems), or null for dt
     double* keep;        // line-structured kernel only: receives the state before the update, or null
     __device__ __forceinline__ double dt_of(size_t k) const { return dt_e ? dt_e[k] : dt; }
+};
+
+// A Runge-Kutta stage combination: base + sum_q c[q] K[idx[q]] over the nonzero coefficients
+// (at most 16 stages).
+struct ErkTerms {
+    int count;
+    int idx[16];
+    double c[16];
+};
+
+// The combination that follows a stage's residual, done in its epilogue: K holds the stage
+// derivatives (n values each), `stage` is the one this residual writes. out == null: none.
+struct ErkTail {
+    ErkTerms terms;
+    int stage;
+    size_t n;
+    const double* base;
+    const double* K;
+    double* out;
 };
 
 }  // namespace sse

@@ -45,44 +45,14 @@ template <int D>
 struct Physics<D, LAW_EULER> {
     static constexpr int NC = D + 2;
 
-    // entropy-conservative two-point flux of Ranocha (tensor form)
+    // ConservativeFlux: the average of the physical fluxes (tensor form). The entropy-conservative
+    // flux of Ranocha is only evaluated contracted, from hoisted states (ec_dot below)
     __device__ static void two_point(const LawParams& P, const double* uL, const double* uR, double* F) {
-        if (P.two_point_flux == 2) {  // ConservativeFlux: average of physical fluxes
-            double FL[D * NC], FR[D * NC];
-            physical_flux(P, uL, FL);
-            physical_flux(P, uR, FR);
+        double FL[D * NC], FR[D * NC];
+        physical_flux(P, uL, FL);
+        physical_flux(P, uR, FR);
 #pragma unroll
-            for (int i = 0; i < D * NC; ++i) F[i] = 0.5 * (FL[i] + FR[i]);
-            return;
-        }
-        double VL[D], VR[D];
-        double sL = 0.0, sR = 0.0, vv = 0.0;
-#pragma unroll
-        for (int m = 0; m < D; ++m) {
-            VL[m] = uL[m + 1] / uL[0];
-            VR[m] = uR[m + 1] / uR[0];
-        }
-#pragma unroll
-        for (int m = 0; m < D; ++m) {
-            sL += VL[m] * VL[m];
-            sR += VR[m] * VR[m];
-            vv += VL[m] * VR[m];
-        }
-        const double pL = P.gm1 * (uL[D + 1] - 0.5 * uL[0] * sL);
-        const double pR = P.gm1 * (uR[D + 1] - 0.5 * uR[0] * sR);
-        const double rho_avg = logmean(uL[0], uR[0]);
-        const double p_avg = 0.5 * (pL + pR);
-        const double Cc = 0.5 * vv + P.inv_gm1 * inv_logmean(uL[0] / pL, uR[0] / pR);
-#pragma unroll
-        for (int n = 0; n < D; ++n) {
-            const double vavg_n = 0.5 * (VL[n] + VR[n]);
-            const double f_rho = rho_avg * vavg_n;
-            F[n * NC + 0] = f_rho;
-#pragma unroll
-            for (int m = 0; m < D; ++m)
-                F[n * NC + m + 1] = f_rho * (0.5 * (VL[m] + VR[m])) + (m == n ? p_avg : 0.0);
-            F[n * NC + D + 1] = f_rho * Cc + 0.5 * (pL * VR[n] + pR * VL[n]);
-        }
+        for (int i = 0; i < D * NC; ++i) F[i] = 0.5 * (FL[i] + FR[i]);
     }
 
     __device__ static void physical_flux(const LawParams& P, const double* u, double* F) {

@@ -1,0 +1,95 @@
+"""The general entropy-conservative time derivative (runtime-sized elements) at the edges of its
+work split, against the CPU oracle: more nodes than a 256-thread workgroup has threads (one
+thread per node, 512 threads), few nodes (many threads per node), even and odd counts (the
+half-way cyclic offset), sparse and dense operators, the atomic and the deterministic variant,
+and the Runge-Kutta stage combination in its epilogue for one, two and three stages.
+
+Bars as in test_gpu_parity.py: 1e-12 for a residual, 1e-10 after Runge-Kutta steps; where the
+derivative itself amplifies rounding (257 nodes on a line) 8 eps times the largest row sum of
+|D| times the largest state, over the largest residual."""
+
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from sse import FluxDifferencingForm
+from sse.conservation_laws import (EntropyConservativeNumericalFlux, EulerEquations,
+                                   LaxFriedrichsNumericalFlux)
+from sse.geometry import make_spatial_discretization
+from sse.mesh import uniform_periodic_mesh
+from sse.reference_approximation import (ModalMulti, NodalMulti, NodalTensor,
+                                         ReferenceApproximationLine)
+from sse.solvers import MI355X, Solver, semidiscretize
+from sse.workloads import density_wave_3d_config, euler_3d_hex, euler_vortex_2d_modal
+
+pytestmark = pytest.mark.gpu
+
+
+def _line(approx, M):
+    law = EulerEquations(1, 1.4)
+
+    def ic(x, t=0.0):
+        rho = 1.0 + 0.3 * np.sin(np.pi * x[0])
+        return np.stack([rho, 0.4 * rho, 2.5 + 0.08 * rho], -1)
+
+    ref = ReferenceApproximationLine(approx)
+    sd = make_spatial_discretization(uniform_periodic_mesh(ref, (0.0, 2.0), M), ref)
+    form = FluxDifferencingForm(inviscid_numerical_flux=LaxFriedrichsNumericalFlux())
+    return law, sd, ic, form, semidiscretize(law, sd, ic, form, (0.0, 1.0))
+
+
+CASES = {
+    "line_257_nodes": lambda: _line(NodalTensor(256), 2),       # one thread per node, 512 threads
+    "line_modal_p2": lambda: _line(ModalMulti(2), 5),           # 3 modes: 85 threads per node
+    "tri_modal_p2": lambda: euler_vortex_2d_modal(M=3, p=2, approx=ModalMulti)[:5],
+    "tri_nodal_p5": lambda: euler_vortex_2d_modal(M=2, p=5, approx=NodalMulti)[:5],
+    "tet_modal_p2": lambda: density_wave_3d_config(M=1, p=2, approx=ModalMulti, ic_strength=0.2)[:5],
+    "tet_modal_p4": lambda: density_wave_3d_config(M=1, p=4, approx=ModalMulti, ic_strength=0.2)[:5],
+    "hex_p2": lambda: euler_3d_hex(M=2, p=2)[:5],
+    "hex_p4": lambda: euler_3d_hex(M=2, p=4)[:5],               # 275 nodes: 512 threads
+}
+
+
+def _rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+@pytest.mark.parametrize("det", [False, True], ids=["atomic", "deterministic"])
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_residual_at_the_edges_of_the_work_split(name, det):
+    import torch
+    from sse import semi_discrete_residual
+    from sse.time_integration import to_device, to_host
+    law, sd, _, form, ode = CASES[name]()
+    solver = Solver(law, sd, form, parallelism=MI355X(deterministic=det))
+    rng = np.random.default_rng(7)
+    u0 = np.asfortranarray(ode.u0 * (1.0 + 1e-3 * rng.standard_normal(ode.u0.shape)))
+    u = to_device(u0)
+    du = torch.empty_like(u)
+    semi_discrete_residual(du, u, solver)
+    torch.cuda.synchronize()
+    assert solver.describe().startswith("generic"), solver.describe()
+    expected = O.residual(solver.arrays, u0)
+    ref = sd.reference_approximation
+    rows = max(np.abs(np.asarray(Dm)).sum(1).max() for Dm in ref.D) / sd.geometric_factors.J_q.min()
+    bar = max(1e-12, 8 * np.finfo(float).eps * rows * np.abs(u0).max() / np.abs(expected).max())
+    if not name.startswith("line_257"):
+        bar = 1e-12
+    assert _rel(to_host(du), expected) <= bar
+
+
+@pytest.mark.parametrize("stages", [1, 2, 3])
+def test_stage_combination_in_the_epilogue(stages):
+    from types import SimpleNamespace
+
+    from sse.time_integration import erk_steps, to_device, to_host
+    # forward Euler, Heun, and a third-order tableau whose second row skips the first stage
+    A = {1: [[0.0]], 2: [[0, 0], [1, 0]], 3: [[0, 0, 0], [0.5, 0, 0], [0, 0.75, 0]]}[stages]
+    b = {1: [1.0], 2: [0.5, 0.5], 3: [2 / 9, 3 / 9, 4 / 9]}[stages]
+    alg = SimpleNamespace(A=np.array(A, dtype=float), b=np.array(b))
+    law, sd, _, form, ode = euler_3d_hex(M=2, p=2)[:5]
+    solver = Solver(law, sd, FluxDifferencingForm(inviscid_numerical_flux=EntropyConservativeNumericalFlux()))
+    u = to_device(ode.u0)
+    erk_steps(solver, u, 1e-3, 3, alg)
+    ref = O.erk_steps(solver.arrays, ode.u0, 1e-3, 3, alg.A, alg.b)
+    assert _rel(to_host(u), ref) <= 1e-10
