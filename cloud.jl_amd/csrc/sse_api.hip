@@ -55,7 +55,7 @@ bool struct_config(int elem, int P, StructConfig* c);
 int struct_occupancy(int elem, int P);
 hipError_t launch_struct(const TensorParams& tp, const StructTables& st, double* dudt, const RKStage& rk,
                          hipStream_t s, int n_blocks);
-size_t std_tensor_config(int elem, int P);
+bool std_tensor_config(int elem, int P);
 size_t vjp_tensor_config(int elem, int P);
 hipError_t launch_vjp_tensor(const TensorParams& tp, const StructTables& st, const double* u, const double* ybar,
                              double* ubar, double* rbar, double* fbar, double* fbar_ext, double* lam_partial,
@@ -63,7 +63,8 @@ hipError_t launch_vjp_tensor(const TensorParams& tp, const StructTables& st, con
                              double* in_store, hipStream_t s);
 hipError_t launch_vjp_sum(const double* lam_partial, int n, double* lam_out, double lam_scale, int accumulate,
                           hipStream_t s);
-hipError_t collapse_metric(double* Lam, const double* c, int NQ, int D, int N_e, hipStream_t s);
+hipError_t collapse_metric(double* Lam, const double* c, const double* W, const double* Jq, double* WoJ, double h,
+                           int NQ, int D, int N_e, hipStream_t s);
 hipError_t launch_std_tensor(const TensorParams& tp, int R, const double* b_member, int tangent, const double* u,
                              double* dudt, const RKStage& rk, hipStream_t s, int which);
 }  // namespace sse
@@ -534,6 +535,122 @@ int build_tensor(sse_handle* h, const sse_desc* D) {
     return 0;
 }
 
+// Stage-1 tables of the line-by-line sum factorisation (LineTables), from the warped-product
+// factors of V
+int upload_lines(sse_handle* h, const sse_desc* D, sse::LineTables* lt) {
+    const int P = D->V_p, n1 = P + 1;
+    const bool tet = D->d == 3;
+    struct Lane {
+        int b1, b2, off, lim;  // lim: last b of the line
+    };
+    std::vector<Lane> lanes;
+    int off = 0;
+    for (int b1 = 0; b1 <= P; ++b1)
+        for (int b2 = 0; b2 <= (tet ? P - b1 : 0); ++b2) {
+            const int lim = P - b1 - b2;
+            lanes.push_back({b1, b2, off, lim});
+            off += lim + 1;
+        }
+    std::stable_sort(lanes.begin(), lanes.end(), [](const Lane& a, const Lane& b) { return a.lim > b.lim; });
+    std::vector<int> mode;
+    for (const Lane& l : lanes) mode.push_back(l.off | l.b1 << 16 | l.b2 << 24);
+    std::vector<double> F1;
+    for (int b = 0; b <= P; ++b)
+        for (int a = 0; a < n1; ++a)
+            for (const Lane& l : lanes)
+                if (l.lim >= b)
+                    F1.push_back(tet ? D->V_C[a + n1 * (l.b1 + n1 * (l.b2 + n1 * b))] : D->V_B[a + n1 * (l.b1 + n1 * b)]);
+    int rc;
+    if ((rc = upload(h, F1, &lt->F1)) || (rc = upload(h, mode, &lt->mode))) return rc;
+    return 0;
+}
+
+// R as line ends and an interpolation on each face (FaceTables). For each face the direction
+// along which its rows of R factorise, R_f[j, (t, a)] = M[j, t] w[a]; structured = false when a
+// face has none (to 1e-12 of its largest entry).
+int upload_faces(sse_handle* h, const sse_desc* D, sse::FaceTables* ft, bool& structured) {
+    const int n1 = D->V_p + 1, d = D->d, nq = D->N_q, nf = D->N_f, nfac = D->N_fac, n2 = nq / n1;
+    structured = false;
+    if (nf != nfac * n2 || nfac > 4) return 0;
+    auto R = [&](int j, int i) { return D->R[j + (size_t)nf * i]; };
+    std::vector<double> w((size_t)nfac * n1, 0.0), Pf((size_t)nfac * n1 * n1, 0.0);
+    ft->general = 0;
+    std::vector<std::vector<std::pair<int, double>>> mrows(nf), mtrows(nf);
+    for (int f = 0; f < nfac; ++f) {
+        bool found = false;
+        for (int l = 0; l < d && !found; ++l) {
+            int st = 1;
+            for (int t = l + 1; t < d; ++t) st *= n1;
+            auto node = [&](int t, int a) { return (t / st) * st * n1 + a * st + t % st; };  // line t of direction l
+            int jm = 0, tm = 0;
+            double big = 0.0;  // the line with the largest entry gives w, scaled to sum 1
+            for (int j = 0; j < n2; ++j)
+                for (int t = 0; t < n2; ++t)
+                    for (int a = 0; a < n1; ++a)
+                        if (std::fabs(R(f * n2 + j, node(t, a))) > big) {
+                            big = std::fabs(R(f * n2 + j, node(t, a)));
+                            jm = j;
+                            tm = t;
+                        }
+            double sum = 0.0, sq = 0.0;
+            for (int a = 0; a < n1; ++a) sum += R(f * n2 + jm, node(tm, a));
+            if (big == 0.0 || std::fabs(sum) < 1e-8 * big) continue;
+            for (int a = 0; a < n1; ++a) {
+                w[(size_t)f * n1 + a] = R(f * n2 + jm, node(tm, a)) / sum;
+                sq += w[(size_t)f * n1 + a] * w[(size_t)f * n1 + a];
+            }
+            std::vector<double> M((size_t)n2 * n2, 0.0);
+            double worst = 0.0;
+            for (int j = 0; j < n2; ++j)
+                for (int t = 0; t < n2; ++t) {
+                    double m = 0.0;
+                    for (int a = 0; a < n1; ++a) m += R(f * n2 + j, node(t, a)) * w[(size_t)f * n1 + a];
+                    m /= sq;
+                    for (int a = 0; a < n1; ++a)
+                        worst = std::max(worst, std::fabs(R(f * n2 + j, node(t, a)) - m * w[(size_t)f * n1 + a]));
+                    M[(size_t)j * n2 + t] = m;
+                }
+            if (worst > 1e-12 * big) continue;
+            found = true;
+            ft->dir[f] = l;
+            // I, I x P or neither (to rounding: 1e-13 of the largest entry, which is about 1)
+            bool ident = true, kron = true;
+            for (int j = 0; j < n2; ++j)
+                for (int t = 0; t < n2; ++t) {
+                    const double m = M[(size_t)j * n2 + t];
+                    const double p = j / n1 == t / n1 ? M[(size_t)(j % n1) * n2 + t % n1] : 0.0;
+                    if (std::fabs(m - (j == t ? 1.0 : 0.0)) > 1e-13) ident = false;
+                    if (std::fabs(m - p) > 1e-13) kron = false;
+                }
+            ft->kind[f] = ident ? 0 : 1;
+            if (!ident && (!kron || d == 2)) ft->general = 1;
+            for (int a = 0; a < n1; ++a)
+                for (int b = 0; b < n1; ++b) Pf[((size_t)f * n1 + a) * n1 + b] = M[(size_t)a * n2 + b];
+            for (int j = 0; j < n2; ++j)
+                for (int t = 0; t < n2; ++t) {
+                    double m = M[(size_t)j * n2 + t];
+                    bool any = false;  // a zero block of R is no entry
+                    for (int a = 0; a < n1; ++a) any |= R(f * n2 + j, node(t, a)) != 0.0;
+                    if (!any) continue;
+                    if (std::fabs(m - 1.0) < 4e-16) m = 1.0;
+                    mrows[f * n2 + j].push_back({f * n2 + t, m});
+                    mtrows[f * n2 + t].push_back({f * n2 + j, m});
+                }
+        }
+        if (!found) return 0;
+    }
+    std::vector<int> mi, mti;
+    std::vector<double> mv, mtv;
+    ell(mrows, ft->m_w, mi, mv);
+    ell(mtrows, ft->mt_w, mti, mtv);
+    int rc;
+    if ((rc = upload(h, w, &ft->w)) || (rc = upload(h, Pf, &ft->P)) || (rc = upload(h, mi, &ft->m_idx)) || (rc = upload(h, mv, &ft->m_val)) ||
+        (rc = upload(h, mti, &ft->mt_idx)) || (rc = upload(h, mtv, &ft->mt_val)))
+        return rc;
+    structured = true;
+    return 0;
+}
+
 // Set up the compile-time-shaped StandardForm kernels of scalar linear laws
 // (ModalTensor Tri/Tet, weight-adjusted mass solve); returns 0 and leaves
 // use_std_tensor false when the discretisation is not one of the compiled shapes.
@@ -551,8 +668,7 @@ int build_std_tensor(sse_handle* h, const sse_desc* D) {
     const int nq = tet ? n1 * n1 * n1 : n1 * n1, nf = tet ? 4 * n1 * n1 : 3 * n1;
     const int np = tet ? n1 * (p + 2) * (p + 3) / 6 : n1 * (p + 2) / 2;
     if (D->N_q != nq || D->N_f != nf || D->N_p != np) return 0;
-    const size_t lds = sse::std_tensor_config(D->element, p);
-    if (lds == 0 || lds > 160 * 1024) return 0;
+    if (!sse::std_tensor_config(D->element, p)) return 0;
     {  // the dense V must be the product of the factors
         std::vector<double> Vw = warped_dense(D);
         if ((int)Vw.size() != nq * np) return 0;
@@ -568,31 +684,8 @@ int build_std_tensor(sse_handle* h, const sse_desc* D) {
     T.elem = D->element;
     T.P = p;
     T.variant = 0;
-    std::vector<std::vector<std::pair<int, double>>> rrows(nf), rtrows(nq);
-    for (int j = 0; j < nf; ++j)
-        for (int i = 0; i < nq; ++i) {
-            const double v = D->R[j + (size_t)nf * i];
-            if (v == 0.0) continue;
-            rrows[j].push_back({i, v});
-            rtrows[i].push_back({j, v});
-        }
-    std::vector<int> r_idx, rt_idx;
-    std::vector<double> r_val, rt_val;
-    ell(rrows, T.wr, r_idx, r_val);
-    ell(rtrows, T.wrt, rt_idx, rt_val);
-    // the kernels read ELL rows four entries at a time
-    auto pad4 = [](int& width, int rows, std::vector<int>& idx, std::vector<double>& val) {
-        const int w4 = (std::max(width, 1) + 3) / 4 * 4;
-        idx.resize((size_t)w4 * rows, -1);
-        val.resize((size_t)w4 * rows, 0.0);
-        width = w4;
-    };
-    pad4(T.wr, nf, r_idx, r_val);
-    pad4(T.wrt, nq, rt_idx, rt_val);
     std::vector<double> VA(D->V_A, D->V_A + (size_t)n1 * n1);
     std::vector<double> VB(D->V_B, D->V_B + (size_t)n1 * n1 * n1);
-    std::vector<double> VC;
-    if (tet) VC.assign(D->V_C, D->V_C + (size_t)n1 * n1 * n1 * n1);
     // D_m = sum_l diag(c_lm) D1_l along the lines of the tensor grid: D1_l row a
     // from the line through node a * stride_l (row sums of a derivative vanish),
     // c by least squares, then the whole of every D_m is checked against it
@@ -655,16 +748,20 @@ int build_std_tensor(sse_handle* h, const sse_desc* D) {
             }
     int rc;
     const double* c_dev = nullptr;
-    if ((rc = upload(h, r_idx, &T.r_idx)) || (rc = upload(h, r_val, &T.r_val)) || (rc = upload(h, rt_idx, &T.rt_idx)) ||
-        (rc = upload(h, rt_val, &T.rt_val)) || (rc = upload(h, VA, &T.VA)) || (rc = upload(h, VB, &T.VB)) ||
-        (rc = upload(h, D1, &T.D1)) || (rc = upload(h, c, &c_dev)))
+    bool structured = false;
+    if ((rc = upload_faces(h, D, &T.faces, structured))) return rc;
+    if (!structured) return 0;
+    if ((rc = upload(h, VA, &T.VA)) || (rc = upload(h, VB, &T.VB)) || (rc = upload(h, D1, &T.D1)) ||
+        (rc = upload(h, c, &c_dev)) || (rc = upload_lines(h, D, &T.lines)))
         return rc;
-    if (tet && (rc = upload(h, VC, &T.VC))) return rc;
-    // the kernels read Lt_ln = sum_m c_lm Lambda_mn in place of Lambda (this handle's copy)
-    hipError_t e = sse::collapse_metric(const_cast<double*>(P.Lam), c_dev, nq, d, P.N_e, nullptr);
+    // the kernels read h W sum_m c_lm Lambda_mn in place of Lambda (this handle's copy), and W / J
+    double* WoJ = nullptr;
+    if ((rc = alloc(h, (size_t)nq * P.N_e, &WoJ))) return rc;
+    T.WoJ = WoJ;
+    hipError_t e = sse::collapse_metric(const_cast<double*>(P.Lam), c_dev, P.W, P.Jq, WoJ, P.skew ? 0.5 : 1.0, nq, d,
+                                        P.N_e, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) return fail(h, SSE_ERR_HIP, std::string("metric set-up: ") + hipGetErrorString(e));
-    h->TP.base = h->P;
     T.xcd_remap = 1;
     h->use_std_tensor = true;
     return 0;
@@ -1164,30 +1261,34 @@ int create_handle(const sse_desc* D, int members, sse_handle** out) {
     }
     const size_t ens = (size_t)members;
     h->members = members;
-    if ((rc = alloc(h, (size_t)N_q * D->N_c * N_e * ens, &P.uq)) ||
-        (rc = alloc(h, (size_t)N_f * D->N_c * N_e * ens, &P.uf)) || (rc = alloc(h, 1, &P.status)))
+    if ((rc = alloc(h, (size_t)N_f * D->N_c * N_e * ens, &P.uf)) || (rc = alloc(h, 1, &P.status)))
         return cleanup_fail(rc);
     if (hipMemset(P.status, 0, sizeof(int)) != hipSuccess) {
         h->err = "hipMemset failed";
         return cleanup_fail(SSE_ERR_HIP);
     }
-    if (P.second_order &&
-        ((rc = alloc(h, (size_t)N_q * d * N_e * ens, &P.qq)) || (rc = alloc(h, (size_t)N_f * d * N_e * ens, &P.qf))))
-        return cleanup_fail(rc);
     if (sse::lds_time_derivative_generic(P) > 64 * 1024 || sse::lds_nodal_values_generic(P) > 64 * 1024 ||
         (P.standard && sse::lds_standard(P) > 64 * 1024)) {
         h->err = "element too large for the LDS-staged kernels";
         return cleanup_fail(SSE_ERR_UNSUPPORTED);
     }
-    if (!P.standard && (rc = build_tensor(h, D))) return cleanup_fail(rc);
-    if (P.standard && (rc = build_std_tensor(h, D))) return cleanup_fail(rc);
     const char* kenv = getenv("SSE_KERNELS");  // "generic", "tensor" (table-driven pairs) or unset
+    const bool only_generic = kenv && !strcmp(kenv, "generic");
+    if (P.standard && !only_generic && (rc = build_std_tensor(h, D))) return cleanup_fail(rc);
+    // intermediates of a residual: u_q and q_q at the volume nodes, in the compile-time-shaped
+    // StandardForm kernels only the modal q
+    if (!h->use_std_tensor && (rc = alloc(h, (size_t)N_q * D->N_c * N_e * ens, &P.uq))) return cleanup_fail(rc);
+    if (P.second_order && ((rc = alloc(h, (size_t)(h->use_std_tensor ? N_p : N_q) * d * N_e * ens, &P.qq)) ||
+                           (rc = alloc(h, (size_t)N_f * d * N_e * ens, &P.qf))))
+        return cleanup_fail(rc);
+    if (h->use_std_tensor) h->TP.base = P;
+    if (!P.standard && (rc = build_tensor(h, D))) return cleanup_fail(rc);
     if (!(kenv && (!strcmp(kenv, "generic") || !strcmp(kenv, "tensor"))) && (rc = build_struct(h, D)))
         return cleanup_fail(rc);
     if (const char* env = getenv("SSE_FORCE_GENERIC")) {
         if (env[0] == '1') h->use_tensor = false;
     }
-    if (kenv && !strcmp(kenv, "generic")) h->use_tensor = h->use_std_tensor = false;
+    if (only_generic) h->use_tensor = false;
     if (!h->use_tensor) h->use_struct = false;
     // the weight-adjusted mass solve with a kept matrix per element (N_p^2 doubles each; up to
     // 16 GiB) in place of V, W/J and V' (SSE_MASS_MATRICES=0: off): tensor kernels and the
@@ -2044,7 +2145,7 @@ void append(std::vector<T>& dst, const T* src, size_t n) {
 // that tangent pairs never straddle two launches)
 int ensemble_chunk(const sse_desc* D, int R) {
     const size_t per_lane =
-        sizeof(double) * (size_t)D->N_e * ((size_t)D->N_q + D->N_f + (size_t)D->d * (D->N_q + D->N_f));
+        sizeof(double) * (size_t)D->N_e * ((size_t)D->N_f + (size_t)D->d * (D->N_p + D->N_f));
     size_t cap = std::max<size_t>(2, ENSEMBLE_BUDGET / std::max<size_t>(per_lane, 1));
     if (const char* env = getenv("SSE_ENSEMBLE_CHUNK")) cap = std::max(2, atoi(env));  // smaller launches, for tests
     cap = std::min<size_t>(cap, 2 * (size_t)R);

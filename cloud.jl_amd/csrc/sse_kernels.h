@@ -87,6 +87,33 @@ struct DevParams {
     int* status;
 };
 
+// Stage-1 tables of the line-by-line sum factorisation (sse_lines.h):
+//   lanes m = (b1, b2) (Tri: b1) by falling number of modes; n(b) of them have a mode b
+//   F1: for each b, [a][m < n(b)]: C[a3, b1, b2, b3] with a = a3, b = b3 on the Tet, B[a2, b1, b2]
+//       with a = a2, b = b2 on the Tri
+//   mode: the first mode number of lane m (bits 0-15), its b1 (16-23) and b2 (24-31)
+struct LineTables {
+    const double* F1;
+    const int* mode;
+};
+
+// R on the tensor grid (sse_lines.h): every face is the end of the grid's lines in one direction,
+// R_f = M_f E_f with E_f[t] = sum_a w_f[a] x(line t, a) the end value of each line of that
+// direction and M_f the interpolation from the lines to the facet nodes. kind 0: M_f = I (the
+// facet nodes lie on the lines); kind 1: M_f = I x P_f, P_f (N1 x N1, row-major) acting on the
+// last index of the face, Tet only (general: the faces' M and M' as ELL rows, -1 pads with value 0; index
+// f N2 + t is line t of face f).
+struct FaceTables {
+    int dir[4];                                      // direction of the lines of each face
+    int kind[4];
+    int general;                                     // some M_f has neither form: use the ELL rows
+    const double* w;                                 // N_fac x N1
+    const double* P;                                 // N_fac x N1 x N1
+    int m_w, mt_w;                                   // row widths
+    const int* m_idx; const double* m_val;           // m_w x N_f
+    const int* mt_idx; const double* mt_val;         // mt_w x N_f
+};
+
 // Tables of the compile-time-shaped tensor-product kernels (Tri/Tet,
 // ModalTensor, Euler). Built once on the host from the reference operators.
 struct TensorParams {
@@ -110,6 +137,10 @@ struct TensorParams {
     const double* VC;
     const double* D1;    // StandardForm scalar kernels: 1D derivative matrix of each collapsed
                          // direction, d x N1 x N1 row-major (D_m = sum_l diag(c_lm) D1_l along lines)
+    LineTables lines;
+    FaceTables faces;
+    const double* WoJ;   // StandardForm scalar kernels: W / J, N_q x N_e (base.Lam then holds
+                         // h W sum_m c_lm Lambda_mn)
     const double* Mw;    // weight-adjusted inverse mass matrix of every element, V' diag(W / J_k) V
                          // (N_p x N_p column-major per element), or null: the kernels then apply
                          // V, W / J_k and V' by sum factorisation

@@ -1,0 +1,283 @@
+// sse_lines.h -- sum-factorised V, V' and line derivatives with a line of nodes per thread.
+//
+// A column (one variable of one element) is one LDS array of padded tensor-grid positions
+// X(a1, a2[, a3]). Every stage of V, V' and of a derivative along a collapsed direction acts
+// on lines of the grid: a thread reads its line's N1 values into registers, applies an
+// N1 x N1 matrix and writes the N1 results back in place. With one thread per output point
+// instead (SumFact of sse_tensor.h) each multiply-add reads one LDS value, which is what
+// bounded those kernels: a CU issues four times as many FP64 multiply-adds as LDS reads.
+// Here a line costs 2 N1 LDS accesses for N1^2 multiply-adds, and the matrices come through
+// the scalar cache where they are the same for all lanes:
+//   stage 3 (A[a1, b1]) and the derivatives D1_l: always;
+//   stage 2 (B[a2, b1, b2]): b1 is uniform over a wavefront (the wavefronts share out b1,
+//     the lanes are (column, a3));
+//   stage 1 (C[a3, b1, b2, b3]): a lane per (column, (b1, b2)) reads its entries of C from an
+//     LDS copy with (b1, b2) fastest (lanes of different columns read the same word). The lanes
+//     go by falling number of modes, so that the entries of one b3 belong to the first ones
+//     and the copy holds no padding.
+// R and R' ride on the same lines (FaceTables): the value at the end of a line is one row of N1
+// uniform weights.
+// In place, the modal position (b1, b2, b3) takes the place of (a1, a2, a3).
+// The strides of a column are the ones with the fewest LDS bank conflicts over the lane
+// patterns of all stages (counted for each N1 on the 64 banks; a fifth to a quarter fewer
+// cycles than the next odd strides).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "sse_tensor.h"
+
+namespace sse {
+
+// a read-only table that no kernel writes: loads with a wave-uniform index go to the scalar unit
+typedef const __attribute__((address_space(4))) double* UniformTable;
+__device__ __forceinline__ UniformTable uniform_table(const double* p) { return (UniformTable)(uintptr_t)p; }
+// the same table, but the compiler does not know it: its entries are loaded again where they are
+// used instead of being kept (spilled) in scalar registers from an earlier stage
+__device__ __forceinline__ UniformTable reload(UniformTable p) {
+    uintptr_t v = (uintptr_t)p;
+    asm volatile("" : "+s"(v));
+    return (UniformTable)v;
+}
+
+template <int ELEM, int P>
+struct LineGrid {
+    using Sh = Shape<ELEM, P>;
+    static constexpr int D = Sh::D, N1 = Sh::N1, NP = Sh::NP, NQ = Sh::NQ;
+    static constexpr bool TET = ELEM == ELEM_TET;
+    static constexpr int N2 = TET ? N1 * N1 : N1;  // lines per direction
+    static constexpr int S2 = !TET ? 1 : N1 == 4 ? 5 : N1;
+    static constexpr int S1 = !TET ? (N1 | 1) : N1 == 3 ? 11 : N1 == 4 ? 24 : N1 == 5 ? 26 : 37;
+    static constexpr int NX = !TET ? N1 * S1 : N1 == 3 ? 41 : N1 == 4 ? 100 : N1 == 5 ? 153 : 228;  // of one column
+    static_assert(NX > (N1 - 1) * (S1 + (TET ? S2 + 1 : 1)), "a column holds its grid");
+    // lanes of stage 1: (b1, b2), b1 + b2 <= P, on the Tet; b1 on the Tri
+    static constexpr int NM = TET ? (P + 1) * (P + 2) / 2 : N1;
+
+    // line t of direction l: first position and stride in X; first node and stride in the
+    // unpadded node numbering (last index fastest)
+    template <int L>
+    __device__ static int base(int t) {
+        if constexpr (!TET) return L == 0 ? t : t * S1;
+        const int hi = t / N1, lo = t - hi * N1;
+        return L == 0 ? hi * S2 + lo : L == 1 ? hi * S1 + lo : hi * S1 + lo * S2;
+    }
+    template <int L>
+    __host__ __device__ static constexpr int stride() {
+        return !TET ? (L == 0 ? S1 : 1) : (L == 0 ? S1 : L == 1 ? S2 : 1);
+    }
+    template <int L>
+    __device__ static int node(int t) {
+        if constexpr (!TET) return L == 0 ? t : t * N1;
+        const int hi = t / N1, lo = t - hi * N1;
+        return L == 0 ? t : L == 1 ? hi * N1 * N1 + lo : t * N1;
+    }
+    template <int L>
+    __host__ __device__ static constexpr int node_stride() {
+        return !TET ? (L == 0 ? N1 : 1) : (L == 0 ? N1 * N1 : L == 1 ? N1 : 1);
+    }
+};
+
+// y[a] = sum_b M[a N1 + b] x[b] (ROW) or sum_b M[b N1 + a] x[b]; M uniform
+template <int N1, bool ROW>
+__device__ __forceinline__ void line_apply(UniformTable M, const double* x, double* y) {
+#pragma unroll
+    for (int a = 0; a < N1; ++a) y[a] = 0.0;
+#pragma unroll
+    for (int b = 0; b < N1; ++b)
+#pragma unroll
+        for (int a = 0; a < N1; ++a) y[a] += M[ROW ? a * N1 + b : b * N1 + a] * x[b];
+}
+
+template <int N1, int ST>
+__device__ __forceinline__ void line_load(const double* X, double* x) {
+#pragma unroll
+    for (int a = 0; a < N1; ++a) x[a] = X[a * ST];
+}
+template <int N1, int ST>
+__device__ __forceinline__ void line_store(double* X, const double* x) {
+#pragma unroll
+    for (int a = 0; a < N1; ++a) X[a * ST] = x[a];
+}
+
+template <int ELEM, int P>
+struct LineFact {
+    using G = LineGrid<ELEM, P>;
+    static constexpr int N1 = G::N1, NM = G::NM;
+
+    struct Modes {  // of a stage-1 lane
+        int off, base, lim;  // first mode number, position of the line in X, last b of the line
+    };
+    __device__ static Modes modes(const int* mode, int m) {
+        const int c = mode[m], b1 = (c >> 16) & 0xff, b2 = c >> 24;
+        return G::TET ? Modes{c & 0xffff, b1 * G::S1 + b2 * G::S2, P - b1 - b2} : Modes{c & 0xffff, b1 * G::S1, P - b1};
+    }
+    // LDS doubles of the stage-1 tables, and their copy (all nt threads; a barrier must follow)
+    static constexpr int NT1 = N1 * G::NP;
+    __device__ static void stage_tables(const LineTables& lt, double* dst, int t, int nt) {
+        for (int i = t; i < NT1; i += nt) dst[i] = lt.F1[i];
+    }
+    // lanes with a mode b, and the first table entry of b
+    __host__ __device__ static constexpr int lanes(int b) {
+        return G::TET ? (P - b + 1) * (P - b + 2) / 2 : P - b + 1;
+    }
+    __host__ __device__ static constexpr int first(int b) {
+        int o = 0;
+        for (int q = 0; q < b; ++q) o += N1 * lanes(q);
+        return o;
+    }
+    // stage 1 of V for one line: modal values x (zero past lim) to N1 values
+    __device__ static void up1(const double* F1, int m, const double* x, double* y) {
+#pragma unroll
+        for (int a = 0; a < N1; ++a) y[a] = 0.0;
+#pragma unroll
+        for (int b = 0; b < N1; ++b)
+            if (m < lanes(b)) {
+#pragma unroll
+                for (int a = 0; a < N1; ++a) y[a] += F1[first(b) + a * lanes(b) + m] * x[b];
+            }
+    }
+    // stage 1 of V': N1 values to the line's modal values (zero past its last)
+    __device__ static void down1(const double* F1, int m, const double* x, double* y) {
+#pragma unroll
+        for (int b = 0; b < N1; ++b) {
+            y[b] = 0.0;
+            if (m < lanes(b)) {
+#pragma unroll
+                for (int a = 0; a < N1; ++a) y[b] += F1[first(b) + a * lanes(b) + m] * x[a];
+            }
+        }
+    }
+    // stage 2 (Tet only) of V and of V' for NCOL columns CS apart, in place; B[a2, b1, b2] =
+    // VB[a2 + N1 (b1 + N1 b2)]. All TS threads call; no barrier inside.
+    template <int NCOL, int TS, int CS = 1>
+    __device__ static void up2(UniformTable B, double* X) {
+        if constexpr (G::TET) {
+            const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+            static_assert(P + 2 <= 2 * (TS / 64), "b1 over the wavefronts");
+            // wavefront w takes b1 = w and, where no wavefront starts there, P + 1 - w (their
+            // work goes with P + 1 - b1)
+            for (int b1 = wave; b1 <= P; b1 = (b1 == wave && P + 1 - wave >= TS / 64) ? P + 1 - wave : P + 1)
+                for (int t = lane; t < NCOL * N1; t += 64) {
+                    const int col = t / N1, a3 = t - col * N1;
+                    double* L = X + col * CS * G::NX + b1 * G::S1 + a3;
+                    double y[N1];
+#pragma unroll
+                    for (int a = 0; a < N1; ++a) y[a] = 0.0;
+#pragma unroll
+                    for (int b2 = 0; b2 <= P; ++b2) {
+                        if (b2 > P - b1) break;
+                        const double x = L[b2 * G::S2];
+#pragma unroll
+                        for (int a = 0; a < N1; ++a) y[a] += B[a + N1 * (b1 + N1 * b2)] * x;
+                    }
+                    line_store<N1, G::S2>(L, y);
+                }
+        }
+    }
+    // NSUM: each input is the sum of NSUM consecutive columns
+    template <int NCOL, int TS, int CS = 1, int NSUM = 1>
+    __device__ static void down2(UniformTable B, double* X) {
+        if constexpr (G::TET) {
+            const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+            static_assert(P + 2 <= 2 * (TS / 64), "b1 over the wavefronts");
+            // wavefront w takes b1 = w and, where no wavefront starts there, P + 1 - w (their
+            // work goes with P + 1 - b1)
+            for (int b1 = wave; b1 <= P; b1 = (b1 == wave && P + 1 - wave >= TS / 64) ? P + 1 - wave : P + 1)
+                for (int t = lane; t < NCOL * N1; t += 64) {
+                    const int col = t / N1, a3 = t - col * N1;
+                    double* L = X + col * CS * G::NX + b1 * G::S1 + a3;
+                    double x[N1];
+                    line_load<N1, G::S2>(L, x);
+#pragma unroll
+                    for (int q = 1; q < NSUM; ++q)
+#pragma unroll
+                        for (int a = 0; a < N1; ++a) x[a] += L[q * G::NX + a * G::S2];
+#pragma unroll
+                    for (int b2 = 0; b2 <= P; ++b2) {
+                        if (b2 > P - b1) break;
+                        double y = 0.0;
+#pragma unroll
+                        for (int a = 0; a < N1; ++a) y += B[a + N1 * (b1 + N1 * b2)] * x[a];
+                        L[b2 * G::S2] = y;
+                    }
+                }
+        }
+    }
+};
+
+// e[f N2 + line] = end value of this line (x, direction L) on every face of direction L
+template <int ELEM, int P, int L>
+__device__ __forceinline__ void line_ends(const FaceTables& ft, const double* x, int line, double* e) {
+    using G = LineGrid<ELEM, P>;
+    constexpr int N1 = G::N1;
+    const UniformTable w = uniform_table(ft.w);
+#pragma unroll
+    for (int f = 0; f < G::Sh::NFAC; ++f) {
+        if (ft.dir[f] != L) continue;
+        double s = 0.0;
+#pragma unroll
+        for (int a = 0; a < N1; ++a) s += w[f * N1 + a] * x[a];
+        e[f * G::N2 + line] = s;
+    }
+}
+
+// r[a] += w_f[a] s[f N2 + line] over the faces of direction L (the transpose)
+template <int ELEM, int P, int L>
+__device__ __forceinline__ void line_ends_t(const FaceTables& ft, const double* s, int line, double* r) {
+    using G = LineGrid<ELEM, P>;
+    constexpr int N1 = G::N1;
+    const UniformTable w = uniform_table(ft.w);
+#pragma unroll
+    for (int f = 0; f < G::Sh::NFAC; ++f) {
+        if (ft.dir[f] != L) continue;
+        const double v = s[f * G::N2 + line];
+#pragma unroll
+        for (int a = 0; a < N1; ++a) r[a] += w[f * N1 + a] * v;
+    }
+}
+
+// Line j0 of N1 facet values (same first face index) of a face of kind 1, in place: P_f' t
+template <int N1>
+__device__ __forceinline__ void face_line_t(UniformTable Pf, double* t) {
+    double x[N1], y[N1];
+    line_load<N1, 1>(t, x);
+    line_apply<N1, false>(Pf, x, y);
+    line_store<N1, 1>(t, y);
+}
+
+// acc[c] += row j of M (TR: of M') times column c of x (columns XS apart). The entries of a row
+// are requested together.
+template <int ELEM, int P, int NCV, int XS, bool TR>
+__device__ __forceinline__ void face_row(const FaceTables& ft, int j, const double* x, double* acc) {
+    using G = LineGrid<ELEM, P>;
+    constexpr int N1 = G::N1, N2 = G::N2, NF = G::Sh::NF;
+    if (ft.general) {
+        const int* idx = TR ? ft.mt_idx : ft.m_idx;
+        const double* val = TR ? ft.mt_val : ft.m_val;
+        const int width = TR ? ft.mt_w : ft.m_w;
+        for (int w = 0; w < width; ++w) {
+            const int i = idx[w * NF + j];
+            if (i < 0) break;
+#pragma unroll
+            for (int c = 0; c < NCV; ++c) acc[c] += val[w * NF + j] * x[c * XS + i];
+        }
+        return;
+    }
+    const int f = j / N2;
+    if (G::TET && (f == 0 ? ft.kind[0] : f == 1 ? ft.kind[1] : f == 2 ? ft.kind[2] : ft.kind[3])) {
+        const int c2 = j % N1, j0 = j - c2;
+        const double* Pf = ft.P + f * N1 * N1 + (TR ? c2 : c2 * N1);
+        double pv[N1];
+#pragma unroll
+        for (int b = 0; b < N1; ++b) pv[b] = Pf[TR ? b * N1 : b];
+#pragma unroll
+        for (int b = 0; b < N1; ++b)
+#pragma unroll
+            for (int c = 0; c < NCV; ++c) acc[c] += pv[b] * x[c * XS + j0 + b];
+    } else {
+#pragma unroll
+        for (int c = 0; c < NCV; ++c) acc[c] += x[c * XS + j];
+    }
+}
+
+}  // namespace sse

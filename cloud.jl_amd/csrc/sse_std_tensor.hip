@@ -9,27 +9,37 @@
 //  * a workgroup advances E "slots" at once. A slot is one element of one
 //    problem; with an ensemble of R problems that share the mesh and differ
 //    only in the diffusion coefficient, consecutive slots are the members of
-//    one element, so they also share its geometric factors. Every operator
-//    entry loaded (V factors, rows of D_m, D_m', R, R') serves all E slots
-//    from registers;
-//  * V and V' are sum-factorised (warped-product factors), the mass solve is
-//    the weight-adjusted one with M^{-1} = I (src/Solvers/mass_matrix.jl:59-75);
+//    one element, so they also share its geometric factors;
+//  * V, V' and the derivatives along collapsed directions go line by line: a thread holds a
+//    line of the tensor grid in registers (sse_lines.h). V is followed and V' preceded on
+//    the same lines by the pointwise and line operations next to them: the weight-adjusted
+//    mass solve (M^{-1} = I, src/Solvers/mass_matrix.jl:59-75) applies stage 3 of V, W/J and
+//    stage 3 of V' to a line at once, and stage 1 of V' and stage 1 of the V after it;
 //  * the reference derivative operators are applied along lines: with
 //    D_m = sum_l diag(c_lm) D1_l (D1_l the 1D derivative in collapsed direction l
 //    on every line of the tensor grid, src/SpatialDiscretizations/
-//    SpatialDiscretizations.jl:414-418) and the per-element metric folded into
-//    Lt_ln = sum_m c_lm Lambda_mn once at set-up,
-//      sum_m D_m' (W Lambda_mn x) = sum_l D1_l' (W Lt_ln x),
-//      sum_m Lambda_mn (D_m x)    = sum_l Lt_ln (D1_l x),
-//    so a node's derivative reads N1 neighbours per direction and no table;
-//  * the BR1 auxiliary variable of all d directions goes through one
-//    three-direction mass solve, and R q_q reuses the stored facet values;
-//  * with the skew-symmetric mapping, R x at the facets is never recomputed:
-//    R u_q = u_f and R f_n = a_n u_f - b q_f,n (R is linear), so the interface
-//    and surface terms combine pointwise at the facet nodes.
+//    SpatialDiscretizations.jl:414-418) and the per-element metric folded with the
+//    quadrature weight into Wt_ln = h W sum_m c_lm Lambda_mn once at set-up (h = 1/2 for the
+//    skew-symmetric mapping, else 1),
+//      h sum_m D_m' (W Lambda_mn x)  = sum_l D1_l' (Wt_ln x),
+//      h W sum_m Lambda_mn (D_m x)   = sum_l Wt_ln (D1_l x).
+//    Each entry of Wt_ln belongs to one line, so a thread loads its own from global memory
+//    (all directions at the start, to be there when they are needed);
+//  * between the kernels only modal coefficients and facet values go through memory: u_q and
+//    q_q are formed again from u and from the modal q (a quarter of the bytes);
+//  * with the skew-symmetric mapping the facet terms combine pointwise (R is linear, so
+//    R u_q = u_f and R f_n = a_n u_f - b q_f,n): the gradient needs 1/2 B nJf_n u^+ and the
+//    time derivative B (-1/2 nJf.a u^+ - halfl |nJf.a| (u^- - u^+) + 1/2 b nJf.q^+).
+//
+// What bounds it: with a node per thread every multiply-add read an LDS value, R' and R walked
+// long table rows one cache latency per entry, and u_q, q_q went through memory. Tet p = 5,
+// 24,576 elements: 807 -> 391 us (1.42 GB of memory traffic, 3.6 TB/s; the gradient and the
+// time derivative each spend about half of a workgroup's life waiting for their first loads);
+// 16 diffusivities on 1,296 Tet p = 3 elements, five steps: 4,640 -> 2,840 us (all data in the
+// caches; the chain of short stages between barriers).
 //
 // Lanes: lane g = k * R + r is member r of element k. Intermediate arrays
-// (u_q, u_f, q_q, q_f) are indexed by lane; states and time steps by
+// (u_f, modal q, q_f) are indexed by lane; states and time steps by
 // r * N_e + k (each member a reference-layout (N_p, 1, N_e) array).
 //
 // Tangent pairs: the residual is linear in u and in b (viscous flux -b q,
@@ -40,7 +50,9 @@
 // kernel knows the pairing (it adds -q(u) to the tangent's viscous flux).
 #include <hip/hip_runtime.h>
 
-#include "sse_tensor.h"
+#include <type_traits>
+
+#include "sse_lines.h"
 
 namespace sse {
 
@@ -51,485 +63,650 @@ struct Ensemble {
                         // is R(v; b) + dR/db(u), dR/db(u) = -(viscous terms of u at b = 1)
 };
 
-// threads per workgroup and slots per workgroup of the three kernels (few slots
-// per workgroup measured fastest: more workgroups in flight hide the latency of
-// the dependent stages better than wider reuse of the small tables)
+// Threads and slots of a workgroup: nodal values (TS1, E1; a line of each slot per thread) and
+// the other two (TS, E; a line of each slot and direction component per thread).
 template <int ELEM, int P>
 struct StdTune;
-#define SSE_STD_TUNE(E_, PP, ts, e1, e2, e3) \
+#define SSE_STD_TUNE(E_, PP, ts1, e1, ts, e) \
     template <>                              \
     struct StdTune<E_, PP> {                 \
-        static constexpr int TS = ts, E1 = e1, E2 = e2, E3 = e3; \
+        static constexpr int TS1 = ts1, E1 = e1, TS = ts, E = e; \
     };
-SSE_STD_TUNE(ELEM_TRI, 2, 64, 8, 2, 2)
-SSE_STD_TUNE(ELEM_TRI, 3, 64, 8, 2, 2)
-SSE_STD_TUNE(ELEM_TRI, 4, 64, 8, 2, 2)
-SSE_STD_TUNE(ELEM_TRI, 5, 64, 8, 2, 2)
-SSE_STD_TUNE(ELEM_TRI, 6, 64, 8, 2, 2)
-SSE_STD_TUNE(ELEM_TET, 2, 64, 8, 2, 2)
-SSE_STD_TUNE(ELEM_TET, 3, 64, 8, 2, 2)
-SSE_STD_TUNE(ELEM_TET, 4, 128, 8, 1, 2)
-SSE_STD_TUNE(ELEM_TET, 5, 256, 8, 1, 2)
+SSE_STD_TUNE(ELEM_TRI, 2, 64, 21, 64, 10)
+SSE_STD_TUNE(ELEM_TRI, 3, 64, 16, 64, 8)
+SSE_STD_TUNE(ELEM_TRI, 4, 64, 12, 64, 6)
+SSE_STD_TUNE(ELEM_TRI, 5, 64, 10, 64, 5)
+SSE_STD_TUNE(ELEM_TRI, 6, 64, 9, 64, 4)
+SSE_STD_TUNE(ELEM_TET, 2, 128, 14, 128, 4)
+SSE_STD_TUNE(ELEM_TET, 3, 192, 12, 192, 4)
+SSE_STD_TUNE(ELEM_TET, 4, 256, 10, 256, 3)
+SSE_STD_TUNE(ELEM_TET, 5, 256, 7, 256, 2)
 #undef SSE_STD_TUNE
+
+// Waves per SIMD the registers must allow (one more spills at either size: Tet p = 5 at
+// 24,576 elements 395 us with 5, 438 us with 6).
+constexpr int std_waves(int P) { return P == 5 ? 5 : 6; }
 
 namespace {
 
-constexpr int cmax(int a, int b) { return a > b ? a : b; }
-
-// waves per SIMD that `lds_doubles` of LDS per workgroup of `threads` allow (160 KB
-// per CU, 4 SIMDs), capped at 7: the register budget a kernel is held to, so that
-// the compiler does not trade the occupancy the LDS allows for early loads
-constexpr int lds_waves(int lds_doubles, int threads) {
-    const int wg = (160 * 1024) / (8 * lds_doubles);
-    const int w = wg * (threads / 64) / 4;
-    return w < 1 ? 1 : (w > 7 ? 7 : w);
-}
-
-// Node i of the tensor grid has coordinate (i / stride_l) % N1 in direction l
-// (the last direction fastest).
-template <int ELEM, int P>
-struct Lines {
-    static constexpr int D = Shape<ELEM, P>::D, N1 = P + 1;
-    __host__ __device__ static constexpr int stride(int l) {
-        return D == 3 ? (l == 0 ? N1 * N1 : (l == 1 ? N1 : 1)) : (l == 0 ? N1 : 1);
+// Slot s works on lane g0 + s (past the last lane: on the last one, storing nothing). The element
+// and the member of a lane come from those of the first slot: a workgroup has few slots, so one
+// subtraction replaces the division when the ensemble has more members than that.
+template <int E>
+struct Slots {
+    unsigned g0, nl, R, k0, r0;
+    __device__ bool valid(int s) const { return g0 + (unsigned)s < nl; }
+    __device__ unsigned clamp(int s) const { return min((unsigned)s, nl - 1 - g0); }
+    __device__ unsigned lane(int s) const { return g0 + clamp(s); }
+    __device__ unsigned element(int s) const {
+        const unsigned q = r0 + clamp(s);
+        return R == 1 ? k0 + q : R >= (unsigned)E ? k0 + (q >= R ? 1u : 0u) : k0 + q / R;
     }
-    __device__ static int coord(int i, int l) { return (i / stride(l)) % N1; }
+    __device__ unsigned member(int s) const {
+        const unsigned q = r0 + clamp(s);
+        return R == 1 ? 0u : R >= (unsigned)E ? (q >= R ? q - R : q) : q % R;
+    }
+    __device__ size_t row(int s, int N_e) const { return (size_t)member(s) * N_e + element(s); }
 };
 
-__device__ __forceinline__ size_t state_row(long long g, int R, int N_e) {
-    const long long k = g / R, r = g - k * R;
-    return (size_t)r * N_e + k;
+template <int E>
+__device__ __forceinline__ Slots<E> slots_of(const TensorParams& tp, const Ensemble& en) {
+    const unsigned g0 = (unsigned)element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * E, R = (unsigned)en.R;
+    const unsigned k0 = R == 1 ? g0 : g0 / R;
+    return Slots<E>{g0, (unsigned)tp.base.N_e * R, R, k0, g0 - k0 * R};
 }
 
-__device__ __forceinline__ double member_b(const DevParams& p, const Ensemble& en, long long g) {
-    return en.b ? en.b[g % en.R] : p.b;
-}
-
-// lane of the exterior state of facet node j of lane g
-__device__ __forceinline__ long long neighbour(const DevParams& p, int R, long long g, int NF, int j, int& jn) {
-    const long long k = g / R, r = g - k * R;
-    const int gl = p.mapP[j + (size_t)NF * k];
+// lane and facet node of the exterior state of facet node j of slot s
+template <int NF, int E>
+__device__ __forceinline__ unsigned neighbour(const DevParams& p, const Slots<E>& sl, int s, int j, int& jn) {
+    const int gl = p.mapP[j + (size_t)NF * sl.element(s)];
     const int kn = gl / NF;
     jn = gl - kn * NF;
-    return (long long)kn * R + r;
+    return (unsigned)kn * sl.R + sl.member(s);
 }
 
-// acc[c] += sum over row `row` of an ELL table (width a multiple of 4, -1 pads
-// with value 0) of val * x[c * XS + idx]: four entries per step, so that a
-// step's loads are in flight together
-template <int NCV, int XS>
-__device__ __forceinline__ void ell_apply(const int* __restrict__ idx, const double* __restrict__ val, int width,
-                                          int nrows, int row, const double* x, double* acc) {
-    for (int w = 0; w < width; w += 4) {
-        int ii[4];
-        double vv[4];
+template <int V>
+using Dir = std::integral_constant<int, V>;
+
+// ends of line `line` of every direction but the first, of one column X
+template <int ELEM, int P>
+__device__ __forceinline__ void other_line_ends(const FaceTables& ft, const double* X, int line, double* e) {
+    using G = LineGrid<ELEM, P>;
+    constexpr int N1 = G::N1;
+    double x[N1];
+    line_load<N1, G::template stride<1>()>(X + G::template base<1>(line), x);
+    line_ends<ELEM, P, 1>(ft, x, line, e);
+    if constexpr (G::TET) {
+        line_load<N1, G::template stride<2>()>(X + G::template base<2>(line), x);
+        line_ends<ELEM, P, 2>(ft, x, line, e);
+    }
+}
+
+// in place, the facet values t of NCOL columns (NF apart) to M' t; the caller's barrier follows.
+// The lines of the faces of kind 1 go to the last threads of the workgroup (the first ones have
+// stage-1 lines of V in the same phase).
+template <int ELEM, int P, int NCOL, int TS>
+__device__ __forceinline__ void face_transpose(const FaceTables& ft, double* t) {
+    using G = LineGrid<ELEM, P>;
+    constexpr int N1 = G::N1, N2 = G::N2, NF = G::Sh::NF;
+    if (ft.general) {
+        constexpr int IT = (NCOL * NF + TS - 1) / TS;
+        double v[IT];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            ii[t] = idx[(w + t) * nrows + row];
-            vv[t] = val[(w + t) * nrows + row];
+        for (int q = 0; q < IT; ++q) {
+            const int o = (int)threadIdx.x + q * TS, c = o / NF;
+            v[q] = 0.0;
+            if (o < NCOL * NF) face_row<ELEM, P, 1, NF, true>(ft, o - c * NF, t + c * NF, v + q);
         }
+        __syncthreads();
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int i = ii[t] < 0 ? 0 : ii[t];
+        for (int q = 0; q < IT; ++q)
+            if ((int)threadIdx.x + q * TS < NCOL * NF) t[threadIdx.x + q * TS] = v[q];
+    } else if constexpr (G::TET) {
 #pragma unroll
-            for (int c = 0; c < NCV; ++c) acc[c] += vv[t] * x[c * XS + i];
+        for (int f = 0; f < 4; ++f) {
+            if (ft.kind[f] == 0) continue;
+            const UniformTable Pf = uniform_table(ft.P) + f * N1 * N1;
+            for (int o = TS - 1 - (int)threadIdx.x; o < NCOL * N1; o += TS) {
+                const int c = o / N1;
+                face_line_t<N1>(Pf, t + c * NF + f * N2 + (o - c * N1) * N1);
+            }
         }
-        if (ii[3] < 0) break;
     }
 }
 
 }  // namespace
 
 // ----------------------------------------------------------------------------- phase 1
-// u_q = V u, u_f = R u_q
+// u_f = R V u
 template <int ELEM, int P>
-struct StdNodalLayout {
-    using Sh = Shape<ELEM, P>;
-    static constexpr int E = StdTune<ELEM, P>::E1;
-    // the sum-factorisation temporary Z lives in u_q's array (dead before V's last stage)
-    static constexpr int u = 0, q = u + E * Sh::NP, z = q, w = q + E * Sh::NQ;
-    static constexpr int size = w + E * cmax(Sh::NW, 1);
-};
-
-template <int ELEM, int P>
-__global__ void __launch_bounds__((StdTune<ELEM, P>::TS))
+__global__ void __launch_bounds__((StdTune<ELEM, P>::TS1))
 k_std_nodal_tensor(TensorParams tp, Ensemble en, const double* __restrict__ u) {
-    using Sh = Shape<ELEM, P>;
+    using G = LineGrid<ELEM, P>;
+    using LF = LineFact<ELEM, P>;
     using T = StdTune<ELEM, P>;
-    using L = StdNodalLayout<ELEM, P>;
-    constexpr int E = T::E1, TS = T::TS, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF;
-    using SF = SumFact<ELEM, P, TS, E>;
+    constexpr int E = T::E1, TS = T::TS1, N1 = G::N1, N2 = G::N2, NM = G::NM, NX = G::NX, NP = G::NP, NF = G::Sh::NF;
+    static_assert(E * N2 <= TS, "a line per thread");
     extern __shared__ double sm[];
+    double* X = sm;              // E columns
+    double* F1 = sm + E * NX;
     const DevParams& p = tp.base;
     const int tl = threadIdx.x;
-    const long long nl = (long long)p.N_e * en.R;
-    const long long g0 = (long long)element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * E;
-    double *su = sm + L::u, *sq = sm + L::q;
-    for (int t = tl; t < E * NP; t += TS) {
-        const int s = t / NP, j = t - s * NP;
-        const long long g = g0 + s;
-        su[t] = g < nl ? u[state_row(g, en.R, p.N_e) * NP + j] : 0.0;
+    const Slots<E> sl = slots_of<E>(tp, en);
+    const UniformTable A = uniform_table(tp.VA), B = uniform_table(tp.VB);
+    LF::stage_tables(tp.lines, F1, tl, TS);
+    __syncthreads();
+    for (int t = tl; t < E * NM; t += TS) {
+        const int s = t / NM, m = t - s * NM;
+        const auto md = LF::modes(tp.lines.mode, m);
+        const double* um = u + sl.row(s, p.N_e) * NP + md.off;
+        double x[N1], y[N1];
+#pragma unroll
+        for (int b = 0; b < N1; ++b) x[b] = b <= md.lim ? um[b] : 0.0;
+        LF::up1(F1, m, x, y);
+        line_store<N1, 1>(X + s * NX + md.base, y);
     }
     __syncthreads();
-    SF::V(tp, tl, su, sq, sm + L::z, sm + L::w);
-    const int nvalid = (int)(nl - g0 < E ? nl - g0 : E);
-    for (int t = tl; t < nvalid * NQ; t += TS) p.uq[(size_t)g0 * NQ + t] = sq[t];
-    for (int j = tl; j < NF; j += TS) {
-        double acc[E];
+    if constexpr (G::TET) {
+        LF::template up2<E, TS>(reload(B), X);
+        __syncthreads();
+    }
+    double* e = F1 + LF::NT1;  // E x NF line ends
+    const int s = tl / N2, line = tl - s * N2;
+    if (tl < E * N2) {
+        double* L = X + s * NX + G::template base<0>(line);
+        double x[N1], y[N1];
+        line_load<N1, G::S1>(L, x);
+        line_apply<N1, false>(reload(A), x, y);
+        line_store<N1, G::S1>(L, y);
+        line_ends<ELEM, P, 0>(tp.faces, y, line, e + s * NF);
+    }
+    __syncthreads();
+    if (tl < E * N2) other_line_ends<ELEM, P>(tp.faces, X + s * NX, line, e + s * NF);
+    __syncthreads();
+    for (int t = tl; t < E * NF; t += TS) {
+        const int q = t / NF, j = t - q * NF;
+        double acc[1] = {0.0};
+        face_row<ELEM, P, 1, NF, false>(tp.faces, j, e + q * NF, acc);
+        if (sl.valid(q)) p.uf[(size_t)sl.lane(q) * NF + j] = acc[0];
+    }
+}
+
+// ----------------------------------------------------------------------------- shared stages
+// One direction of the terms of r for the line `line`: SIGN VT of column x, with
+// VT = D1_l' (Wt x) - Wt (D1_l x) (skew) or D1_l' (Wt x), plus R' of the facet terms fs = M' t
+// (fs null: none) on the faces of that direction; on top of r_col unless it is the first direction
+template <int ELEM, int P, int L, bool SKEW, int SIGN>
+__device__ __forceinline__ void volume_line(UniformTable D1, const FaceTables& ft, const double* x_col,
+                                            const double* wt, const double* fs, int line, const double* r_col,
+                                            double* r) {
+    using G = LineGrid<ELEM, P>;
+    constexpr int N1 = G::N1, ST = G::template stride<L>();
+    const int base = G::template base<L>(line);
+    const UniformTable M = D1 + L * N1 * N1;
+    double x[N1], g[N1];
+    line_load<N1, ST>(x_col + base, x);
+    if constexpr (L == G::D - 1) {
 #pragma unroll
-        for (int s = 0; s < E; ++s) acc[s] = 0.0;
-        ell_apply<E, NQ>(tp.r_idx, tp.r_val, tp.wr, NF, j, sq, acc);
+        for (int a = 0; a < N1; ++a) r[a] = 0.0;
+    } else {
+        line_load<N1, ST>(r_col + base, r);
+    }
 #pragma unroll
-        for (int s = 0; s < E; ++s)
-            if (s < nvalid) p.uf[(size_t)(g0 + s) * NF + j] = acc[s];
+    for (int b = 0; b < N1; ++b) g[b] = wt[b] * x[b];
+#pragma unroll
+    for (int a = 0; a < N1; ++a) {  // a row and a column of D1_l at a time (few registers)
+        double y = 0.0, z = 0.0;
+#pragma unroll
+        for (int b = 0; b < N1; ++b) {
+            y += M[b * N1 + a] * g[b];
+            if constexpr (SKEW) z += M[a * N1 + b] * x[b];
+        }
+        if constexpr (SKEW) y -= wt[a] * z;
+        r[a] += SIGN > 0 ? y : -y;
+    }
+    if (fs) line_ends_t<ELEM, P, L>(ft, fs, line, r);
+}
+
+// The middle of the weight-adjusted mass solve for NCOL columns CS apart whose V' has gone
+// through stage 2: [stage 1 of V', stage 1 of V], stage 2, [stage 3 of V, W/J, stage 3 of V'],
+// stage 2 of V'. NSUM: the columns start as sums of NSUM consecutive ones (Tri; on the Tet
+// stage 2 has added them). Ends with a barrier.
+// on1, c1, m1, md1: this thread's stage-1 line (column c1, lane m1) of all columns; on, col,
+// line, wj: its line along the first direction and W / J there.
+template <int ELEM, int P, int TS, int NCOL, int CS, int NSUM>
+__device__ __forceinline__ void mass_middle(const TensorParams& tp, const double* F1, double* X, bool on1, int c1,
+                                            int m1, const typename LineFact<ELEM, P>::Modes& md1, bool on, int col,
+                                            int line, const double* wj) {
+    using G = LineGrid<ELEM, P>;
+    using LF = LineFact<ELEM, P>;
+    constexpr int N1 = G::N1, NX = G::NX;
+    const UniformTable A = uniform_table(tp.VA), B = uniform_table(tp.VB);
+    if (on1 && c1 % CS == 0) {
+        const int m = m1;
+        double* L = X + c1 * NX + md1.base;
+        double x[N1], y[N1];
+        line_load<N1, 1>(L, x);
+#pragma unroll
+        for (int q = 1; q < NSUM; ++q)
+#pragma unroll
+            for (int a = 0; a < N1; ++a) x[a] += L[q * NX + a];
+        LF::down1(F1, m, x, y);
+        LF::up1(F1, m, y, x);
+        line_store<N1, 1>(L, x);
+    }
+    __syncthreads();
+    if constexpr (G::TET) {
+        LF::template up2<NCOL, TS, CS>(reload(B), X);
+        __syncthreads();
+    }
+    if (on && col % CS == 0) {
+        double* L = X + col * NX + G::template base<0>(line);
+        double x[N1], y[N1];
+        line_load<N1, G::S1>(L, x);
+        line_apply<N1, false>(reload(A), x, y);
+#pragma unroll
+        for (int a = 0; a < N1; ++a) y[a] *= wj[a];
+        line_apply<N1, true>(reload(A), y, x);
+        line_store<N1, G::S1>(L, x);
+    }
+    __syncthreads();
+    if constexpr (G::TET) {
+        LF::template down2<NCOL, TS, CS>(reload(B), X);
+        __syncthreads();
     }
 }
 
 // ----------------------------------------------------------------------------- BR1 auxiliary variable
-// q_m = M^{-1} V' [ -VT_m(u_q) + R' (B J_f u*_m) ],  u*_m = 1/2 (u^- + u^+) n_m,
-// VT_n(x) = h sum_m D_m' (W Lambda_mn x) - h W sum_m Lambda_mn (D_m x) + R' (1/2 B nJf_n R x)
-// (h = 1/2, skew-symmetric mapping) or sum_m D_m' (W Lambda_mn x) (standard mapping).
-// With the skew form the facet terms combine to R' (1/2 B nJf_n u^+). All d
-// directions go through each pass together.
-template <int ELEM, int P, bool SKEW>
+// q_n = M^{-1} V' [ -VT_n(u_q) + R' (B J_f u*_n) ],  u*_n = 1/2 (u^- + u^+) n_n,
+// VT_n(x) = sum_l D1_l' (Wt_ln x) - Wt_ln (D1_l x) + R' (1/2 B nJf_n R x) (skew-symmetric
+// mapping) or sum_l D1_l' (Wt_ln x) (standard mapping). With the skew form the facet terms
+// combine to R' (1/2 B nJf_n u^+). Writes the modal q_n and q_f,n = R V q_n.
+template <int ELEM, int P>
 struct StdAuxLayout {
-    using Sh = Shape<ELEM, P>;
-    static constexpr int E = StdTune<ELEM, P>::E2, D = Sh::D;
-    static constexpr int A = cmax(D * Sh::NQ, D * (Sh::NZ + Sh::NP));  // D1_l u, then SumFact Z and y
-    static constexpr int B = cmax(D * Sh::NQ, D * Sh::NW);             // g_ln of one n, then SumFact W
-    // u^- only for the standard mapping
-    static constexpr int uq = 0, up = uq + E * Sh::NQ, um = up + E * Sh::NF, a = um + (SKEW ? 0 : E * Sh::NF);
-    static constexpr int b = a + E * A, r = b + E * B, tf = r + E * D * Sh::NQ;
-    static constexpr int d1 = tf + E * D * Sh::NF;
-    static constexpr int size = d1 + D * Sh::N1 * Sh::N1;
+    using G = LineGrid<ELEM, P>;
+    static constexpr int E = StdTune<ELEM, P>::E, D = G::D;
+    static constexpr int u = 0, r = u + E * G::NX, tf = r + E * D * G::NX, f1 = r + E * D * G::NX + E * D * G::Sh::NF;
+    static constexpr int size = f1 + LineFact<ELEM, P>::NT1;
 };
 
 template <int ELEM, int P, bool SKEW>
-__global__ void __launch_bounds__((StdTune<ELEM, P>::TS), (lds_waves(StdAuxLayout<ELEM, P, SKEW>::size, StdTune<ELEM, P>::TS)))
-    k_std_aux_tensor(TensorParams tp, Ensemble en) {
-    using Sh = Shape<ELEM, P>;
+__global__ void __launch_bounds__((StdTune<ELEM, P>::TS), std_waves(P))
+    k_std_aux_tensor(TensorParams tp, Ensemble en, const double* __restrict__ u) {
+    using G = LineGrid<ELEM, P>;
+    using LF = LineFact<ELEM, P>;
     using T = StdTune<ELEM, P>;
-    using L = StdAuxLayout<ELEM, P, SKEW>;
-    using LN = Lines<ELEM, P>;
-    constexpr int E = T::E2, TS = T::TS, D = Sh::D, NQ = Sh::NQ, NF = Sh::NF, N1 = Sh::N1;
-    using SF = SumFact<ELEM, P, TS, D * E>;
+    using L = StdAuxLayout<ELEM, P>;
+    constexpr int E = T::E, TS = T::TS, D = G::D, N1 = G::N1, N2 = G::N2, NM = G::NM, NX = G::NX, NP = G::NP,
+                  NQ = G::NQ, NF = G::Sh::NF;
+    static_assert(E * D * N2 <= TS, "a line per thread");
     extern __shared__ double sm[];
     const DevParams& p = tp.base;
     const int tl = threadIdx.x;
-    const int R = en.R;
-    const long long nl = (long long)p.N_e * R;
-    const long long g0 = (long long)element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * E;
-    const int nvalid = (int)(nl - g0 < E ? nl - g0 : E);
-    double *suq = sm + L::uq, *sup = sm + L::up, *sum = sm + L::um, *sDu = sm + L::a, *sg = sm + L::b,
-           *sr = sm + L::r, *stf = sm + L::tf, *sD1 = sm + L::d1;
-    constexpr double h = SKEW ? 0.5 : 1.0;
+    const Slots<E> sl = slots_of<E>(tp, en);
+    const UniformTable A = uniform_table(tp.VA), B = uniform_table(tp.VB), D1 = uniform_table(tp.D1);
+    double *xu = sm + L::u, *xr = sm + L::r, *stf = sm + L::tf, *F1 = sm + L::f1;
 
-    for (int t = tl; t < D * N1 * N1; t += TS) sD1[t] = tp.D1[t];
-    for (int t = tl; t < E * NQ; t += TS) suq[t] = t < nvalid * NQ ? p.uq[(size_t)g0 * NQ + t] : 0.0;
+    // this thread's line (slot, component n, line) and its metric entries of every direction
+    const bool on = tl < E * D * N2;
+    const int ls = on ? tl / (D * N2) : 0, ln = on ? (tl / N2) % D : 0, line = tl % N2;
+    double wt[D][N1];  // requested well before its pass: the last two directions now
+    const double* Wk = p.Lam + ((size_t)sl.element(ls) * D * D + D * ln) * NQ;
+    auto load_wt = [&](auto l) {
+        constexpr int l_ = decltype(l)::value;
+#pragma unroll
+        for (int a = 0; a < N1; ++a)
+            wt[l_][a] = Wk[l_ * NQ + G::template node<l_>(line) + a * G::template node_stride<l_>()];
+    };
+    // and its stage-1 line (column c1 of E D)
+    static_assert(E * D * NM <= TS, "a stage-1 line per thread");
+    const bool on1 = tl < E * D * NM;
+    const int c1 = tl / NM, m1 = tl % NM;
+    const auto md1 = LF::modes(tp.lines.mode, m1);
+    // this thread's facet nodes: the neighbours first (their states hang on them)
+    constexpr int IT = (E * NF + TS - 1) / TS;
+    unsigned gn[IT];
+    int jn[IT];
+#pragma unroll
+    for (int q = 0; q < IT; ++q) {
+        const int t = min(tl + q * TS, E * NF - 1), s = t / NF;
+        gn[q] = neighbour<NF>(p, sl, s, t - s * NF, jn[q]);
+    }
+    // everything the prologue reads is requested before the first of it is used: modal u of the
+    // stage-1 line (column s1 of the first E), the facet states, the metric entries
+    const int s1 = min(c1, E - 1);
+    double xm[N1], uo[IT], ui[IT], nJ[IT][D];
+    {
+        const double* um = u + sl.row(s1, p.N_e) * NP + md1.off;
+#pragma unroll
+        for (int b = 0; b < N1; ++b) xm[b] = um[min(b, md1.lim)];
+    }
+#pragma unroll
+    for (int q = 0; q < IT; ++q) {
+        const int t = min(tl + q * TS, E * NF - 1), s = t / NF, j = t - s * NF;
+        const unsigned g = sl.lane(s);
+        uo[q] = p.uf[(size_t)gn[q] * NF + jn[q]];
+        if (!SKEW) ui[q] = p.uf[(size_t)g * NF + j];
+        const double* n = p.nJf + (size_t)sl.element(s) * D * NF + D * j;
+#pragma unroll
+        for (int m = 0; m < D; ++m) nJ[q][m] = n[m];
+    }
+    LF::stage_tables(tp.lines, F1, tl, TS);
+    load_wt(Dir<D - 1>{});
+    if constexpr (D == 3) load_wt(Dir<1>{});
+    // facet terms: 1/2 B nJf_n u^+ (skew) or 1/2 B nJf_n (u^- + u^+)
+#pragma unroll
+    for (int q = 0; q < IT; ++q) {
+        const int t = tl + q * TS;
+        if (t >= E * NF) break;
+        const int s = t / NF, j = t - s * NF;
+        const double x = 0.5 * p.B[j] * (SKEW ? uo[q] : ui[q] + uo[q]);
+#pragma unroll
+        for (int n = 0; n < D; ++n) stf[(s * D + n) * NF + j] = nJ[q][n] * x;
+    }
+    __syncthreads();
+    if (tl < E * NM) {  // stage 1 of V u
+        double y[N1];
+#pragma unroll
+        for (int b = 0; b < N1; ++b) xm[b] = b <= md1.lim ? xm[b] : 0.0;
+        LF::up1(F1, m1, xm, y);
+        line_store<N1, 1>(xu + s1 * NX + md1.base, y);
+    }
+    face_transpose<ELEM, P, E * D, TS>(tp.faces, stf);
+    __syncthreads();
+    if constexpr (G::TET) {
+        LF::template up2<E, TS>(reload(B), xu);
+        __syncthreads();
+    }
+    if (tl < E * N2) {
+        double* X = xu + (tl / N2) * NX + G::template base<0>(tl % N2);
+        double x[N1], y[N1];
+        line_load<N1, G::S1>(X, x);
+        line_apply<N1, false>(reload(A), x, y);
+        line_store<N1, G::S1>(X, y);
+    }
+    __syncthreads();
+    // r_n -= VT_n(u_q), one direction after the other; the last (along a1) goes on with stage
+    // 3 of V'
+    double wj[N1];  // W / J along this thread's line, for the mass solve
+    auto load_woj = [&]() {
+        const double* w = tp.WoJ + (size_t)sl.element(ls) * NQ + G::template node<0>(line);
+#pragma unroll
+        for (int a = 0; a < N1; ++a) wj[a] = w[a * G::template node_stride<0>()];
+    };
+    const double* xc = xu + ls * NX;
+    double* rc = xr + (ls * D + ln) * NX;
+    auto pass = [&](auto l) {
+        constexpr int l_ = decltype(l)::value;
+        if constexpr (l_ == D - 1) load_wt(Dir<0>{});
+        if constexpr (l_ == 1) load_woj();
+        if (on) {
+            double r[N1];
+            volume_line<ELEM, P, l_, SKEW, -1>(reload(D1), tp.faces, xc, wt[l_], stf + (ls * D + ln) * NF, line, rc,
+                                               r);
+            if constexpr (l_ == 0) {
+                double w[N1];
+                line_apply<N1, true>(reload(A), r, w);
+                line_store<N1, G::S1>(rc + G::template base<0>(line), w);
+            } else {
+                line_store<N1, G::template stride<l_>()>(rc + G::template base<l_>(line), r);
+            }
+        }
+        __syncthreads();
+    };
+    if constexpr (D == 3) pass(Dir<2>{});
+    pass(Dir<1>{});
+    pass(Dir<0>{});
+    if constexpr (G::TET) {
+        LF::template down2<E * D, TS>(reload(B), xr);
+        __syncthreads();
+    }
+    mass_middle<ELEM, P, TS, E * D, 1, 1>(tp, F1, xr, on1, c1, m1, md1, on, ls * D + ln, line, wj);
+    // modal q_n out, and V q_n
+    if (on1) {
+        const int s = c1 / D;
+        double* X = xr + c1 * NX + md1.base;
+        double x[N1], y[N1];
+        line_load<N1, 1>(X, x);
+        LF::down1(F1, m1, x, y);
+        if (sl.valid(s)) {
+            double* q = p.qq + ((size_t)sl.lane(s) * D + (c1 - s * D)) * NP + md1.off;
+#pragma unroll
+            for (int b = 0; b < N1; ++b)
+                if (b <= md1.lim) q[b] = y[b];
+        }
+        LF::up1(F1, m1, y, x);
+        line_store<N1, 1>(X, x);
+    }
+    __syncthreads();
+    if constexpr (G::TET) {
+        LF::template up2<E * D, TS>(reload(B), xr);
+        __syncthreads();
+    }
+    // q_f = R q_q: the ends of the lines, then the interpolation on the faces
+    double* e = stf + (ls * D + ln) * NF;
+    if (on) {
+        double* X = rc + G::template base<0>(line);
+        double x[N1], y[N1];
+        line_load<N1, G::S1>(X, x);
+        line_apply<N1, false>(reload(A), x, y);
+        line_store<N1, G::S1>(X, y);
+        line_ends<ELEM, P, 0>(tp.faces, y, line, e);
+    }
+    __syncthreads();
+    if (on) other_line_ends<ELEM, P>(tp.faces, rc, line, e);
+    __syncthreads();
     for (int t = tl; t < E * NF; t += TS) {
         const int s = t / NF, j = t - s * NF;
-        const long long g = g0 + s;
-        double up = 0.0, um = 0.0;
-        if (s < nvalid) {
-            int jn;
-            const long long gn = neighbour(p, R, g, NF, j, jn);
-            up = p.uf[(size_t)gn * NF + jn];
-            if (!SKEW) um = p.uf[(size_t)g * NF + j];
+        double acc[D];
+#pragma unroll
+        for (int n = 0; n < D; ++n) acc[n] = 0.0;
+        face_row<ELEM, P, D, NF, false>(tp.faces, j, stf + s * D * NF, acc);
+        if (sl.valid(s)) {
+#pragma unroll
+            for (int n = 0; n < D; ++n) p.qf[((size_t)sl.lane(s) * D + n) * NF + j] = acc[n];
         }
-        sup[t] = up;
-        if (!SKEW) sum[t] = um;
-    }
-    __syncthreads();
-    if constexpr (SKEW) {  // D1_l u_q along the lines of each direction l
-        for (int i = tl; i < NQ; i += TS) {
-#pragma unroll
-            for (int l = 0; l < D; ++l) {
-                const int sl = LN::stride(l), a = LN::coord(i, l), base = i - a * sl;
-                const double* drow = sD1 + (l * N1 + a) * N1;
-                double acc[E];
-#pragma unroll
-                for (int s = 0; s < E; ++s) acc[s] = 0.0;
-#pragma unroll
-                for (int bb = 0; bb < N1; ++bb) {
-                    const double dv = drow[bb];
-#pragma unroll
-                    for (int s = 0; s < E; ++s) acc[s] += dv * suq[s * NQ + base + bb * sl];
-                }
-#pragma unroll
-                for (int s = 0; s < E; ++s) sDu[(s * D + l) * NQ + i] = acc[s];
-            }
-        }
-        __syncthreads();
-    }
-    // facet: 1/2 B nJf_n u^+ (skew) or 1/2 B nJf_n (u^- + u^+)
-    for (int t = tl; t < E * NF; t += TS) {
-        const int s = t / NF, j = t - s * NF;
-        const long long k = (g0 + (s < nvalid ? s : 0)) / R;
-        const double* nJ = p.nJf + (size_t)k * D * NF + D * j;
-        const double x = 0.5 * p.B[j] * (SKEW ? sup[t] : sup[t] + sum[t]);  // sum unread when SKEW
-#pragma unroll
-        for (int n = 0; n < D; ++n) stf[(s * D + n) * NF + j] = nJ[n] * x;
-    }
-    // one direction n at a time (three g_ln arrays in LDS instead of nine):
-    //   g_ln = h W Lt_ln u_q;  r_n = h W sum_l Lt_ln (D1_l u_q) - sum_l D1_l' g_ln + R' tf_n
-    // node i's sums stay in registers across the passes
-    static_assert(NQ <= TS, "one volume node per thread");
-    double acc[E * D];
-#pragma unroll
-    for (int c = 0; c < E * D; ++c) acc[c] = 0.0;
-#pragma unroll 1
-    for (int n = 0; n < D; ++n) {
-        for (int t = tl; t < E * NQ; t += TS) {
-            const int s = t / NQ, i = t - s * NQ;
-            const long long k = (g0 + (s < nvalid ? s : 0)) / R;
-            const double* Lk = p.Lam + (size_t)k * NQ * D * D;
-            const double hw = h * p.W[i];
-            const double x = suq[t];
-            double dterm = 0.0;
-#pragma unroll
-            for (int l = 0; l < D; ++l) {
-                const double lam = Lk[i + NQ * (l + D * n)];
-                sg[(s * D + l) * NQ + i] = hw * lam * x;
-                if constexpr (SKEW) dterm += lam * sDu[(s * D + l) * NQ + i];
-            }
-            sr[(s * D + n) * NQ + i] = hw * dterm;
-        }
-        __syncthreads();
-        if (tl < NQ) {
-            const int i = tl;
-#pragma unroll 1
-            for (int l = 0; l < D; ++l) {
-                const int sl = LN::stride(l), a = LN::coord(i, l), base = i - a * sl;
-#pragma unroll
-                for (int bb = 0; bb < N1; ++bb) {
-                    const double dv = sD1[(l * N1 + bb) * N1 + a];
-#pragma unroll
-                    for (int s = 0; s < E; ++s) acc[s * D + n] -= dv * sg[(s * D + l) * NQ + base + bb * sl];
-                }
-            }
-        }
-        __syncthreads();
-    }
-    if (tl < NQ) {
-        const int i = tl;
-        ell_apply<E * D, NF>(tp.rt_idx, tp.rt_val, tp.wrt, NQ, i, stf, acc);
-#pragma unroll
-        for (int c = 0; c < E * D; ++c) sr[c * NQ + i] += acc[c];
-    }
-    __syncthreads();
-    // three-direction mass solve: q = V' (W/J o V (V' r)); then q_q = V q
-    double* sZ = sDu;
-    double* sy = sDu + E * D * Sh::NZ;
-    double* sW = sg;
-    SF::Vt(tp, tl, sr, sy, sZ, sW);
-    SF::V(tp, tl, sy, sr, sZ, sW);
-    for (int t = tl; t < E * D * NQ; t += TS) {
-        const int c = t / NQ, i = t - c * NQ, s = c / D;
-        const long long k = (g0 + (s < nvalid ? s : 0)) / R;
-        sr[t] *= p.W[i] / p.Jq[(size_t)k * NQ + i];
-    }
-    __syncthreads();
-    SF::Vt(tp, tl, sr, sy, sZ, sW);
-    SF::V(tp, tl, sy, sr, sZ, sW);
-    for (int t = tl; t < nvalid * D * NQ; t += TS) p.qq[(size_t)g0 * D * NQ + t] = sr[t];
-    for (int j = tl; j < NF; j += TS) {  // q_f = R q_q
-        double acc[E * D];
-#pragma unroll
-        for (int c = 0; c < E * D; ++c) acc[c] = 0.0;
-        ell_apply<E * D, NQ>(tp.r_idx, tp.r_val, tp.wr, NF, j, sr, acc);
-#pragma unroll
-        for (int c = 0; c < E * D; ++c)
-            if (c < nvalid * D) p.qf[((size_t)g0 * D + c) * NF + j] = acc[c];
     }
 }
 
 // ----------------------------------------------------------------------------- time derivative
 // dudt = M^{-1} V' [ sum_n VT_n(f_n) - R' (B J_f f*) ],  f_n = a_n u - b q_n,
-// f* = a.n {u} + halfλ |a.n| [u] - b {q}.n (LF; BR1 when second order).
+// f* = a.n {u} + halfl |a.n| [u] - b {q}.n (LF; BR1 when second order).
 template <int ELEM, int P>
 struct StdTdLayout {
-    using Sh = Shape<ELEM, P>;
-    static constexpr int E = StdTune<ELEM, P>::E3, D = Sh::D;
-    static constexpr int F = 2 * D * Sh::NQ;  // f_n and G_m, then SumFact Z, W, y, tmp
-    static_assert(F >= Sh::NZ + cmax(Sh::NW, 1) + Sh::NP + Sh::NQ, "mass-solve scratch");
-    static constexpr int f = 0, r = f + E * F, t = r + E * Sh::NQ, d1 = t + E * Sh::NF;
-    static constexpr int size = d1 + D * Sh::N1 * Sh::N1;
+    using G = LineGrid<ELEM, P>;
+    static constexpr int E = StdTune<ELEM, P>::E, D = G::D;
+    static constexpr int f = 0, r = f + E * D * G::NX, t = r + E * D * G::NX, f1 = r + E * D * G::NX + E * G::Sh::NF;
+    static constexpr int size = f1 + LineFact<ELEM, P>::NT1;
 };
 
 template <int ELEM, int P, bool SKEW, bool SECOND>
-__global__ void __launch_bounds__((StdTune<ELEM, P>::TS))
-k_std_td_tensor(TensorParams tp, Ensemble en, double* __restrict__ dudt, RKStage rk) {
-    using Sh = Shape<ELEM, P>;
+__global__ void __launch_bounds__((StdTune<ELEM, P>::TS), std_waves(P))
+    k_std_td_tensor(TensorParams tp, Ensemble en, const double* __restrict__ u, double* __restrict__ dudt, RKStage rk) {
+    using G = LineGrid<ELEM, P>;
+    using LF = LineFact<ELEM, P>;
     using T = StdTune<ELEM, P>;
     using L = StdTdLayout<ELEM, P>;
-    constexpr int E = T::E3, TS = T::TS, D = Sh::D, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF;
-    using SF = SumFact<ELEM, P, TS, E>;
+    constexpr int E = T::E, TS = T::TS, D = G::D, N1 = G::N1, N2 = G::N2, NM = G::NM, NX = G::NX, NP = G::NP,
+                  NQ = G::NQ, NF = G::Sh::NF;
     extern __shared__ double sm[];
     const DevParams& p = tp.base;
     const int tl = threadIdx.x;
-    const int R = en.R;
-    const long long nl = (long long)p.N_e * R;
-    const long long g0 = (long long)element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * E;
-    const int nvalid = (int)(nl - g0 < E ? nl - g0 : E);
-    double *sf = sm + L::f, *sG = sf + E * D * NQ, *sr = sm + L::r, *st = sm + L::t, *sD1 = sm + L::d1;
-    constexpr double h = SKEW ? 0.5 : 1.0;
-    using LN = Lines<ELEM, P>;
-    constexpr int N1 = Sh::N1;
-    for (int t = tl; t < D * N1 * N1; t += TS) sD1[t] = tp.D1[t];
-
-    // volume fluxes f_n and G_l = h W sum_n Lt_ln f_n
-    for (int t = tl; t < E * NQ; t += TS) {
-        const int s = t / NQ, i = t - s * NQ;
-        const long long g = g0 + (s < nvalid ? s : 0);
-        const long long k = g / R;
-        const double bm = SECOND ? member_b(p, en, g) : 0.0;
-        const bool tan = SECOND && en.tangent && ((g % R) & 1) && s < nvalid;
-        const double x = s < nvalid ? p.uq[(size_t)g * NQ + i] : 0.0;
-        double f[D];
+    const Slots<E> sl = slots_of<E>(tp, en);
+    const UniformTable A = uniform_table(tp.VA), B = uniform_table(tp.VB), D1 = uniform_table(tp.D1);
+    double *xf = sm + L::f, *xr = sm + L::r, *st = sm + L::t, *F1 = sm + L::f1;
+    const bool on = tl < E * D * N2;
+    const int ls = on ? tl / (D * N2) : 0, ln = on ? (tl / N2) % D : 0, line = tl % N2;
+    double wt[D][N1];  // requested well before its pass: the last two directions now
+    const double* Wk = p.Lam + ((size_t)sl.element(ls) * D * D + D * ln) * NQ;
+    auto load_wt = [&](auto l) {
+        constexpr int l_ = decltype(l)::value;
 #pragma unroll
-        for (int n = 0; n < D; ++n) {
-            f[n] = p.law.a[n] * x;
+        for (int a = 0; a < N1; ++a)
+            wt[l_][a] = Wk[l_ * NQ + G::template node<l_>(line) + a * G::template node_stride<l_>()];
+    };
+    // and its stage-1 line (column c1 of E D)
+    static_assert(E * D * NM <= TS, "a stage-1 line per thread");
+    const bool on1 = tl < E * D * NM;
+    const int c1 = tl / NM, m1 = tl % NM;
+    const auto md1 = LF::modes(tp.lines.mode, m1);
+    auto member_b = [&](int s) { return en.b ? en.b[sl.member(s)] : p.b; };
+    auto is_tangent = [&](int s) { return SECOND && en.tangent && (sl.member(s) & 1); };
+    // this thread's facet nodes: the neighbours first (their states hang on them)
+    constexpr int IT = (E * NF + TS - 1) / TS;
+    unsigned gns[IT];
+    int jns[IT];
+#pragma unroll
+    for (int q = 0; q < IT; ++q) {
+        const int t = min(tl + q * TS, E * NF - 1), s = t / NF;
+        gns[q] = neighbour<NF>(p, sl, s, t - s * NF, jns[q]);
+    }
+    // modal u and q_n of the stage-1 line (slot s1, component n1), used after the facets
+    const int cc = min(c1, E * D - 1), s1 = cc / D, n1 = cc - s1 * D;
+    double xm[N1], qm[N1];
+    {
+        const double* um = u + sl.row(s1, p.N_e) * NP + md1.off;
+#pragma unroll
+        for (int b = 0; b < N1; ++b) xm[b] = um[min(b, md1.lim)];
+        if constexpr (SECOND) {
+            const double* q = p.qq + ((size_t)sl.lane(s1) * D + n1) * NP + md1.off;
+#pragma unroll
+            for (int b = 0; b < N1; ++b) qm[b] = q[min(b, md1.lim)];
+        }
+    }
+    // facet values 1/2 B sum_n nJf_n (R f_n) - B J_f f* (the first term with the skew form only)
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int t = tl + it * TS;
+        if (t >= E * NF) break;
+        const int s = t / NF, j = t - s * NF, jn = jns[it];
+        const unsigned g = sl.lane(s), gn = gns[it];
+        const double um = p.uf[(size_t)g * NF + j], up = p.uf[(size_t)gn * NF + jn];
+        const double* nJ = p.nJf + (size_t)sl.element(s) * D * NF + D * j;
+        double an = 0.0;  // J_f a.n
+#pragma unroll
+        for (int m = 0; m < D; ++m) an += p.law.a[m] * nJ[m];
+        double val = -0.5 * an * (SKEW ? up : um + up);
+        if (p.law.inviscid_flux == 1) val -= p.law.half_lambda * fabs(an) * (um - up);
+        if constexpr (SECOND) {
+            const double bm = member_b(s);
+            const bool tan = is_tangent(s);
+            double qn = 0.0;
+#pragma unroll
+            for (int m = 0; m < D; ++m) {
+                double q = bm * p.qf[((size_t)gn * D + m) * NF + jn];
+                if (!SKEW) q += bm * p.qf[((size_t)g * D + m) * NF + j];
+                if (tan) {  // + the pair's u at unit b
+                    q += p.qf[((size_t)(gn - 1) * D + m) * NF + jn];
+                    if (!SKEW) q += p.qf[((size_t)(g - 1) * D + m) * NF + j];
+                }
+                qn += q * nJ[m];
+            }
+            val += 0.5 * qn;
+        }
+        st[t] = p.B[j] * val;
+    }
+    LF::stage_tables(tp.lines, F1, tl, TS);
+    load_wt(Dir<D - 1>{});
+    if constexpr (D == 3) load_wt(Dir<1>{});
+    {  // modal f_n = a_n u - b q_n
+        const double an = n1 == 0 ? p.law.a[0] : n1 == 1 ? p.law.a[1] : p.law.a[2];
+        const double bm = SECOND ? member_b(s1) : 0.0;
+        const bool tan = is_tangent(s1);
+#pragma unroll
+        for (int b = 0; b < N1; ++b) {
+            xm[b] *= an;
             if constexpr (SECOND) {
-                f[n] -= bm * (s < nvalid ? p.qq[((size_t)g * D + n) * NQ + i] : 0.0);
-                if (tan) f[n] -= p.qq[((size_t)(g - 1) * D + n) * NQ + i];  // dR/db(u) of the pair's u
+                xm[b] -= bm * qm[b];
+                if (tan)  // dR/db(u) of the pair's u
+                    xm[b] -= p.qq[((size_t)sl.lane(s1) * D + n1 - D) * NP + md1.off + min(b, md1.lim)];
             }
-            sf[(s * D + n) * NQ + i] = f[n];
+            if (b > md1.lim) xm[b] = 0.0;
         }
-        const double* Lk = p.Lam + (size_t)k * NQ * D * D;
-        const double hw = h * p.W[i];
-#pragma unroll
-        for (int m = 0; m < D; ++m) {
-            double a = 0.0;
-#pragma unroll
-            for (int n = 0; n < D; ++n) a += Lk[i + NQ * (m + D * n)] * f[n];
-            sG[(s * D + m) * NQ + i] = hw * a;
-        }
-    }
-    // facet values: 1/2 B sum_n nJf_n (R f_n) - B J_f f*
-    for (int t = tl; t < E * NF; t += TS) {
-        const int s = t / NF, j = t - s * NF;
-        double val = 0.0;
-        if (s < nvalid) {
-            const long long g = g0 + s;
-            const long long k = g / R;
-            int jn;
-            const long long gn = neighbour(p, R, g, NF, j, jn);
-            const double um = p.uf[(size_t)g * NF + j], up = p.uf[(size_t)gn * NF + jn];
-            const double jf = p.Jf[(size_t)k * NF + j];
-            const double* nJ = p.nJf + (size_t)k * D * NF + D * j;
-            double an = 0.0;
-#pragma unroll
-            for (int m = 0; m < D; ++m) an += p.law.a[m] * nJ[m];
-            an /= jf;  // a . n
-            double fs = 0.5 * an * (um + up);
-            if (p.law.inviscid_flux == 1) fs += p.law.half_lambda * fabs(an) * (um - up);
-            double surf = SKEW ? an * jf * um : 0.0;  // sum_n nJf_n a_n u^-
-            if constexpr (SECOND) {
-                const double bm = member_b(p, en, g);
-                double qn = 0.0, qm = 0.0;
-#pragma unroll
-                for (int m = 0; m < D; ++m) {
-                    const double qi = p.qf[((size_t)g * D + m) * NF + j];
-                    const double qo = p.qf[((size_t)gn * D + m) * NF + jn];
-                    qn += (qi + qo) * nJ[m];
-                    qm += qi * nJ[m];
-                }
-                qn *= bm;
-                qm *= bm;
-                if (en.tangent && ((g % R) & 1)) {  // + the pair's u at unit b
-#pragma unroll
-                    for (int m = 0; m < D; ++m) {
-                        const double qi = p.qf[((size_t)(g - 1) * D + m) * NF + j];
-                        const double qo = p.qf[((size_t)(gn - 1) * D + m) * NF + jn];
-                        qn += (qi + qo) * nJ[m];
-                        qm += qi * nJ[m];
-                    }
-                }
-                fs -= 0.5 * qn / jf;
-                if (SKEW) surf -= qm;
-            }
-            val = 0.5 * p.B[j] * surf - p.B[j] * jf * fs;
-        }
-        st[t] = val;
     }
     __syncthreads();
-    // r = sum_l D1_l' G_l - h W sum_{l,n} Lt_ln (D1_l f_n) + R' t
-    for (int i = tl; i < NQ; i += TS) {
-        double acc[E];
+    if (on1) {  // stage 1 of V f_n
+        double y[N1];
+        LF::up1(F1, m1, xm, y);
+        line_store<N1, 1>(xf + c1 * NX + md1.base, y);
+    }
+    face_transpose<ELEM, P, E, TS>(tp.faces, st);
+    __syncthreads();
+    if constexpr (G::TET) {
+        LF::template up2<E * D, TS>(reload(B), xf);
+        __syncthreads();
+    }
+    double wj[N1];  // W / J along this thread's line, for the mass solve
+    auto load_woj = [&]() {
+        const double* w = tp.WoJ + (size_t)sl.element(ls) * NQ + G::template node<0>(line);
 #pragma unroll
-        for (int s = 0; s < E; ++s) acc[s] = 0.0;
-#pragma unroll 1
-        for (int l = 0; l < D; ++l) {
-            const int sl = LN::stride(l), a = LN::coord(i, l), base = i - a * sl;
-#pragma unroll
-            for (int bb = 0; bb < N1; ++bb) {
-                const double dv = sD1[(l * N1 + bb) * N1 + a];
-#pragma unroll
-                for (int s = 0; s < E; ++s) acc[s] += dv * sG[(s * D + l) * NQ + base + bb * sl];
-            }
-            if constexpr (SKEW) {
-                double y[E][D];
-#pragma unroll
-                for (int s = 0; s < E; ++s)
-#pragma unroll
-                    for (int n = 0; n < D; ++n) y[s][n] = 0.0;
-                const double* drow = sD1 + (l * N1 + a) * N1;
-#pragma unroll
-                for (int bb = 0; bb < N1; ++bb) {
-                    const double dv = drow[bb];
-#pragma unroll
-                    for (int s = 0; s < E; ++s)
-#pragma unroll
-                        for (int n = 0; n < D; ++n) y[s][n] += dv * sf[(s * D + n) * NQ + base + bb * sl];
-                }
-                const double hw = h * p.W[i];
-#pragma unroll
-                for (int s = 0; s < E; ++s) {
-                    const long long k = (g0 + (s < nvalid ? s : 0)) / R;
-                    const double* Lk = p.Lam + (size_t)k * NQ * D * D;
-                    double c = 0.0;
-#pragma unroll
-                    for (int n = 0; n < D; ++n) c += Lk[i + NQ * (l + D * n)] * y[s][n];
-                    acc[s] -= hw * c;
-                }
+        for (int a = 0; a < N1; ++a) wj[a] = w[a * G::template node_stride<0>()];
+    };
+    const double* xc = xf + (ls * D + ln) * NX;
+    double* rc = xr + (ls * D + ln) * NX;
+    if (on) {
+        double* X = xf + (ls * D + ln) * NX + G::template base<0>(line);
+        double x[N1], y[N1];
+        line_load<N1, G::S1>(X, x);
+        line_apply<N1, false>(reload(A), x, y);
+        line_store<N1, G::S1>(X, y);
+    }
+    __syncthreads();
+    auto pass = [&](auto l) {
+        constexpr int l_ = decltype(l)::value;
+        if constexpr (l_ == D - 1) load_wt(Dir<0>{});
+        if constexpr (l_ == 1) load_woj();
+        if (on) {
+            double r[N1];
+            // R' of the facet values joins component 0
+            volume_line<ELEM, P, l_, SKEW, 1>(reload(D1), tp.faces, xc, wt[l_], ln == 0 ? st + ls * NF : nullptr,
+                                              line, rc, r);
+            if constexpr (l_ == 0) {
+                double w[N1];
+                line_apply<N1, true>(reload(A), r, w);
+                line_store<N1, G::S1>(rc + G::template base<0>(line), w);
+            } else {
+                line_store<N1, G::template stride<l_>()>(rc + G::template base<l_>(line), r);
             }
         }
-        ell_apply<E, NF>(tp.rt_idx, tp.rt_val, tp.wrt, NQ, i, st, acc);
+        __syncthreads();
+    };
+    if constexpr (D == 3) pass(Dir<2>{});
+    pass(Dir<1>{});
+    pass(Dir<0>{});
+    // the D components add up in the next stage of V'; then the mass solve of one column per slot
+    if constexpr (G::TET) {
+        LF::template down2<E, TS, D, D>(reload(B), xr);
+        __syncthreads();
+    }
+    mass_middle<ELEM, P, TS, E, D, G::TET ? 1 : D>(tp, F1, xr, on1, c1, m1, md1, on, ls * D + ln, line, wj);
+    if (on1 && c1 % D == 0 && sl.valid(c1 / D)) {
+        const int s = c1 / D;
+        const auto& md = md1;
+        const size_t row = sl.row(s, p.N_e), o = row * NP + md.off;
+        double x[N1], y[N1];
+        line_load<N1, 1>(xr + s * D * NX + md.base, x);
+        LF::down1(F1, m1, x, y);
+        const double dt = rk.dt_e ? rk.dt_e[row] : rk.dt;
 #pragma unroll
-        for (int s = 0; s < E; ++s) sr[s * NQ + i] = acc[s];
-    }
-    __syncthreads();
-    // mass solve: o = V' (W/J o V (V' r))
-    double* sZ = sf;
-    double* sW = sZ + E * Sh::NZ;
-    double* sy = sW + E * cmax(Sh::NW, 1);
-    double* sx = sy + E * NP;
-    SF::Vt(tp, tl, sr, sy, sZ, sW);
-    SF::V(tp, tl, sy, sx, sZ, sW);
-    for (int t = tl; t < E * NQ; t += TS) {
-        const int s = t / NQ, i = t - s * NQ;
-        const long long k = (g0 + (s < nvalid ? s : 0)) / R;
-        sx[t] *= p.W[i] / p.Jq[(size_t)k * NQ + i];
-    }
-    __syncthreads();
-    SF::Vt(tp, tl, sx, sy, sZ, sW);
-    for (int t = tl; t < nvalid * NP; t += TS) {
-        const int s = t / NP, j = t - s * NP;
-        const size_t o = state_row(g0 + s, R, p.N_e) * NP + j;
-        if (!rk.active) {
-            dudt[o] = sy[t];
-        } else {
-            const double kt = (rk.A == 0.0 ? 0.0 : rk.A * rk.tmp[o]) + (rk.dt_e ? rk.dt_e[o / NP] : rk.dt) * sy[t];
-            rk.tmp[o] = kt;
-            rk.u[o] += rk.B * kt;
+        for (int b = 0; b < N1; ++b) {
+            if (b > md.lim) continue;
+            if (!rk.active) {
+                dudt[o + b] = y[b];
+            } else {
+                const double kt = (rk.A == 0.0 ? 0.0 : rk.A * rk.tmp[o + b]) + dt * y[b];
+                rk.tmp[o + b] = kt;
+                rk.u[o + b] += rk.B * kt;
+            }
         }
     }
 }
 
 // ----------------------------------------------------------------------------- set-up
-// In place: Lambda_mn -> Lt_ln = sum_m c_lm Lambda_mn at every node of every
-// element (c: N_q x d x d, c[(i d + l) d + m]).
-__global__ void k_collapse_metric(double* __restrict__ Lam, const double* __restrict__ c, int NQ, int D,
+// In place: Lambda_mn -> Wt_ln = h W sum_m c_lm Lambda_mn at every node of every
+// element (c: N_q x d x d, c[(i d + l) d + m]); WoJ = W / J.
+__global__ void k_collapse_metric(double* __restrict__ Lam, const double* __restrict__ c, const double* __restrict__ W,
+                                  const double* __restrict__ Jq, double* __restrict__ WoJ, double h, int NQ, int D,
                                   long long n_nodes) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_nodes) return;
@@ -543,24 +720,26 @@ __global__ void k_collapse_metric(double* __restrict__ Lam, const double* __rest
         for (int n = 0; n < D; ++n) {
             double s = 0.0;
             for (int m = 0; m < D; ++m) s += c[(i * D + l) * D + m] * in[m + 3 * n];
-            out[l + 3 * n] = s;
+            out[l + 3 * n] = s * (h * W[i]);
         }
     for (int l = 0; l < D; ++l)
         for (int n = 0; n < D; ++n) Lk[i + NQ * (l + D * n)] = out[l + 3 * n];
+    WoJ[t] = W[i] / Jq[t];
 }
 
-hipError_t collapse_metric(double* Lam, const double* c, int NQ, int D, int N_e, hipStream_t s) {
+hipError_t collapse_metric(double* Lam, const double* c, const double* W, const double* Jq, double* WoJ, double h,
+                           int NQ, int D, int N_e, hipStream_t s) {
     const long long n = (long long)NQ * N_e;
-    hipLaunchKernelGGL(k_collapse_metric, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, Lam, c, NQ, D, n);
+    hipLaunchKernelGGL(k_collapse_metric, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, Lam, c, W, Jq, WoJ, h, NQ,
+                       D, n);
     return hipGetLastError();
 }
 
 // ----------------------------------------------------------------------------- launch
 template <int ELEM, int P>
 size_t std_tensor_lds(int which) {
-    if (which == 0) return sizeof(double) * StdNodalLayout<ELEM, P>::size;
-    if (which == 1) return sizeof(double) * cmax(StdAuxLayout<ELEM, P, true>::size, StdAuxLayout<ELEM, P, false>::size);
-    if (which == 3) return sizeof(double) * StdAuxLayout<ELEM, P, true>::size;
+    if (which == 0) return sizeof(double) * (StdTune<ELEM, P>::E1 * (LineGrid<ELEM, P>::NX + LineGrid<ELEM, P>::Sh::NF) + LineFact<ELEM, P>::NT1);
+    if (which == 1) return sizeof(double) * StdAuxLayout<ELEM, P>::size;
     return sizeof(double) * StdTdLayout<ELEM, P>::size;
 }
 
@@ -568,37 +747,27 @@ template <int ELEM, int P, bool SKEW, bool SECOND>
 hipError_t launch_std_tensor_t(const TensorParams& tp, const Ensemble& en, const double* u, double* dudt,
                                const RKStage& rk, hipStream_t s, int which) {
     using T = StdTune<ELEM, P>;
-    static bool attr_set = false;
-    const size_t l0 = std_tensor_lds<ELEM, P>(0), l1 = std_tensor_lds<ELEM, P>(SKEW ? 3 : 1),
-                 l2 = std_tensor_lds<ELEM, P>(2);
-    if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_std_nodal_tensor<ELEM, P>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)l0);
-        if (e == hipSuccess && SECOND)
-            e = hipFuncSetAttribute((const void*)k_std_aux_tensor<ELEM, P, SKEW>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)l1);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)k_std_td_tensor<ELEM, P, SKEW, SECOND>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)l2);
-        if (e != hipSuccess) return e;
-        attr_set = true;
-    }
+    static_assert(sizeof(double) * StdTdLayout<ELEM, P>::size <= 64 * 1024 &&
+                      sizeof(double) * StdAuxLayout<ELEM, P>::size <= 64 * 1024 &&
+                      sizeof(double) * (T::E1 * (LineGrid<ELEM, P>::NX + LineGrid<ELEM, P>::Sh::NF) + LineFact<ELEM, P>::NT1) <= 64 * 1024,
+                  "within the default dynamic LDS limit");
     const long long nl = (long long)tp.base.N_e * en.R;
+    auto blocks = [&](int e) { return dim3((unsigned)((nl + e - 1) / e)); };
     if (which & 1) {
-        const int nb = (int)((nl + T::E1 - 1) / T::E1);
-        hipLaunchKernelGGL((k_std_nodal_tensor<ELEM, P>), dim3(nb), dim3(T::TS), l0, s, tp, en, u);
+        hipLaunchKernelGGL((k_std_nodal_tensor<ELEM, P>), blocks(T::E1), dim3(T::TS1), (std_tensor_lds<ELEM, P>(0)), s,
+                           tp, en, u);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
     if (which & 2) {
         if (SECOND) {
-            const int nb = (int)((nl + T::E2 - 1) / T::E2);
-            hipLaunchKernelGGL((k_std_aux_tensor<ELEM, P, SKEW>), dim3(nb), dim3(T::TS), l1, s, tp, en);
+            hipLaunchKernelGGL((k_std_aux_tensor<ELEM, P, SKEW>), blocks(T::E), dim3(T::TS),
+                               (std_tensor_lds<ELEM, P>(1)), s, tp, en, u);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         }
-        const int nb = (int)((nl + T::E3 - 1) / T::E3);
-        hipLaunchKernelGGL((k_std_td_tensor<ELEM, P, SKEW, SECOND>), dim3(nb), dim3(T::TS), l2, s, tp, en, dudt, rk);
+        hipLaunchKernelGGL((k_std_td_tensor<ELEM, P, SKEW, SECOND>), blocks(T::E), dim3(T::TS),
+                           (std_tensor_lds<ELEM, P>(2)), s, tp, en, u, dudt, rk);
         return hipGetLastError();
     }
     return hipSuccess;
@@ -619,15 +788,13 @@ hipError_t launch_std_tensor_p(const TensorParams& tp, const Ensemble& en, const
     SSE_CASE(ELEM_TRI, 6) SSE_CASE(ELEM_TET, 2) SSE_CASE(ELEM_TET, 3) SSE_CASE(ELEM_TET, 4)          \
     SSE_CASE(ELEM_TET, 5)
 
-// largest LDS of the three kernels, or 0 if (elem, P) has no compiled kernels
-size_t std_tensor_config(int elem, int P) {
-#define SSE_CASE(E_, PP)                                                                              \
-    if (elem == E_ && P == PP)                                                                        \
-        return cmax(cmax((int)std_tensor_lds<E_, PP>(0), (int)std_tensor_lds<E_, PP>(1)),             \
-                    (int)std_tensor_lds<E_, PP>(2));
+// (elem, P) has compiled kernels
+bool std_tensor_config(int elem, int P) {
+#define SSE_CASE(E_, PP) \
+    if (elem == E_ && P == PP) return true;
     SSE_STD_CASES
 #undef SSE_CASE
-    return 0;
+    return false;
 }
 
 hipError_t launch_std_tensor(const TensorParams& tp, int R, const double* b_member, int tangent, const double* u,
