@@ -386,6 +386,122 @@ std::vector<double> warped_dense(const sse_desc* D) {
     return V;
 }
 
+// Stage-1 tables of the line-by-line sum factorisation (LineTables), from the warped-product
+// factors of V
+int upload_lines(sse_handle* h, const sse_desc* D, sse::LineTables* lt) {
+    const int P = D->V_p, n1 = P + 1;
+    const bool tet = D->d == 3;
+    struct Lane {
+        int b1, b2, off, lim;  // lim: last b of the line
+    };
+    std::vector<Lane> lanes;
+    int off = 0;
+    for (int b1 = 0; b1 <= P; ++b1)
+        for (int b2 = 0; b2 <= (tet ? P - b1 : 0); ++b2) {
+            const int lim = P - b1 - b2;
+            lanes.push_back({b1, b2, off, lim});
+            off += lim + 1;
+        }
+    std::stable_sort(lanes.begin(), lanes.end(), [](const Lane& a, const Lane& b) { return a.lim > b.lim; });
+    std::vector<int> mode;
+    for (const Lane& l : lanes) mode.push_back(l.off | l.b1 << 16 | l.b2 << 24);
+    std::vector<double> F1;
+    for (int b = 0; b <= P; ++b)
+        for (int a = 0; a < n1; ++a)
+            for (const Lane& l : lanes)
+                if (l.lim >= b)
+                    F1.push_back(tet ? D->V_C[a + n1 * (l.b1 + n1 * (l.b2 + n1 * b))] : D->V_B[a + n1 * (l.b1 + n1 * b)]);
+    int rc;
+    if ((rc = upload(h, F1, &lt->F1)) || (rc = upload(h, mode, &lt->mode))) return rc;
+    return 0;
+}
+
+// R as line ends and an interpolation on each face (FaceTables). For each face the direction
+// along which its rows of R factorise, R_f[j, (t, a)] = M[j, t] w[a]; structured = false when a
+// face has none (to 1e-12 of its largest entry).
+int upload_faces(sse_handle* h, const sse_desc* D, sse::FaceTables* ft, bool& structured) {
+    const int n1 = D->V_p + 1, d = D->d, nq = D->N_q, nf = D->N_f, nfac = D->N_fac, n2 = nq / n1;
+    structured = false;
+    if (nf != nfac * n2 || nfac > 4) return 0;
+    auto R = [&](int j, int i) { return D->R[j + (size_t)nf * i]; };
+    std::vector<double> w((size_t)nfac * n1, 0.0), Pf((size_t)nfac * n1 * n1, 0.0);
+    ft->general = 0;
+    std::vector<std::vector<std::pair<int, double>>> mrows(nf), mtrows(nf);
+    for (int f = 0; f < nfac; ++f) {
+        bool found = false;
+        for (int l = 0; l < d && !found; ++l) {
+            int st = 1;
+            for (int t = l + 1; t < d; ++t) st *= n1;
+            auto node = [&](int t, int a) { return (t / st) * st * n1 + a * st + t % st; };  // line t of direction l
+            int jm = 0, tm = 0;
+            double big = 0.0;  // the line with the largest entry gives w, scaled to sum 1
+            for (int j = 0; j < n2; ++j)
+                for (int t = 0; t < n2; ++t)
+                    for (int a = 0; a < n1; ++a)
+                        if (std::fabs(R(f * n2 + j, node(t, a))) > big) {
+                            big = std::fabs(R(f * n2 + j, node(t, a)));
+                            jm = j;
+                            tm = t;
+                        }
+            double sum = 0.0, sq = 0.0;
+            for (int a = 0; a < n1; ++a) sum += R(f * n2 + jm, node(tm, a));
+            if (big == 0.0 || std::fabs(sum) < 1e-8 * big) continue;
+            for (int a = 0; a < n1; ++a) {
+                w[(size_t)f * n1 + a] = R(f * n2 + jm, node(tm, a)) / sum;
+                sq += w[(size_t)f * n1 + a] * w[(size_t)f * n1 + a];
+            }
+            std::vector<double> M((size_t)n2 * n2, 0.0);
+            double worst = 0.0;
+            for (int j = 0; j < n2; ++j)
+                for (int t = 0; t < n2; ++t) {
+                    double m = 0.0;
+                    for (int a = 0; a < n1; ++a) m += R(f * n2 + j, node(t, a)) * w[(size_t)f * n1 + a];
+                    m /= sq;
+                    for (int a = 0; a < n1; ++a)
+                        worst = std::max(worst, std::fabs(R(f * n2 + j, node(t, a)) - m * w[(size_t)f * n1 + a]));
+                    M[(size_t)j * n2 + t] = m;
+                }
+            if (worst > 1e-12 * big) continue;
+            found = true;
+            ft->dir[f] = l;
+            // I, I x P or neither (to rounding: 1e-13 of the largest entry, which is about 1)
+            bool ident = true, kron = true;
+            for (int j = 0; j < n2; ++j)
+                for (int t = 0; t < n2; ++t) {
+                    const double m = M[(size_t)j * n2 + t];
+                    const double p = j / n1 == t / n1 ? M[(size_t)(j % n1) * n2 + t % n1] : 0.0;
+                    if (std::fabs(m - (j == t ? 1.0 : 0.0)) > 1e-13) ident = false;
+                    if (std::fabs(m - p) > 1e-13) kron = false;
+                }
+            ft->kind[f] = ident ? 0 : 1;
+            if (!ident && (!kron || d == 2)) ft->general = 1;
+            for (int a = 0; a < n1; ++a)
+                for (int b = 0; b < n1; ++b) Pf[((size_t)f * n1 + a) * n1 + b] = M[(size_t)a * n2 + b];
+            for (int j = 0; j < n2; ++j)
+                for (int t = 0; t < n2; ++t) {
+                    double m = M[(size_t)j * n2 + t];
+                    bool any = false;  // a zero block of R is no entry
+                    for (int a = 0; a < n1; ++a) any |= R(f * n2 + j, node(t, a)) != 0.0;
+                    if (!any) continue;
+                    if (std::fabs(m - 1.0) < 4e-16) m = 1.0;
+                    mrows[f * n2 + j].push_back({f * n2 + t, m});
+                    mtrows[f * n2 + t].push_back({f * n2 + j, m});
+                }
+        }
+        if (!found) return 0;
+    }
+    std::vector<int> mi, mti;
+    std::vector<double> mv, mtv;
+    ell(mrows, ft->m_w, mi, mv);
+    ell(mtrows, ft->mt_w, mti, mtv);
+    int rc;
+    if ((rc = upload(h, w, &ft->w)) || (rc = upload(h, Pf, &ft->P)) || (rc = upload(h, mi, &ft->m_idx)) || (rc = upload(h, mv, &ft->m_val)) ||
+        (rc = upload(h, mti, &ft->mt_idx)) || (rc = upload(h, mtv, &ft->mt_val)))
+        return rc;
+    structured = true;
+    return 0;
+}
+
 // Set up the compile-time-shaped tensor kernels when the discretisation is one
 // of the compiled (element, degree) shapes; returns 0 (and leaves use_tensor
 // false) when it is not.
@@ -528,126 +644,13 @@ int build_tensor(sse_handle* h, const sse_desc* D) {
         (rc = upload(h, VB, &T.VB)))
         return rc;
     if (d == 3 && (rc = upload(h, VC, &T.VC))) return rc;
+    bool structured = false;
+    if ((rc = upload_lines(h, D, &T.lines)) || (rc = upload_faces(h, D, &T.faces, structured))) return rc;
+    if (!structured) return 0;
     T.xcd_remap = 1;
     if (cfg.lds1 > 160 * 1024 || cfg.lds2 > 160 * 1024) return 0;
     if (T.wv > 16 || T.wf > 16 || T.wrt > 10) return 0;  // TENSOR_MAXW, TENSOR_MAXR
     h->use_tensor = true;
-    return 0;
-}
-
-// Stage-1 tables of the line-by-line sum factorisation (LineTables), from the warped-product
-// factors of V
-int upload_lines(sse_handle* h, const sse_desc* D, sse::LineTables* lt) {
-    const int P = D->V_p, n1 = P + 1;
-    const bool tet = D->d == 3;
-    struct Lane {
-        int b1, b2, off, lim;  // lim: last b of the line
-    };
-    std::vector<Lane> lanes;
-    int off = 0;
-    for (int b1 = 0; b1 <= P; ++b1)
-        for (int b2 = 0; b2 <= (tet ? P - b1 : 0); ++b2) {
-            const int lim = P - b1 - b2;
-            lanes.push_back({b1, b2, off, lim});
-            off += lim + 1;
-        }
-    std::stable_sort(lanes.begin(), lanes.end(), [](const Lane& a, const Lane& b) { return a.lim > b.lim; });
-    std::vector<int> mode;
-    for (const Lane& l : lanes) mode.push_back(l.off | l.b1 << 16 | l.b2 << 24);
-    std::vector<double> F1;
-    for (int b = 0; b <= P; ++b)
-        for (int a = 0; a < n1; ++a)
-            for (const Lane& l : lanes)
-                if (l.lim >= b)
-                    F1.push_back(tet ? D->V_C[a + n1 * (l.b1 + n1 * (l.b2 + n1 * b))] : D->V_B[a + n1 * (l.b1 + n1 * b)]);
-    int rc;
-    if ((rc = upload(h, F1, &lt->F1)) || (rc = upload(h, mode, &lt->mode))) return rc;
-    return 0;
-}
-
-// R as line ends and an interpolation on each face (FaceTables). For each face the direction
-// along which its rows of R factorise, R_f[j, (t, a)] = M[j, t] w[a]; structured = false when a
-// face has none (to 1e-12 of its largest entry).
-int upload_faces(sse_handle* h, const sse_desc* D, sse::FaceTables* ft, bool& structured) {
-    const int n1 = D->V_p + 1, d = D->d, nq = D->N_q, nf = D->N_f, nfac = D->N_fac, n2 = nq / n1;
-    structured = false;
-    if (nf != nfac * n2 || nfac > 4) return 0;
-    auto R = [&](int j, int i) { return D->R[j + (size_t)nf * i]; };
-    std::vector<double> w((size_t)nfac * n1, 0.0), Pf((size_t)nfac * n1 * n1, 0.0);
-    ft->general = 0;
-    std::vector<std::vector<std::pair<int, double>>> mrows(nf), mtrows(nf);
-    for (int f = 0; f < nfac; ++f) {
-        bool found = false;
-        for (int l = 0; l < d && !found; ++l) {
-            int st = 1;
-            for (int t = l + 1; t < d; ++t) st *= n1;
-            auto node = [&](int t, int a) { return (t / st) * st * n1 + a * st + t % st; };  // line t of direction l
-            int jm = 0, tm = 0;
-            double big = 0.0;  // the line with the largest entry gives w, scaled to sum 1
-            for (int j = 0; j < n2; ++j)
-                for (int t = 0; t < n2; ++t)
-                    for (int a = 0; a < n1; ++a)
-                        if (std::fabs(R(f * n2 + j, node(t, a))) > big) {
-                            big = std::fabs(R(f * n2 + j, node(t, a)));
-                            jm = j;
-                            tm = t;
-                        }
-            double sum = 0.0, sq = 0.0;
-            for (int a = 0; a < n1; ++a) sum += R(f * n2 + jm, node(tm, a));
-            if (big == 0.0 || std::fabs(sum) < 1e-8 * big) continue;
-            for (int a = 0; a < n1; ++a) {
-                w[(size_t)f * n1 + a] = R(f * n2 + jm, node(tm, a)) / sum;
-                sq += w[(size_t)f * n1 + a] * w[(size_t)f * n1 + a];
-            }
-            std::vector<double> M((size_t)n2 * n2, 0.0);
-            double worst = 0.0;
-            for (int j = 0; j < n2; ++j)
-                for (int t = 0; t < n2; ++t) {
-                    double m = 0.0;
-                    for (int a = 0; a < n1; ++a) m += R(f * n2 + j, node(t, a)) * w[(size_t)f * n1 + a];
-                    m /= sq;
-                    for (int a = 0; a < n1; ++a)
-                        worst = std::max(worst, std::fabs(R(f * n2 + j, node(t, a)) - m * w[(size_t)f * n1 + a]));
-                    M[(size_t)j * n2 + t] = m;
-                }
-            if (worst > 1e-12 * big) continue;
-            found = true;
-            ft->dir[f] = l;
-            // I, I x P or neither (to rounding: 1e-13 of the largest entry, which is about 1)
-            bool ident = true, kron = true;
-            for (int j = 0; j < n2; ++j)
-                for (int t = 0; t < n2; ++t) {
-                    const double m = M[(size_t)j * n2 + t];
-                    const double p = j / n1 == t / n1 ? M[(size_t)(j % n1) * n2 + t % n1] : 0.0;
-                    if (std::fabs(m - (j == t ? 1.0 : 0.0)) > 1e-13) ident = false;
-                    if (std::fabs(m - p) > 1e-13) kron = false;
-                }
-            ft->kind[f] = ident ? 0 : 1;
-            if (!ident && (!kron || d == 2)) ft->general = 1;
-            for (int a = 0; a < n1; ++a)
-                for (int b = 0; b < n1; ++b) Pf[((size_t)f * n1 + a) * n1 + b] = M[(size_t)a * n2 + b];
-            for (int j = 0; j < n2; ++j)
-                for (int t = 0; t < n2; ++t) {
-                    double m = M[(size_t)j * n2 + t];
-                    bool any = false;  // a zero block of R is no entry
-                    for (int a = 0; a < n1; ++a) any |= R(f * n2 + j, node(t, a)) != 0.0;
-                    if (!any) continue;
-                    if (std::fabs(m - 1.0) < 4e-16) m = 1.0;
-                    mrows[f * n2 + j].push_back({f * n2 + t, m});
-                    mtrows[f * n2 + t].push_back({f * n2 + j, m});
-                }
-        }
-        if (!found) return 0;
-    }
-    std::vector<int> mi, mti;
-    std::vector<double> mv, mtv;
-    ell(mrows, ft->m_w, mi, mv);
-    ell(mtrows, ft->mt_w, mti, mtv);
-    int rc;
-    if ((rc = upload(h, w, &ft->w)) || (rc = upload(h, Pf, &ft->P)) || (rc = upload(h, mi, &ft->m_idx)) || (rc = upload(h, mv, &ft->m_val)) ||
-        (rc = upload(h, mti, &ft->mt_idx)) || (rc = upload(h, mtv, &ft->mt_val)))
-        return rc;
-    structured = true;
     return 0;
 }
 

@@ -75,6 +75,9 @@ struct LineGrid {
     __host__ __device__ static constexpr int node_stride() {
         return !TET ? (L == 0 ? N1 : 1) : (L == 0 ? N1 * N1 : L == 1 ? N1 : 1);
     }
+    __host__ __device__ static constexpr int position(int i) {  // of node i in X
+        return TET ? (i / (N1 * N1)) * S1 + ((i / N1) % N1) * S2 + i % N1 : (i / N1) * S1 + i % N1;
+    }
 };
 
 // y[a] = sum_b M[a N1 + b] x[b] (ROW) or sum_b M[b N1 + a] x[b]; M uniform
@@ -279,5 +282,157 @@ __device__ __forceinline__ void face_row(const FaceTables& ft, int j, const doub
         for (int c = 0; c < NCV; ++c) acc[c] += x[c * XS + j];
     }
 }
+
+// ends of line `line` of every direction but the first, of one column X
+template <int ELEM, int P>
+__device__ __forceinline__ void other_line_ends(const FaceTables& ft, const double* X, int line, double* e) {
+    using G = LineGrid<ELEM, P>;
+    constexpr int N1 = G::N1;
+    double x[N1];
+    line_load<N1, G::template stride<1>()>(X + G::template base<1>(line), x);
+    line_ends<ELEM, P, 1>(ft, x, line, e);
+    if constexpr (G::TET) {
+        line_load<N1, G::template stride<2>()>(X + G::template base<2>(line), x);
+        line_ends<ELEM, P, 2>(ft, x, line, e);
+    }
+}
+
+// The columns of the Euler kernels: a workgroup of TS threads holds NC columns of each of E
+// elements (column s NC + e); a thread has one line of the first direction and one stage-1 line.
+// Every step works on all columns at once and ends with a barrier.
+template <int ELEM, int P>
+struct EulerTune;
+// E and TS: all lines of E elements in one go with few idle threads, and for the Tet enough
+// columns to fill the lanes of stage 2 (E NC N1 of 64)
+#define SSE_EULER_TUNE(E_, PP, e, ts) \
+    template <>                       \
+    struct EulerTune<E_, PP> {        \
+        static constexpr int E = e, TS = ts; \
+    };
+SSE_EULER_TUNE(ELEM_TRI, 2, 5, 64)
+SSE_EULER_TUNE(ELEM_TRI, 3, 4, 64)
+SSE_EULER_TUNE(ELEM_TRI, 4, 3, 64)
+SSE_EULER_TUNE(ELEM_TRI, 5, 2, 64)
+SSE_EULER_TUNE(ELEM_TRI, 6, 2, 64)
+SSE_EULER_TUNE(ELEM_TET, 2, 4, 192)
+SSE_EULER_TUNE(ELEM_TET, 3, 3, 256)
+SSE_EULER_TUNE(ELEM_TET, 4, 2, 256)
+SSE_EULER_TUNE(ELEM_TET, 5, 2, 384)
+#undef SSE_EULER_TUNE
+
+template <int ELEM, int P>
+struct EulerLines {
+    using G = LineGrid<ELEM, P>;
+    using LF = LineFact<ELEM, P>;
+    using T = EulerTune<ELEM, P>;
+    static constexpr int E = T::E, TS = T::TS, NC = G::Sh::NC, NCOL = E * NC, N1 = G::N1, N2 = G::N2, NM = G::NM,
+                         NX = G::NX;
+    static_assert(NCOL * N2 <= TS && NCOL * NM <= TS, "a line per thread");
+    UniformTable A, B;
+    const double* F1;
+    bool on, on1;
+    int col, line, c1, m1;
+    typename LF::Modes md1;
+
+    __device__ EulerLines(const TensorParams& tp, const double* F1_)
+        : A(uniform_table(tp.VA)), B(uniform_table(tp.VB)), F1(F1_) {
+        const int t = threadIdx.x;
+        on = t < NCOL * N2;
+        on1 = t < NCOL * NM;
+        col = on ? t / N2 : 0;
+        line = t % N2;
+        c1 = on1 ? t / NM : 0;
+        m1 = t % NM;
+        md1 = LF::modes(tp.lines.mode, m1);
+    }
+    // LDS column W / J of each element (all threads; a barrier must follow)
+    template <typename Elem>
+    __device__ static void stage_woj(const DevParams& p, Elem element, double* woj) {
+        constexpr int NQ = G::NQ;
+        for (int t = threadIdx.x; t < E * NQ; t += TS) {
+            const int s = t / NQ, i = t - s * NQ;
+            woj[s * NX + G::position(i)] = p.W[i] * rcp_refined(p.Jq[(size_t)element(s) * NQ + i]);
+        }
+    }
+    __device__ double* line1(double* X) const { return X + c1 * NX + md1.base; }
+    __device__ double* line3(double* X) const { return X + col * NX + G::template base<0>(line); }
+    // stage 2 of V, of V'
+    __device__ void up2(double* X) const {
+        if constexpr (G::TET) {
+            LF::template up2<NCOL, TS>(reload(B), X);
+            __syncthreads();
+        }
+    }
+    __device__ void down2(double* X) const {
+        if constexpr (G::TET) {
+            LF::template down2<NCOL, TS>(reload(B), X);
+            __syncthreads();
+        }
+    }
+    // stage 3 of V: the nodal values; then(y) sees this thread's line before the barrier
+    template <typename F>
+    __device__ void up3(double* X, F then) const {
+        if (on) {
+            double x[N1], y[N1];
+            line_load<N1, G::S1>(line3(X), x);
+            line_apply<N1, false>(reload(A), x, y);
+            line_store<N1, G::S1>(line3(X), y);
+            then(y);
+        }
+        __syncthreads();
+    }
+    // stage 3 of V'
+    __device__ void down3(double* X) const {
+        if (on) {
+            double x[N1], y[N1];
+            line_load<N1, G::S1>(line3(X), x);
+            line_apply<N1, true>(reload(A), x, y);
+            line_store<N1, G::S1>(line3(X), y);
+        }
+        __syncthreads();
+    }
+    // stage 3 of V, W/J (an LDS column per element), stage 3 of V'
+    __device__ void scale3(double* X, const double* woj) const {
+        if (on) {
+            double x[N1], y[N1];
+            line_load<N1, G::S1>(line3(X), x);
+            line_apply<N1, false>(reload(A), x, y);
+            line_load<N1, G::S1>(woj + (col / NC) * NX + G::template base<0>(line), x);
+#pragma unroll
+            for (int a = 0; a < N1; ++a) y[a] *= x[a];
+            line_apply<N1, true>(reload(A), y, x);
+            line_store<N1, G::S1>(line3(X), x);
+        }
+        __syncthreads();
+    }
+    // stage 1 of V', then stage 1 of V
+    __device__ void turn1(double* X) const {
+        if (on1) {
+            double x[N1], y[N1];
+            line_load<N1, 1>(line1(X), x);
+            LF::down1(F1, m1, x, y);
+            LF::up1(F1, m1, y, x);
+            line_store<N1, 1>(line1(X), x);
+        }
+        __syncthreads();
+    }
+    // stage 1 of V from modal coefficients x (zero past the last mode)
+    __device__ void up1(double* X, const double* x) const {
+        if (on1) {
+            double y[N1];
+            LF::up1(F1, m1, x, y);
+            line_store<N1, 1>(line1(X), y);
+        }
+        __syncthreads();
+    }
+    // from stage 1 of V to stage 1 of V: V' (W/J V .) between them, i.e. the weight-adjusted
+    // mass solve (mass_matrix.jl:59-75) of modal values whose stage 1 of V is done
+    __device__ void mass(double* X, const double* woj) const {
+        up2(X);
+        scale3(X, woj);
+        down2(X);
+        turn1(X);
+    }
+};
 
 }  // namespace sse

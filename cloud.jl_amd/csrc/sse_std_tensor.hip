@@ -128,20 +128,6 @@ __device__ __forceinline__ unsigned neighbour(const DevParams& p, const Slots<E>
 template <int V>
 using Dir = std::integral_constant<int, V>;
 
-// ends of line `line` of every direction but the first, of one column X
-template <int ELEM, int P>
-__device__ __forceinline__ void other_line_ends(const FaceTables& ft, const double* X, int line, double* e) {
-    using G = LineGrid<ELEM, P>;
-    constexpr int N1 = G::N1;
-    double x[N1];
-    line_load<N1, G::template stride<1>()>(X + G::template base<1>(line), x);
-    line_ends<ELEM, P, 1>(ft, x, line, e);
-    if constexpr (G::TET) {
-        line_load<N1, G::template stride<2>()>(X + G::template base<2>(line), x);
-        line_ends<ELEM, P, 2>(ft, x, line, e);
-    }
-}
-
 // in place, the facet values t of NCOL columns (NF apart) to M' t; the caller's barrier follows.
 // The lines of the faces of kind 1 go to the last threads of the workgroup (the first ones have
 // stage-1 lines of V in the same phase).

@@ -34,32 +34,32 @@ struct Shape<ELEM_TET, P> {
     static constexpr int NW = (P + 1) * N1 * N1;  // W[b1][a2][a3]
 };
 
-// Launch shape of the two kernels. K2 (time_derivative): team size TS, EPB
-// elements per block, R pairs per thread per pass. K1 (nodal_values): TS1, EPB1.
+// Launch shape of the table-driven time_derivative: team size TS, EPB elements per block, R
+// pairs per thread per pass.
 // V selects among variants of the same (element, degree) compiled for tuning.
 template <int ELEM, int P, int V>
 struct Tune;
-#define SSE_TUNE(E, PP, VV, ts, epb, r, ts1, epb1)                                       \
+#define SSE_TUNE(E, PP, VV, ts, epb, r)                                                \
     template <>                                                                        \
     struct Tune<E, PP, VV> {                                                           \
-        static constexpr int TS = ts, EPB = epb, R = r, TS1 = ts1, EPB1 = epb1;         \
+        static constexpr int TS = ts, EPB = epb, R = r;                                \
     };
-SSE_TUNE(ELEM_TRI, 2, 0, 64, 2, 1, 64, 2)
-SSE_TUNE(ELEM_TRI, 3, 0, 64, 2, 2, 64, 2)
-SSE_TUNE(ELEM_TRI, 4, 0, 64, 2, 3, 64, 2)
-SSE_TUNE(ELEM_TRI, 5, 0, 64, 2, 5, 64, 2)
-SSE_TUNE(ELEM_TRI, 6, 0, 64, 2, 7, 64, 2)
-SSE_TUNE(ELEM_TET, 2, 0, 64, 2, 3, 64, 2)
-SSE_TUNE(ELEM_TET, 3, 0, 128, 1, 3, 64, 2)
-SSE_TUNE(ELEM_TET, 4, 0, 128, 1, 2, 128, 2)
-SSE_TUNE(ELEM_TET, 4, 1, 128, 1, 2, 64, 1)
-SSE_TUNE(ELEM_TET, 4, 2, 128, 1, 2, 128, 2)
-SSE_TUNE(ELEM_TET, 4, 3, 128, 2, 2, 128, 4)
-SSE_TUNE(ELEM_TET, 4, 4, 128, 1, 1, 64, 2)
-SSE_TUNE(ELEM_TET, 5, 0, 256, 1, 2, 256, 1)
-SSE_TUNE(ELEM_TET, 5, 1, 256, 1, 2, 128, 2)
-SSE_TUNE(ELEM_TET, 3, 1, 64, 2, 3, 64, 4)
-SSE_TUNE(ELEM_TRI, 4, 1, 64, 2, 3, 64, 4)
+SSE_TUNE(ELEM_TRI, 2, 0, 64, 2, 1)
+SSE_TUNE(ELEM_TRI, 3, 0, 64, 2, 2)
+SSE_TUNE(ELEM_TRI, 4, 0, 64, 2, 3)
+SSE_TUNE(ELEM_TRI, 5, 0, 64, 2, 5)
+SSE_TUNE(ELEM_TRI, 6, 0, 64, 2, 7)
+SSE_TUNE(ELEM_TET, 2, 0, 64, 2, 3)
+SSE_TUNE(ELEM_TET, 3, 0, 128, 1, 3)
+SSE_TUNE(ELEM_TET, 4, 0, 128, 1, 2)
+SSE_TUNE(ELEM_TET, 4, 1, 128, 1, 2)
+SSE_TUNE(ELEM_TET, 4, 2, 128, 1, 2)
+SSE_TUNE(ELEM_TET, 4, 3, 128, 2, 2)
+SSE_TUNE(ELEM_TET, 4, 4, 128, 1, 1)
+SSE_TUNE(ELEM_TET, 5, 0, 256, 1, 2)
+SSE_TUNE(ELEM_TET, 5, 1, 256, 1, 2)
+SSE_TUNE(ELEM_TET, 3, 1, 64, 2, 3)
+SSE_TUNE(ELEM_TRI, 4, 1, 64, 2, 3)
 #undef SSE_TUNE
 
 // Line-structured operator tables (host-built from the descriptor's S, C and R).

@@ -5,8 +5,9 @@
 // Same algorithm as the reference (src/Solvers/flux_differencing_form.jl), with
 // the work organised for CDNA4:
 //   * V and V' are applied sum-factorised (the WarpedTensorProductMap2D/3D
-//     algorithm of src/MatrixFreeOperators/warped_product_{2d,3d}.jl), one
-//     thread per output point, all variables at once, stages staged in LDS;
+//     algorithm of src/MatrixFreeOperators/warped_product_{2d,3d}.jl): in nodal_values a
+//     line of the tensor grid per thread (sse_lines.h), in time_derivative one thread
+//     per output point, all variables at once, stages staged in LDS;
 //   * the Hadamard sum and the facet correction are one list of unique pairs:
 //     each volume pair (i < j) of the union sparsity of S_1..S_d and each
 //     nonzero C_ij is evaluated exactly once per element; contributions go to
@@ -19,7 +20,7 @@
 // A "team" of TS threads owns one element; a block holds EPB teams.
 #include <hip/hip_runtime.h>
 
-#include "sse_tensor.h"
+#include "sse_lines.h"
 
 namespace sse {
 
@@ -53,173 +54,115 @@ hipError_t launch_weight_adjusted_inverse(const DevParams& p, double* Mw, hipStr
 }
 
 // ----------------------------------------------------------------------------- nodal_values
-// The sum-factorisation temporary Z shares the volume-node array: in V it is dead
-// before the last stage writes the output, in V' the input is dead after the first
-// stage. The modal input u and the modal w share one array (u is dead after u_q = V u).
+// u_q = V u -> w = V' (WJ c2e(u_q)) -> M^{-1} w -> w_q = V w -> u_q = e2c(w_q), u_f = e2c(R w_q),
+// line by line (EulerLines), M^{-1} = V' (W/J V .) by the same transforms: a kept matrix per
+// element would be 38 % of this kernel's memory traffic at Tet p = 4, and a line's transform is
+// cheap. R is the ends of the lines and the interpolation on the faces (FaceTables).
+// With a node per thread (every multiply-add reading LDS, R in table rows) the whole residual
+// took 669 us at 24,576 Tet p = 4 elements and 42.3 us at 8,192 Tri p = 3, now 595 and 27.9 us.
 template <int ELEM, int P>
 struct K1Layout {
+    using L = EulerLines<ELEM, P>;
     using Sh = Shape<ELEM, P>;
-    static constexpr int NC = Sh::NC;
-    static_assert(Sh::NZ <= Sh::NQ, "Z inside the volume-node array");
-    static constexpr int off_a = 0;                                  // NC x NQ (and Z)
-    static constexpr int off_z = off_a;                              // NC x NZ
-    static constexpr int off_W = off_a + NC * Sh::NQ;                // NC x NW
-    static constexpr int off_u = off_W + NC * (Sh::NW > 0 ? Sh::NW : 1);  // NC x NP: u, then w
-    static constexpr int off_w = off_u;
-    static constexpr int size = off_u + NC * Sh::NP;
+    static constexpr int x = 0, woj = x + L::NCOL * L::NX, f1 = woj + L::E * L::NX, e = f1 + L::LF::NT1;
+    static constexpr int size = e + L::NCOL * Sh::NF;
 };
 
-template <int ELEM, int P, int VAR>
-__global__ void __launch_bounds__((Tune<ELEM, P, VAR>::TS1 * Tune<ELEM, P, VAR>::EPB1))
+template <int ELEM, int P>
+__global__ void __launch_bounds__((EulerTune<ELEM, P>::TS), (ELEM == ELEM_TET ? 6 : 1))
 k_nodal_values_tensor(TensorParams tp, const double* __restrict__ u) {
     using Sh = Shape<ELEM, P>;
-    using T = Tune<ELEM, P, VAR>;
-    using SF = SumFact<ELEM, P, T::TS1>;
+    using G = LineGrid<ELEM, P>;
+    using EL = EulerLines<ELEM, P>;
     using L = K1Layout<ELEM, P>;
-    constexpr int D = Sh::D, NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF, TS = T::TS1;
-    extern __shared__ double smem[];
+    constexpr int D = Sh::D, NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF, N1 = G::N1, NX = G::NX;
+    constexpr int E = EL::E, TS = EL::TS, ITQ = (E * NQ + TS - 1) / TS;
+    extern __shared__ double sm[];
     const DevParams& p = tp.base;
-    const int team = threadIdx.x / TS, tl = threadIdx.x - team * TS;
-    const int nb = gridDim.x;
-    const int k = element_of_block(blockIdx.x, nb, tp.xcd_remap) * T::EPB1 + team;
-    const bool valid = k < p.N_e;
-    const int kk = valid ? k : 0;
-    double* sm = smem + team * L::size;
-    double* su = sm + L::off_u;
-    double* sa = sm + L::off_a;
-    double* sw = sm + L::off_w;
-    double* sZ = sm + L::off_z;
-    double* sW = sm + L::off_W;
-    using Ph = Physics<D, LAW_EULER>;
-
-    // the factors of V, shared by the block's teams, after the teams' arrays
-    using VF = VFactors<ELEM, P>;
-    double* sfac = smem + T::EPB1 * L::size;
-    VF::stage(tp, sfac, threadIdx.x, TS * T::EPB1);
-    const TensorParams tq = VF::in_lds(tp, sfac);
-    const double* uk = u + (size_t)kk * NP * NC;
-    for (int t = tl; t < NP * NC; t += TS) su[t] = uk[t];
+    const int tl = threadIdx.x;
+    const int k0 = element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * E, last = p.N_e - 1;
+    auto element = [&](int s) { return min(k0 + s, last); };  // past the last: computed, not stored
+    double *X = sm + L::x, *woj = sm + L::woj, *F1 = sm + L::f1, *es = sm + L::e;
+    EL::LF::stage_tables(tp.lines, F1, tl, TS);
+    const EL el(tp, F1);
+    double J[ITQ], um[N1];
+    {
+        const int s = el.c1 / NC, e = el.c1 - s * NC;
+        const double* uk = u + ((size_t)element(s) * NC + e) * NP + el.md1.off;
+#pragma unroll
+        for (int b = 0; b < N1; ++b) um[b] = b <= el.md1.lim ? uk[b] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < ITQ; ++q) {
+        const int t = min(tl + q * TS, E * NQ - 1), s = t / NQ;
+        J[q] = p.Jq[(size_t)element(s) * NQ + (t - s * NQ)];
+    }
     __syncthreads();
-    SF::V(tq, tl, su, sa, sZ, sW);  // u_q = V u
-    const double* Jk = p.Jq + (size_t)kk * NQ;
+    el.up1(X, um);
+    el.up2(X);
+    el.up3(X, [](const double*) {});  // u_q = V u
     bool ok = true;
-    for (int i = tl; i < NQ; i += TS) {  // w_q = WJ c2e(u_q)
+#pragma unroll
+    for (int q = 0; q < ITQ; ++q) {  // w_q = WJ c2e(u_q)
+        const int t = tl + q * TS;
+        if (t >= E * NQ) break;
+        const int s = t / NQ, i = t - s * NQ;
+        double* x = X + s * NC * NX + G::position(i);
         double ub[NC], wb[NC];
 #pragma unroll
-        for (int e = 0; e < NC; ++e) ub[e] = sa[e * NQ + i];
+        for (int e = 0; e < NC; ++e) ub[e] = x[e * NX];
         ok &= c2e_fast<D>(p.law, ub, wb);
-        const double wj = p.W[i] * Jk[i];
+        const double W = p.W[i], wj = W * J[q];
+        woj[s * NX + G::position(i)] = W * rcp_refined(J[q]);
 #pragma unroll
-        for (int e = 0; e < NC; ++e) sa[e * NQ + i] = wb[e] * wj;
+        for (int e = 0; e < NC; ++e) x[e * NX] = wb[e] * wj;
     }
     __syncthreads();
-    // the kept weight-adjusted inverse is staged where u_q and the temporary W were
-    constexpr bool MW = NP * NP <= L::off_u - L::off_a;
-    MassPrefetch<NP, TS> pre;
-    if constexpr (MW) {
-        if (tp.Mw) mass_prefetch<NP, TS>(tp.Mw + (size_t)kk * NP * NP, tl, pre);
-    }
-    SF::Vt(tq, tl, sa, sw, sZ, sW);  // w = V' (WJ w_q)
-    if (MW && tp.Mw) {               // WADG: w = V' diag(W/J) V w with the kept matrix
-        mass_apply_staged<NP, NC, TS>(pre, sa, sw, tl);
-    } else {                         // WADG by sum factorisation: J^{-1} W (V w), then V'
-        SF::V(tq, tl, sw, sa, sZ, sW);
-        for (int i = tl; i < NQ; i += TS) {
-            const double jw = p.W[i] / Jk[i];
+    el.down3(X);
+    el.down2(X);
+    el.turn1(X);
+    el.mass(X, woj);
+    el.up2(X);
+    double* ec = es + el.col * NF;
+    el.up3(X, [&](const double* y) { line_ends<ELEM, P, 0>(tp.faces, y, el.line, ec); });  // w_q = V w
+    if (el.on) other_line_ends<ELEM, P>(tp.faces, X + el.col * NX, el.line, ec);
 #pragma unroll
-            for (int e = 0; e < NC; ++e) sa[e * NQ + i] *= jw;
-        }
-        __syncthreads();
-        SF::Vt(tq, tl, sa, sw, sZ, sW);
-    }
-    SF::V(tq, tl, sw, sa, sZ, sW);   // w_q = V w
-    double* uqk = p.uq + (size_t)kk * NQ * NC;
-    double* ufk = p.uf + (size_t)kk * NF * NC;
-    for (int i = tl; i < NQ; i += TS) {  // u_q = e2c(w_q)
+    for (int q = 0; q < ITQ; ++q) {  // u_q = e2c(w_q)
+        const int t = tl + q * TS;
+        if (t >= E * NQ) break;
+        const int s = t / NQ, i = t - s * NQ;
+        const double* x = X + s * NC * NX + G::position(i);
         double ub[NC], wb[NC];
 #pragma unroll
-        for (int e = 0; e < NC; ++e) wb[e] = sa[e * NQ + i];
+        for (int e = 0; e < NC; ++e) wb[e] = x[e * NX];
         ok &= e2c_fast<D>(p.law, wb, ub);
-        if (valid) {
+        if (k0 + s <= last) {
+            double* uqk = p.uq + (size_t)(k0 + s) * NQ * NC;
 #pragma unroll
             for (int e = 0; e < NC; ++e) uqk[e * NQ + i] = ub[e];
         }
     }
-    // u_f = e2c(R w_q). A row's entries are taken four at a time, their loads issued
-    // together (entries past the table width or the row's end are -1; a group whose first
-    // entry is -1 ends the row)
-    constexpr int G = 8;  // entries per load group
-    auto row_sum = [&](int j, int w_begin, int w_end, double* wb) {
-        for (int w0 = w_begin; w0 < w_end; w0 += G) {
-            int ii[G];
-            double rv[G];
-#pragma unroll
-            for (int q = 0; q < G; ++q) {
-                const bool in = w0 + q < w_end;
-                ii[q] = in ? tp.r_idx[(w0 + q) * NF + j] : -1;
-                rv[q] = in ? tp.r_val[(w0 + q) * NF + j] : 0.0;
-            }
-            if (ii[0] < 0) break;
-#pragma unroll
-            for (int q = 0; q < G; ++q) {
-                if (ii[q] < 0) continue;
-#pragma unroll
-                for (int e = 0; e < NC; ++e) wb[e] += rv[q] * sa[e * NQ + ii[q]];
-            }
-        }
-    };
-    auto store_facet = [&](int j, const double* wb) {
-        double ub[NC];
-        ok &= e2c_fast<D>(p.law, wb, ub);
-        if (valid) {
-#pragma unroll
-            for (int e = 0; e < NC; ++e) ufk[e * NF + j] = ub[e];
-            if (tp.uf_ext) {  // also the neighbour's exterior state: uf_ext at mapP(j, k) = u_f(j, k)
-                const int g = p.mapP[j + (size_t)NF * k];
-                const int kn = g / NF, jn = g - kn * NF;
-                double* uxn = tp.uf_ext + (size_t)kn * NF * NC;
-#pragma unroll
-                for (int e = 0; e < NC; ++e) uxn[e * NF + jn] = ub[e];
-            }
-        }
-    };
-    // On a tet the last facet nodes (those of the face whose nodes each see a whole plane
-    // of volume nodes) have the long rows: the team's otherwise idle threads take the
-    // second half of the last NHELP rows and hand their partial sums over in LDS (the
-    // modal array, dead by now)
-    constexpr int NHELP = NF < TS ? TS - NF : 0;
-    constexpr bool HELP = ELEM == ELEM_TET && NHELP > 0 && NHELP <= NP;
-    if constexpr (HELP) {
-        const int wh = (tp.wr / 2 + 3) / 4 * 4;  // split point (a multiple of four)
-        const bool helper = tl >= NF;
-        const int j = helper ? tl - NHELP : tl, h = j - (NF - NHELP);
-        const bool split = h >= 0;
-        double wb[NC];
+    __syncthreads();
+    for (int t = tl; t < E * NF; t += TS) {  // u_f = e2c(R w_q)
+        const int s = t / NF, j = t - s * NF, k = element(s);
+        const int g = tp.uf_ext ? p.mapP[j + (size_t)NF * k] : 0;
+        double ub[NC], wb[NC];
 #pragma unroll
         for (int e = 0; e < NC; ++e) wb[e] = 0.0;
-        row_sum(j, helper ? wh : 0, (split && !helper) ? wh : tp.wr, wb);
-        if (helper) {
+        face_row<ELEM, P, NC, NF, false>(tp.faces, j, es + s * NC * NF, wb);
+        ok &= e2c_fast<D>(p.law, wb, ub);
+        if (k0 + s > last) continue;
+        double* ufk = p.uf + (size_t)k * NF * NC;
 #pragma unroll
-            for (int e = 0; e < NC; ++e) sw[e * NHELP + h] = wb[e];
-        }
-        __syncthreads();
-        if (!helper) {
-            if (split) {
+        for (int e = 0; e < NC; ++e) ufk[e * NF + j] = ub[e];
+        if (tp.uf_ext) {  // also the neighbour's exterior state: uf_ext at mapP(j, k) = u_f(j, k)
+            const int kn = g / NF, jn = g - kn * NF;
+            double* uxn = tp.uf_ext + (size_t)kn * NF * NC;
 #pragma unroll
-                for (int e = 0; e < NC; ++e) wb[e] += sw[e * NHELP + h];
-            }
-            store_facet(j, wb);
-        }
-    } else {
-        for (int j = tl; j < NF; j += TS) {
-            double wb[NC];
-#pragma unroll
-            for (int e = 0; e < NC; ++e) wb[e] = 0.0;
-            row_sum(j, 0, tp.wr, wb);
-            store_facet(j, wb);
+            for (int e = 0; e < NC; ++e) uxn[e * NF + jn] = ub[e];
         }
     }
-    if (valid && !ok) atomicOr(p.status, 1);
+    if (!ok) atomicOr(p.status, 1);
 }
 
 // ----------------------------------------------------------------------------- time_derivative
@@ -466,7 +409,7 @@ TensorConfig tensor_config_of() {
     using Sh = Shape<ELEM, P>;
     using T = Tune<ELEM, P, VAR>;
     return TensorConfig{T::TS, T::EPB, T::R,
-                        (int)(sizeof(double) * (K1Layout<ELEM, P>::size * T::EPB1 + VFactors<ELEM, P>::size)),
+                        (int)(sizeof(double) * K1Layout<ELEM, P>::size),
                         (int)(sizeof(double) * K2Layout<ELEM, P, VAR>::size * T::EPB), Sh::NQ, Sh::NF, Sh::NP};
 }
 
@@ -477,7 +420,7 @@ hipError_t launch_tensor_t(const TensorParams& tp, const double* u, double* dudt
     const TensorConfig c = tensor_config_of<ELEM, P, VAR>();
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e1 = hipFuncSetAttribute((const void*)k_nodal_values_tensor<ELEM, P, VAR>,
+        hipError_t e1 = hipFuncSetAttribute((const void*)k_nodal_values_tensor<ELEM, P>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, c.lds1);
         hipError_t e2 = hipFuncSetAttribute((const void*)k_time_derivative_tensor<ELEM, P, VAR>,
                                             hipFuncAttributeMaxDynamicSharedMemorySize, c.lds2);
@@ -486,8 +429,9 @@ hipError_t launch_tensor_t(const TensorParams& tp, const double* u, double* dudt
         attr_set = true;
     }
     if (which & 1) {
-        const int nb = (tp.base.N_e + T::EPB1 - 1) / T::EPB1;
-        hipLaunchKernelGGL((k_nodal_values_tensor<ELEM, P, VAR>), dim3(nb), dim3(T::TS1 * T::EPB1), c.lds1, s, tp, u);
+        using N = EulerTune<ELEM, P>;
+        hipLaunchKernelGGL((k_nodal_values_tensor<ELEM, P>), dim3((tp.base.N_e + N::E - 1) / N::E), dim3(N::TS), c.lds1,
+                           s, tp, u);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
