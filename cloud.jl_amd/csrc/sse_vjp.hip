@@ -457,14 +457,23 @@ __global__ void __launch_bounds__(VT) k_vjp_v2(DevParams p, const double* __rest
     if (threadIdx.x == 0) lam_partial[k] = tot;
 }
 
-// out = scale * sum_k partial[k] (+ out when accumulating), in a fixed order
-__global__ void __launch_bounds__(VT) k_vjp_sum(const double* __restrict__ partial, int n, double* __restrict__ out,
-                                                double scale, int accumulate) {
-    __shared__ double red[VT];
+// out = scale * sum_k partial[k] (+ out when accumulating), in a fixed order. One workgroup of
+// the largest size with eight loads of a thread in flight: the sum over 10,368 elements waits
+// for memory latency (13 us with 256 threads and one load at a time).
+constexpr int VSUM = 1024;
+__global__ void __launch_bounds__(VSUM) k_vjp_sum(const double* __restrict__ partial, int n, double* __restrict__ out,
+                                                  double scale, int accumulate) {
+    __shared__ double red[VSUM];
     double s = 0.0;
-    for (int k = threadIdx.x; k < n; k += VT) s += partial[k];
-    const double tot = block_sum_vjp(s, red);
-    if (threadIdx.x == 0) out[0] = (accumulate ? out[0] : 0.0) + scale * tot;
+#pragma unroll 8
+    for (int k = threadIdx.x; k < n; k += VSUM) s += partial[k];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int h = VSUM / 2; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[0] = (accumulate ? out[0] : 0.0) + scale * red[0];
 }
 
 size_t lds_vjp_v1(const DevParams& p) {
@@ -497,13 +506,13 @@ hipError_t launch_vjp_t(const DevParams& p, const double* u, const double* ybar,
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((k_vjp_v2<D>), dim3(p.N_e), dim3(VT), lds_vjp_v2(p), s, p, u, rbar, fbar, ubar, lam_partial);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_vjp_sum, dim3(1), dim3(VT), 0, s, lam_partial, p.N_e, lam_out, lam_scale, accumulate);
+    hipLaunchKernelGGL(k_vjp_sum, dim3(1), dim3(VSUM), 0, s, lam_partial, p.N_e, lam_out, lam_scale, accumulate);
     return hipGetLastError();
 }
 
 hipError_t launch_vjp_sum(const double* lam_partial, int n, double* lam_out, double lam_scale, int accumulate,
                           hipStream_t s) {
-    hipLaunchKernelGGL(k_vjp_sum, dim3(1), dim3(VT), 0, s, lam_partial, n, lam_out, lam_scale, accumulate);
+    hipLaunchKernelGGL(k_vjp_sum, dim3(1), dim3(VSUM), 0, s, lam_partial, n, lam_out, lam_scale, accumulate);
     return hipGetLastError();
 }
 

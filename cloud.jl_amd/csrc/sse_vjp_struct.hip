@@ -3,7 +3,7 @@
 // reverse of the line-structured time derivative (sse_struct.hip) and of the
 // entropy projection, same algebra as the general kernels of sse_vjp.hip.
 //
-//   dudt = M^{-1} V' r_q        ->  rbar = V M^{-1} ybar         (phase V1, sum-factorised)
+//   dudt = M^{-1} V' r_q        ->  rbar = V M^{-1} ybar         (phase V1, line by line)
 //   r_q -= R' f_f               ->  fbar = -R rbar
 //   f_f = B J_f f*(u_f, u_f+)   ->  interface flux adjoint at each facet node, for its own
 //                                   flux and for the neighbour's flux at the shared node
@@ -17,11 +17,13 @@
 // The pull-back through u = e2c(w) at the projected states uses du/dw in closed
 // form from the states' (rho, v, p), so the projection is not recomputed. The
 // facet-correction sums are the only ones whose order varies from run to run
-// (LDS atomics); every other sum has a fixed order.
+// (LDS atomics); every other sum has a fixed order. V1 and V3 apply V and V' to lines of the
+// grid (EulerLines, sse_lines.h); with a node per thread and kept mass matrices they took 40 and
+// 59 us at 10,368 Tet p = 3 elements, now 31 and 38 us.
 #include <hip/hip_runtime.h>
 
 #include "sse_adjoint.h"
-#include "sse_tensor.h"
+#include "sse_lines.h"
 
 namespace sse {
 
@@ -64,15 +66,13 @@ struct VjpLayout {
     static_assert(NC <= D * D && T::TS <= ST, "aliases fit");
 };
 
-// LDS of the reverse projection (phase V3)
+// LDS of V1 and of the reverse projection V3 (EulerLines)
 template <int ELEM, int P>
-struct VjpProjLayout {
-    using Sh = Shape<ELEM, P>;
-    static constexpr int NC = Sh::NC;
-    static constexpr int off_z = 0, off_W = off_z + NC * Sh::NZ, off_y = off_W + NC * (Sh::NW > 0 ? Sh::NW : 1);
-    static constexpr int off_x = off_y + NC * Sh::NP, off_u = off_x + NC * Sh::NQ, off_u0 = off_u + NC * Sh::NP;
-    static constexpr int off_w = off_u0 + NC * Sh::NQ;  // w_q' cotangent
-    static constexpr int size = off_w + NC * Sh::NQ;
+struct VjpLinesLayout {
+    using L = EulerLines<ELEM, P>;
+    static constexpr int x = 0, woj = x + L::NCOL * L::NX, f1 = woj + L::E * L::NX, more = f1 + L::LF::NT1;
+    static constexpr int size1 = more + L::NCOL * L::G::Sh::NF;  // V1: line ends
+    static constexpr int size3 = more + L::NCOL * L::NX;         // V3: V u
 };
 
 }  // namespace
@@ -95,79 +95,61 @@ struct VjpOut {
 // V1: rbar = V M^{-1} ybar (M^{-1} = V' (W / J) V, weight-adjusted), fbar = -R rbar,
 // fbar also into the neighbour's exterior slot [k][e][j] (mapP is an involution)
 template <int ELEM, int P>
-__global__ void __launch_bounds__((VjpTune<ELEM, P>::TS))
+__global__ void __launch_bounds__((EulerTune<ELEM, P>::TS))
 k_vjp_v1_tensor(TensorParams tp, const double* ybar, double* __restrict__ rbar, double* __restrict__ fbar,
                 double* __restrict__ fbar_ext, VjpIn in) {
     using Sh = Shape<ELEM, P>;
-    constexpr int TS = VjpTune<ELEM, P>::TS, NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF;
-    using SF = SumFact<ELEM, P, TS>;
+    using G = LineGrid<ELEM, P>;
+    using EL = EulerLines<ELEM, P>;
+    using L = VjpLinesLayout<ELEM, P>;
+    constexpr int E = EL::E, TS = EL::TS, NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF, N1 = G::N1;
     extern __shared__ double sm[];
     const DevParams& p = tp.base;
-    const int k = element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap), tl = threadIdx.x;
-    double* sy = sm;                 // NC x NP
-    double* sx = sy + NC * NP;       // NC x NQ; also the sum-factorisation temporary Z
-    double* sZ = sx;                 // (dead before V's last stage, and after V''s first)
-    double* sW = sx + NC * NQ;       // NC x NW
-    // the factors of V in LDS after the work arrays
-    using VF = VFactors<ELEM, P>;
-    double* sfac = sW + NC * (Sh::NW > 0 ? Sh::NW : 1);
-    VF::stage(tp, sfac, tl, TS);
-    const TensorParams tq = VF::in_lds(tp, sfac);
-    // the kept weight-adjusted inverse (requested with ybar), staged in x and W
-    constexpr bool MW = NP * NP <= NC * (NQ + Sh::NW);
-    MassPrefetch<NP, TS> pre;
-    if constexpr (MW) {
-        if (tp.Mw) mass_prefetch<NP, TS>(tp.Mw + (size_t)k * NP * NP, tl, pre);
-    }
-    const size_t kb = (size_t)k * NP * NC;
-    for (int t = tl; t < NP * NC; t += TS) {
-        double y = in.a == 0.0 ? 0.0 : in.a * ybar[kb + t];
-        if (in.x) y += in.b * in.x[kb + t];
-        if (in.store) in.store[kb + t] = y;
-        sy[t] = y;
-    }
-    __syncthreads();
-    if (MW && tp.Mw) {  // M^{-1} ybar = V' diag(W/J) V ybar with the kept matrix
-        mass_apply_staged<NP, NC, TS>(pre, sx, sy, tl);
-    } else {
-        SF::V(tq, tl, sy, sx, sZ, sW);
-        const double* Jk = p.Jq + (size_t)k * NQ;
-        for (int i = tl; i < NQ; i += TS) {
-            const double jw = p.W[i] / Jk[i];
+    const int tl = threadIdx.x;
+    const int k0 = element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * E, last = p.N_e - 1;
+    auto element = [&](int s) { return min(k0 + s, last); };  // past the last: computed, not stored
+    double *X = sm + L::x, *woj = sm + L::woj, *F1 = sm + L::f1, *es = sm + L::more;
+    EL::LF::stage_tables(tp.lines, F1, tl, TS);
+    const EL el(tp, F1);
+    double y[N1];
+    {
+        const int s = el.c1 / NC, e = el.c1 - s * NC;
+        const size_t o = ((size_t)element(s) * NC + e) * NP + el.md1.off;
+        const bool mine = el.on1 && k0 + s <= last;
 #pragma unroll
-            for (int e = 0; e < NC; ++e) sx[e * NQ + i] *= jw;
+        for (int b = 0; b < N1; ++b) {
+            y[b] = 0.0;
+            if (b > el.md1.lim) continue;
+            if (in.a != 0.0) y[b] = in.a * ybar[o + b];
+            if (in.x) y[b] += in.b * in.x[o + b];
+            if (in.store && mine) in.store[o + b] = y[b];
         }
-        __syncthreads();
-        SF::Vt(tq, tl, sx, sy, sZ, sW);
     }
-    SF::V(tq, tl, sy, sx, sZ, sW);
-    double* rk = rbar + (size_t)k * NQ * NC;
-    for (int t = tl; t < NQ * NC; t += TS) rk[t] = sx[t];
-    for (int j = tl; j < NF; j += TS) {
-        const int g = p.mapP[j + (size_t)NF * k];
+    EL::stage_woj(p, element, woj);
+    __syncthreads();
+    el.up1(X, y);
+    el.mass(X, woj);  // M^{-1} ybar
+    el.up2(X);
+    double* ec = es + el.col * NF;
+    el.up3(X, [&](const double* r) {
+        const int s = el.col / NC;
+        if (k0 + s <= last) {
+            double* rk = rbar + ((size_t)(k0 + s) * NC + (el.col - s * NC)) * NQ + G::template node<0>(el.line);
+#pragma unroll
+            for (int a = 0; a < N1; ++a) rk[a * G::template node_stride<0>()] = r[a];
+        }
+        line_ends<ELEM, P, 0>(tp.faces, r, el.line, ec);
+    });
+    if (el.on) other_line_ends<ELEM, P>(tp.faces, X + el.col * G::NX, el.line, ec);
+    __syncthreads();
+    for (int t = tl; t < E * NF; t += TS) {
+        const int s = t / NF, j = t - s * NF, k = k0 + s;
+        if (k > last) continue;
+        const int g = p.mapP[j + (size_t)NF * k], kn = g / NF, jn = g - kn * NF;
         double acc[NC];
 #pragma unroll
         for (int e = 0; e < NC; ++e) acc[e] = 0.0;
-        // the row four entries at a time, their loads issued together (entries past the
-        // table width count as padding, index -1; a group whose first entry is padding ends it)
-        for (int w0 = 0; w0 < tp.wr; w0 += 4) {
-            int ii[4];
-            double rv[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const bool in = w0 + q < tp.wr;
-                ii[q] = in ? tp.r_idx[(w0 + q) * NF + j] : -1;
-                rv[q] = in ? tp.r_val[(w0 + q) * NF + j] : 0.0;
-            }
-            if (ii[0] < 0) break;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (ii[q] < 0) continue;
-#pragma unroll
-                for (int e = 0; e < NC; ++e) acc[e] += rv[q] * sx[e * NQ + ii[q]];
-            }
-        }
-        const int kn = g / NF, jn = g - kn * NF;
+        face_row<ELEM, P, NC, NF, false>(tp.faces, j, es + s * NC * NF, acc);
         double* fk = fbar + (size_t)k * NF * NC;
         double* fx = fbar_ext + (size_t)kn * NF * NC;
 #pragma unroll
@@ -197,7 +179,6 @@ k_vjp_v2_tensor(TensorParams tp, StructTables st, double* __restrict__ rbar, con
     using T = VjpTune<ELEM, P>;
     using L = VjpLayout<ELEM, P>;
     using A = EulerAdj<Sh::D>;
-    using SF = SumFact<ELEM, P, T::TS>;
     constexpr int D = Sh::D, NC = Sh::NC, NH = L::NH, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF, NPF = Sh::NPF;
     constexpr int N1 = Sh::N1, TS = T::TS, MAXITEM = L::MAXITEM, SPLIT = T::SPLIT, NT = TS / SPLIT;
     // each unordered line pair once, as in the forward kernel: cyclic offsets
@@ -645,88 +626,81 @@ k_vjp_v2_tensor(TensorParams tp, StructTables st, double* __restrict__ rbar, con
     if (tt == 0) lam_partial[k] = (out.accumulate ? lam_partial[k] : 0.0) + out.scale * red[0];
 }
 
-// V3: the reverse of w_q' = V M^{-1} V' (WJ c2e(V u)), sum-factorised, one element per
-// workgroup: ubar (+)= scale * V' c2e'(V u)' (WJ V M^{-1} V' wbar), M^{-1} = V' (W/J V .).
-// Its own kernel so that these low-register stages run at higher occupancy than V2.
+// V3: the reverse of w_q' = V M^{-1} V' (WJ c2e(V u)): ubar (+)= scale *
+// V' c2e'(V u)' (WJ V M^{-1} V' wbar), M^{-1} = V' (W/J V .). Its own kernel so that these
+// low-register stages run at higher occupancy than V2.
 template <int ELEM, int P>
-__global__ void __launch_bounds__((VjpTune<ELEM, P>::TS))
+__global__ void __launch_bounds__((EulerTune<ELEM, P>::TS))
 k_vjp_v3_tensor(TensorParams tp, const double* __restrict__ u, const double* __restrict__ wbar,
                 double* __restrict__ ubar, VjpOut out) {
     using Sh = Shape<ELEM, P>;
-    using T = VjpTune<ELEM, P>;
-    using L = VjpProjLayout<ELEM, P>;
+    using G = LineGrid<ELEM, P>;
+    using EL = EulerLines<ELEM, P>;
+    using L = VjpLinesLayout<ELEM, P>;
     using A = EulerAdj<Sh::D>;
-    using SF = SumFact<ELEM, P, T::TS>;
-    constexpr int NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, TS = T::TS;
+    constexpr int E = EL::E, TS = EL::TS, NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, N1 = G::N1, NX = G::NX;
     extern __shared__ double sm[];
     const DevParams& p = tp.base;
-    const int k = element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap);
-    const int tt = threadIdx.x;
-    double* sZ = sm + L::off_z;
-    double* sW = sm + L::off_W;
-    double* sy = sm + L::off_y;
-    double* sx = sm + L::off_x;
-    double* su = sm + L::off_u;
-    double* su0 = sm + L::off_u0;
-    double* sw = sm + L::off_w;
-    using VF = VFactors<ELEM, P>;
-    double* sfac = sm + L::size;  // the factors of V in LDS after the work arrays
-    VF::stage(tp, sfac, tt, TS);
-    const TensorParams tq = VF::in_lds(tp, sfac);
-    // the kept weight-adjusted inverse (requested with u and the cotangent), staged in the
-    // temporaries Z and W
-    constexpr bool MW = NP * NP <= L::off_y - L::off_z;
-    MassPrefetch<NP, TS> pre;
-    if constexpr (MW) {
-        if (tp.Mw) mass_prefetch<NP, TS>(tp.Mw + (size_t)k * NP * NP, tt, pre);
-    }
-    const double* uk = u + (size_t)k * NP * NC;
-    const double* wk = wbar + (size_t)k * NQ * NC;
-    for (int t = tt; t < NP * NC; t += TS) su[t] = uk[t];
-    for (int t = tt; t < NQ * NC; t += TS) sw[t] = wk[t];
-    __syncthreads();
-    SF::V(tq, tt, su, su0, sZ, sW);   // V u
-    SF::Vt(tq, tt, sw, sy, sZ, sW);   // V' (w_q' cotangent)
-    const double* Jk = p.Jq + (size_t)k * NQ;
-    if (MW && tp.Mw) {                // M^{-1} = V' (W/J V .) with the kept matrix
-        mass_apply_staged<NP, NC, TS>(pre, sZ, sy, tt);
-    } else {
-        SF::V(tq, tt, sy, sx, sZ, sW);
-        for (int i = tt; i < NQ; i += TS) {
-            const double jw = p.W[i] / Jk[i];
+    const int tl = threadIdx.x;
+    const int k0 = element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * E, last = p.N_e - 1;
+    auto element = [&](int s) { return min(k0 + s, last); };  // past the last: computed, not stored
+    double *X = sm + L::x, *woj = sm + L::woj, *F1 = sm + L::f1, *U = sm + L::more;
+    EL::LF::stage_tables(tp.lines, F1, tl, TS);
+    const EL el(tp, F1);
+    const int s1 = el.c1 / NC, s3 = el.col / NC;
+    const size_t o1 = ((size_t)element(s1) * NC + (el.c1 - s1 * NC)) * NP + el.md1.off;
+    double um[N1], w[N1];
 #pragma unroll
-            for (int e = 0; e < NC; ++e) sx[e * NQ + i] *= jw;
-        }
-        __syncthreads();
-        SF::Vt(tq, tt, sx, sy, sZ, sW);
+    for (int b = 0; b < N1; ++b) um[b] = b <= el.md1.lim ? u[o1 + b] : 0.0;
+    {
+        const double* wk = wbar + ((size_t)element(s3) * NC + (el.col - s3 * NC)) * NQ + G::template node<0>(el.line);
+#pragma unroll
+        for (int a = 0; a < N1; ++a) w[a] = wk[a * G::template node_stride<0>()];
     }
-    SF::V(tq, tt, sy, sx, sZ, sW);    // V (M^{-1} V' w_q'bar), then times WJ and through c2e
-    for (int i = tt; i < NQ; i += TS) {
-        const double wj = p.W[i] * Jk[i];
+    EL::stage_woj(p, element, woj);
+    if (el.on) line_store<N1, G::S1>(el.line3(X), w);
+    __syncthreads();
+    el.up1(U, um);
+    el.up2(U);
+    el.up3(U, [](const double*) {});  // V u
+    el.down3(X);                      // V' (w_q' cotangent)
+    el.down2(X);
+    el.turn1(X);
+    el.mass(X, woj);
+    el.up2(X);
+    el.up3(X, [](const double*) {});  // V (M^{-1} V' w_q'bar), then times WJ and through c2e
+    for (int t = tl; t < E * NQ; t += TS) {
+        const int s = t / NQ, i = t - s * NQ, q = s * NC * NX + G::position(i);
+        const double wj = p.W[i] * p.Jq[(size_t)element(s) * NQ + i];
         double u0[NC], wb[NC], ub[NC];
 #pragma unroll
         for (int e = 0; e < NC; ++e) {
-            u0[e] = su0[e * NQ + i];
-            wb[e] = wj * sx[e * NQ + i];
+            u0[e] = U[q + e * NX];
+            wb[e] = wj * X[q + e * NX];
             ub[e] = 0.0;
         }
         A::c2e_adj(p.law, u0, wb, ub);
 #pragma unroll
-        for (int e = 0; e < NC; ++e) sw[e * NQ + i] = ub[e];
+        for (int e = 0; e < NC; ++e) X[q + e * NX] = ub[e];
     }
     __syncthreads();
-    SF::Vt(tq, tt, sw, sy, sZ, sW);
-    double* outk = ubar + (size_t)k * NP * NC;
-    for (int t = tt; t < NP * NC; t += TS) outk[t] = (out.accumulate ? outk[t] : 0.0) + out.scale * sy[t];
+    el.down3(X);
+    el.down2(X);
+    if (el.on1 && k0 + s1 <= last) {
+        double x[N1], y[N1];
+        line_load<N1, 1>(el.line1(X), x);
+        EL::LF::down1(F1, el.m1, x, y);
+#pragma unroll
+        for (int b = 0; b < N1; ++b)
+            if (b <= el.md1.lim) ubar[o1 + b] = (out.accumulate ? ubar[o1 + b] : 0.0) + out.scale * y[b];
+    }
 }
 
 // ----------------------------------------------------------------------------- launch
 template <int ELEM, int P>
 size_t vjp_tensor_lds(int which) {
-    using Sh = Shape<ELEM, P>;
-    if (which == 1)
-        return sizeof(double) * (Sh::NC * (Sh::NP + Sh::NQ + (Sh::NW > 0 ? Sh::NW : 1)) + VFactors<ELEM, P>::size);
-    if (which == 3) return sizeof(double) * (VjpProjLayout<ELEM, P>::size + VFactors<ELEM, P>::size);
+    if (which == 1) return sizeof(double) * VjpLinesLayout<ELEM, P>::size1;
+    if (which == 3) return sizeof(double) * VjpLinesLayout<ELEM, P>::size3;
     return sizeof(double) * VjpLayout<ELEM, P>::size;
 }
 
@@ -752,8 +726,9 @@ hipError_t launch_vjp_tensor_t(const TensorParams& tp, const StructTables& st, c
         if (e != hipSuccess) return e;
         attr = true;
     }
-    const int nb = tp.base.N_e;
-    hipLaunchKernelGGL((k_vjp_v1_tensor<ELEM, P>), dim3(nb), dim3(T::TS), l1, s, tp, ybar, rbar, fbar, fbar_ext, in);
+    using N = EulerTune<ELEM, P>;
+    const int nb = tp.base.N_e, nl = (nb + N::E - 1) / N::E;
+    hipLaunchKernelGGL((k_vjp_v1_tensor<ELEM, P>), dim3(nl), dim3(N::TS), l1, s, tp, ybar, rbar, fbar, fbar_ext, in);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (st.det)
@@ -764,7 +739,7 @@ hipError_t launch_vjp_tensor_t(const TensorParams& tp, const StructTables& st, c
                            fbar_ext, lam_partial, VjpOut{scale, accumulate});
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_vjp_v3_tensor<ELEM, P>), dim3(nb), dim3(T::TS), l3, s, tp, u, rbar, ubar,
+    hipLaunchKernelGGL((k_vjp_v3_tensor<ELEM, P>), dim3(nl), dim3(N::TS), l3, s, tp, u, rbar, ubar,
                        VjpOut{scale, accumulate});
     return hipGetLastError();
 }
