@@ -53,6 +53,7 @@ struct StructConfig {
 };
 bool struct_config(int elem, int P, StructConfig* c);
 int struct_occupancy(int elem, int P);
+bool struct_keeps_mass(int elem, int P);
 hipError_t launch_struct(const TensorParams& tp, const StructTables& st, double* dudt, const RKStage& rk,
                          hipStream_t s, int n_blocks);
 bool std_tensor_config(int elem, int P);
@@ -619,18 +620,16 @@ int build_tensor(sse_handle* h, const sse_desc* D) {
         for (int o = 0; o < N_f; ++o)
             for (int w = 0; w < (int)fin[ps][o].size(); ++w) ft[((size_t)ps * T.wf + w) * N_f + o] = fin[ps][o][w];
     }
-    // R and R' as ELL tables
-    std::vector<std::vector<std::pair<int, double>>> rrows(N_f), rtrows(N_q);
+    // R' as an ELL table
+    std::vector<std::vector<std::pair<int, double>>> rtrows(N_q);
     for (int j = 0; j < N_f; ++j)
         for (int i = 0; i < N_q; ++i) {
             const double v = D->R[j + (size_t)N_f * i];
             if (v == 0.0) continue;
-            rrows[j].push_back({i, v});
             rtrows[i].push_back({j, v});
         }
-    std::vector<int> r_idx, rt_idx;
-    std::vector<double> r_val, rt_val;
-    ell(rrows, T.wr, r_idx, r_val);
+    std::vector<int> rt_idx;
+    std::vector<double> rt_val;
     ell(rtrows, T.wrt, rt_idx, rt_val);
     const int P1 = D->V_p + 1;
     std::vector<double> VA(D->V_A, D->V_A + (size_t)D->V_M[0] * P1);
@@ -639,7 +638,7 @@ int build_tensor(sse_handle* h, const sse_desc* D) {
     if (d == 3) VC.assign(D->V_C, D->V_C + (size_t)D->V_M[2] * P1 * P1 * P1);
     int rc;
     if ((rc = upload(h, pk, &T.pk)) || (rc = upload(h, cf, &T.cf)) || (rc = upload(h, vt, &T.vt)) ||
-        (rc = upload(h, ft, &T.ft)) || (rc = upload(h, r_idx, &T.r_idx)) || (rc = upload(h, r_val, &T.r_val)) ||
+        (rc = upload(h, ft, &T.ft)) ||
         (rc = upload(h, rt_idx, &T.rt_idx)) || (rc = upload(h, rt_val, &T.rt_val)) || (rc = upload(h, VA, &T.VA)) ||
         (rc = upload(h, VB, &T.VB)))
         return rc;
@@ -1294,9 +1293,10 @@ int create_handle(const sse_desc* D, int members, sse_handle** out) {
     if (only_generic) h->use_tensor = false;
     if (!h->use_tensor) h->use_struct = false;
     // the weight-adjusted mass solve with a kept matrix per element (N_p^2 doubles each; up to
-    // 16 GiB) in place of V, W/J and V' (SSE_MASS_MATRICES=0: off): tensor kernels and the
-    // general entropy-conservative time derivative
-    if ((h->use_tensor || P.ec) && P.has_V && (size_t)N_p * N_p * N_e * sizeof(double) <= ((size_t)16 << 30)) {
+    // 16 GiB) in place of V, W/J and V' (SSE_MASS_MATRICES=0: off): the line-structured time
+    // derivative of small elements and the general entropy-conservative one
+    const bool keeps = h->use_tensor ? h->use_struct && sse::struct_keeps_mass(D->element, D->V_p) : P.ec != 0;
+    if (keeps && P.has_V && (size_t)N_p * N_p * N_e * sizeof(double) <= ((size_t)16 << 30)) {
         const char* menv = getenv("SSE_MASS_MATRICES");
         if (!(menv && menv[0] == '0')) {
             double* Mw = nullptr;
@@ -1344,12 +1344,11 @@ int sse_describe(const sse_handle* h, char* buf, int32_t len) {
                  h->struct_blocks, S.n_items, S.ch, T.wrt, S.det ? " deterministic" : "");
     } else if (h->use_tensor) {
         const sse::TensorParams& T = h->TP;
-        snprintf(buf, len, "tensor elem=%d P=%d variant=%d pairs=%d vol_pairs=%d passes=%d pass_size=%d wv=%d wf=%d wrt=%d wr=%d",
-                 T.elem, T.P, T.variant, T.n_pairs, T.n_vol_pairs, T.n_pass, T.pass_size, T.wv, T.wf, T.wrt, T.wr);
+        snprintf(buf, len, "tensor elem=%d P=%d variant=%d pairs=%d vol_pairs=%d passes=%d pass_size=%d wv=%d wf=%d wrt=%d",
+                 T.elem, T.P, T.variant, T.n_pairs, T.n_vol_pairs, T.n_pass, T.pass_size, T.wv, T.wf, T.wrt);
     } else if (h->use_std_tensor) {
-        snprintf(buf, len, "standard tensor elem=%d P=%d N_e=%d members=%d mapping=%s%s wr=%d wrt=%d", h->TP.elem,
-                 h->TP.P, P.N_e, h->members, P.skew ? "skew" : "standard", P.second_order ? " br1" : "", h->TP.wr,
-                 h->TP.wrt);
+        snprintf(buf, len, "standard tensor elem=%d P=%d N_e=%d members=%d mapping=%s%s", h->TP.elem,
+                 h->TP.P, P.N_e, h->members, P.skew ? "skew" : "standard", P.second_order ? " br1" : "");
     } else if (P.standard) {
         snprintf(buf, len, "standard d=%d N_p=%d N_q=%d N_f=%d N_c=%d N_e=%d mapping=%s%s", P.d, P.N_p, P.N_q, P.N_f,
                  P.N_c, P.N_e, P.skew ? "skew" : "standard", P.second_order ? " br1" : "");

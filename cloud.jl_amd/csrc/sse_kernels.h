@@ -123,15 +123,13 @@ struct TensorParams {
     int variant;     // compiled launch-shape variant
     int n_pairs;     // volume pairs (union sparsity of S, i < j) followed by facet pairs (nonzeros of C)
     int n_vol_pairs;
-    int n_pass, pass_size, wv, wf, wrt, wr;
+    int n_pass, pass_size, wv, wf, wrt;
     const int* pk;       // n_pairs: i | j << 12 | kind << 24 (kind 0 volume pair, 1 facet pair)
     const double* cf;    // d x n_pairs: S_m[i,j] (volume) or C_ij in row 0 (facet)
     const int* vt;       // n_pass x wv x N_q: slot * 2 + (1 if subtracted), -1 = none
     const int* ft;       // n_pass x wf x N_f
     const int* rt_idx;   // wrt x N_q: R' rows (facet node), -1 = none
     const double* rt_val;
-    const int* r_idx;    // wr x N_f: R rows (volume node), -1 = none
-    const double* r_val;
     const double* VA;    // warped-product factors (column-major, as in the reference)
     const double* VB;
     const double* VC;
@@ -142,8 +140,9 @@ struct TensorParams {
     const double* WoJ;   // StandardForm scalar kernels: W / J, N_q x N_e (base.Lam then holds
                          // h W sum_m c_lm Lambda_mn)
     const double* Mw;    // weight-adjusted inverse mass matrix of every element, V' diag(W / J_k) V
-                         // (N_p x N_p column-major per element), or null: the kernels then apply
-                         // V, W / J_k and V' by sum factorisation
+                         // (N_p x N_p column-major per element), or null: the line-structured
+                         // time derivative then applies V, W / J_k and V' (it uses the matrix
+                         // for small N_p only)
     int xcd_remap;       // 1: spread contiguous element ranges over the 8 XCDs
     double* uf_ext;      // when set, nodal_values also writes each facet state into the
                          // neighbour's exterior slot [k][e][j] (mapP is an involution)

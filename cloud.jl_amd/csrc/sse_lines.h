@@ -156,10 +156,8 @@ struct LineFact {
     __device__ static void up2(UniformTable B, double* X) {
         if constexpr (G::TET) {
             const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
-            static_assert(P + 2 <= 2 * (TS / 64), "b1 over the wavefronts");
-            // wavefront w takes b1 = w and, where no wavefront starts there, P + 1 - w (their
-            // work goes with P + 1 - b1)
-            for (int b1 = wave; b1 <= P; b1 = (b1 == wave && P + 1 - wave >= TS / 64) ? P + 1 - wave : P + 1)
+            // b1 back and forth over the wavefronts: the work of b1 falls with it
+            for (int q = 0, b1 = wave; b1 <= P; ++q, b1 = (q & 1) ? (q + 1) * (TS / 64) - 1 - wave : q * (TS / 64) + wave)
                 for (int t = lane; t < NCOL * N1; t += 64) {
                     const int col = t / N1, a3 = t - col * N1;
                     double* L = X + col * CS * G::NX + b1 * G::S1 + a3;
@@ -182,10 +180,8 @@ struct LineFact {
     __device__ static void down2(UniformTable B, double* X) {
         if constexpr (G::TET) {
             const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
-            static_assert(P + 2 <= 2 * (TS / 64), "b1 over the wavefronts");
-            // wavefront w takes b1 = w and, where no wavefront starts there, P + 1 - w (their
-            // work goes with P + 1 - b1)
-            for (int b1 = wave; b1 <= P; b1 = (b1 == wave && P + 1 - wave >= TS / 64) ? P + 1 - wave : P + 1)
+            // b1 back and forth over the wavefronts: the work of b1 falls with it
+            for (int q = 0, b1 = wave; b1 <= P; ++q, b1 = (q & 1) ? (q + 1) * (TS / 64) - 1 - wave : q * (TS / 64) + wave)
                 for (int t = lane; t < NCOL * N1; t += 64) {
                     const int col = t / N1, a3 = t - col * N1;
                     double* L = X + col * CS * G::NX + b1 * G::S1 + a3;
@@ -283,6 +279,40 @@ __device__ __forceinline__ void face_row(const FaceTables& ft, int j, const doub
     }
 }
 
+// in place, the facet values t of NCOL columns (NF apart) to M' t; the caller's barrier follows.
+// tt: the thread among the TS (the whole workgroup calls: general has a barrier inside).
+// The lines of the faces of kind 1 go to the last threads of the workgroup (the first ones have
+// stage-1 lines of V in the same phase).
+template <int ELEM, int P, int NCOL, int TS>
+__device__ __forceinline__ void face_transpose(const FaceTables& ft, double* t, int tt) {
+    using G = LineGrid<ELEM, P>;
+    constexpr int N1 = G::N1, N2 = G::N2, NF = G::Sh::NF;
+    if (ft.general) {
+        constexpr int IT = (NCOL * NF + TS - 1) / TS;
+        double v[IT];
+#pragma unroll
+        for (int q = 0; q < IT; ++q) {
+            const int o = tt + q * TS, c = o / NF;
+            v[q] = 0.0;
+            if (o < NCOL * NF) face_row<ELEM, P, 1, NF, true>(ft, o - c * NF, t + c * NF, v + q);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < IT; ++q)
+            if (tt + q * TS < NCOL * NF) t[tt + q * TS] = v[q];
+    } else if constexpr (G::TET) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            if (ft.kind[f] == 0) continue;
+            const UniformTable Pf = uniform_table(ft.P) + f * N1 * N1;
+            for (int o = TS - 1 - tt; o < NCOL * N1; o += TS) {
+                const int c = o / N1;
+                face_line_t<N1>(Pf, t + c * NF + f * N2 + (o - c * N1) * N1);
+            }
+        }
+    }
+}
+
 // ends of line `line` of every direction but the first, of one column X
 template <int ELEM, int P>
 __device__ __forceinline__ void other_line_ends(const FaceTables& ft, const double* X, int line, double* e) {
@@ -297,13 +327,10 @@ __device__ __forceinline__ void other_line_ends(const FaceTables& ft, const doub
     }
 }
 
-// The columns of the Euler kernels: a workgroup of TS threads holds NC columns of each of E
-// elements (column s NC + e); a thread has one line of the first direction and one stage-1 line.
-// Every step works on all columns at once and ends with a barrier.
+// Elements and threads of a workgroup of the Euler kernels that only transform: all lines of E elements in one go with few idle threads, and for the Tet enough
+// columns to fill the lanes of stage 2 (E NC N1 of 64)
 template <int ELEM, int P>
 struct EulerTune;
-// E and TS: all lines of E elements in one go with few idle threads, and for the Tet enough
-// columns to fill the lanes of stage 2 (E NC N1 of 64)
 #define SSE_EULER_TUNE(E_, PP, e, ts) \
     template <>                       \
     struct EulerTune<E_, PP> {        \
@@ -320,12 +347,15 @@ SSE_EULER_TUNE(ELEM_TET, 4, 2, 256)
 SSE_EULER_TUNE(ELEM_TET, 5, 2, 384)
 #undef SSE_EULER_TUNE
 
-template <int ELEM, int P>
+// The columns of the Euler kernels: TS threads hold NC columns of each of E elements (column
+// s NC + e); a thread has one line of the first direction and one stage-1 line. Every step works
+// on all columns at once and ends with a barrier. t: the thread among the TS (on the Tet the TS
+// threads are the workgroup).
+template <int ELEM, int P, int E_, int TS_>
 struct EulerLines {
     using G = LineGrid<ELEM, P>;
     using LF = LineFact<ELEM, P>;
-    using T = EulerTune<ELEM, P>;
-    static constexpr int E = T::E, TS = T::TS, NC = G::Sh::NC, NCOL = E * NC, N1 = G::N1, N2 = G::N2, NM = G::NM,
+    static constexpr int E = E_, TS = TS_, NC = G::Sh::NC, NCOL = E * NC, N1 = G::N1, N2 = G::N2, NM = G::NM,
                          NX = G::NX;
     static_assert(NCOL * N2 <= TS && NCOL * NM <= TS, "a line per thread");
     UniformTable A, B;
@@ -334,9 +364,8 @@ struct EulerLines {
     int col, line, c1, m1;
     typename LF::Modes md1;
 
-    __device__ EulerLines(const TensorParams& tp, const double* F1_)
+    __device__ EulerLines(const TensorParams& tp, const double* F1_, int t)
         : A(uniform_table(tp.VA)), B(uniform_table(tp.VB)), F1(F1_) {
-        const int t = threadIdx.x;
         on = t < NCOL * N2;
         on1 = t < NCOL * NM;
         col = on ? t / N2 : 0;
@@ -432,6 +461,47 @@ struct EulerLines {
         scale3(X, woj);
         down2(X);
         turn1(X);
+    }
+};
+
+template <int ELEM, int P>
+using EulerGroup = EulerLines<ELEM, P, EulerTune<ELEM, P>::E, EulerTune<ELEM, P>::TS>;
+
+// R' at one node: its weight on each face (line_weights: requested early) and, with S = M' t of
+// NC columns of facet values NF apart, r[e] -= sum_f w_f S_e[f, line of the node]
+template <int ELEM, int P>
+struct NodeLift {
+    using G = LineGrid<ELEM, P>;
+    static constexpr int N1 = G::N1, N2 = G::N2, NF = G::Sh::NF, NFAC = G::Sh::NFAC;
+    double w[NFAC];
+    __device__ static void coords(int i, int dir, int& a, int& line) {
+        if constexpr (G::TET) {
+            const int a1 = i / N2, a2 = (i / N1) % N1, a3 = i % N1;
+            a = dir == 0 ? a1 : dir == 1 ? a2 : a3;
+            line = dir == 0 ? a2 * N1 + a3 : dir == 1 ? a1 * N1 + a3 : a1 * N1 + a2;
+        } else {
+            const int a1 = i / N1, a2 = i % N1;
+            a = dir == 0 ? a1 : a2;
+            line = dir == 0 ? a2 : a1;
+        }
+    }
+    __device__ void request(const FaceTables& ft, int i) {
+#pragma unroll
+        for (int f = 0; f < NFAC; ++f) {
+            int a, line;
+            coords(i, ft.dir[f], a, line);
+            w[f] = ft.w[f * N1 + a];
+        }
+    }
+    template <int NC>
+    __device__ void apply(const FaceTables& ft, int i, const double* S, double* r) const {
+#pragma unroll
+        for (int f = 0; f < NFAC; ++f) {
+            int a, line;
+            coords(i, ft.dir[f], a, line);
+#pragma unroll
+            for (int e = 0; e < NC; ++e) r[e] -= w[f] * S[e * NF + f * N2 + line];
+        }
     }
 };
 

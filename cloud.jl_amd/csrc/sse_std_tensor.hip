@@ -128,39 +128,6 @@ __device__ __forceinline__ unsigned neighbour(const DevParams& p, const Slots<E>
 template <int V>
 using Dir = std::integral_constant<int, V>;
 
-// in place, the facet values t of NCOL columns (NF apart) to M' t; the caller's barrier follows.
-// The lines of the faces of kind 1 go to the last threads of the workgroup (the first ones have
-// stage-1 lines of V in the same phase).
-template <int ELEM, int P, int NCOL, int TS>
-__device__ __forceinline__ void face_transpose(const FaceTables& ft, double* t) {
-    using G = LineGrid<ELEM, P>;
-    constexpr int N1 = G::N1, N2 = G::N2, NF = G::Sh::NF;
-    if (ft.general) {
-        constexpr int IT = (NCOL * NF + TS - 1) / TS;
-        double v[IT];
-#pragma unroll
-        for (int q = 0; q < IT; ++q) {
-            const int o = (int)threadIdx.x + q * TS, c = o / NF;
-            v[q] = 0.0;
-            if (o < NCOL * NF) face_row<ELEM, P, 1, NF, true>(ft, o - c * NF, t + c * NF, v + q);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < IT; ++q)
-            if ((int)threadIdx.x + q * TS < NCOL * NF) t[threadIdx.x + q * TS] = v[q];
-    } else if constexpr (G::TET) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-            if (ft.kind[f] == 0) continue;
-            const UniformTable Pf = uniform_table(ft.P) + f * N1 * N1;
-            for (int o = TS - 1 - (int)threadIdx.x; o < NCOL * N1; o += TS) {
-                const int c = o / N1;
-                face_line_t<N1>(Pf, t + c * NF + f * N2 + (o - c * N1) * N1);
-            }
-        }
-    }
-}
-
 }  // namespace
 
 // ----------------------------------------------------------------------------- phase 1
@@ -398,7 +365,7 @@ __global__ void __launch_bounds__((StdTune<ELEM, P>::TS), std_waves(P))
         LF::up1(F1, m1, xm, y);
         line_store<N1, 1>(xu + s1 * NX + md1.base, y);
     }
-    face_transpose<ELEM, P, E * D, TS>(tp.faces, stf);
+    face_transpose<ELEM, P, E * D, TS>(tp.faces, stf, tl);
     __syncthreads();
     if constexpr (G::TET) {
         LF::template up2<E, TS>(reload(B), xu);
@@ -616,7 +583,7 @@ __global__ void __launch_bounds__((StdTune<ELEM, P>::TS), std_waves(P))
         LF::up1(F1, m1, xm, y);
         line_store<N1, 1>(xf + c1 * NX + md1.base, y);
     }
-    face_transpose<ELEM, P, E, TS>(tp.faces, st);
+    face_transpose<ELEM, P, E, TS>(tp.faces, st, tl);
     __syncthreads();
     if constexpr (G::TET) {
         LF::template up2<E * D, TS>(reload(B), xf);

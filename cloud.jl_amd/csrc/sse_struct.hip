@@ -20,9 +20,13 @@
 // A team of TS threads owns one element. The exterior facet state is read
 // contiguously: phase 1 writes each facet state also into the neighbour's
 // exterior slot (the reference's u_f[CI[mapP[:,k]], :] gather).
+//
+// The lift, V' and the mass solve at the end took 37 % of a workgroup's life at Tet p = 4 with a
+// node per thread (table rows of R', every multiply-add reading LDS, 9.8 KB of kept matrix). On
+// lines (EulerLines, NodeLift) the residual of 24,576 elements went from 595 to 557 us.
 #include <hip/hip_runtime.h>
 
-#include "sse_tensor.h"
+#include "sse_lines.h"
 
 namespace sse {
 
@@ -55,17 +59,19 @@ struct StructLayout {
     static constexpr int ST = NC * (Sh::NQ + Sh::NF) > NC * MAXITEM ? NC * (Sh::NQ + Sh::NF) : NC * MAXITEM;
     static constexpr int off_fn = off_st + ST;                 // D x NFAC reference face normals
     static constexpr int size = off_fn + D * Sh::NFAC;
-    static constexpr int off_ff = off_h;                       // NC x NF (after the pair phase)
-    static constexpr int off_r = off_hf;                       // NC x NQ
-    static constexpr int off_rb = off_L;                       // NC x NQ partial rows of split threads
-    static constexpr int off_y = off_L;                        // NC x NP
-    static constexpr int off_z = off_st;                       // NC x NZ
-    static constexpr int off_W = off_z + NC * Sh::NZ;          // NC x NW
-    static_assert(NC * Sh::NF <= NH * Sh::NQ, "f_f alias");
-    static_assert(NC * Sh::NQ <= NH * Sh::NF + D * Sh::NF + ST, "r_q alias");
-    static_assert(NC * Sh::NP <= D * D * Sh::NQ, "y alias");
-    static_assert(NC * Sh::NQ <= D * D * Sh::NQ, "split partial-row alias");
-    static_assert(off_W + NC * Sh::NW <= off_fn, "sum-factorisation temporaries alias");
+    // after the pair phase, in the space of the states and the metric
+    using Lines = EulerLines<ELEM, P, 1, T::TS>;
+    static constexpr int off_ff = 0;                           // NC x NF facet fluxes
+    static constexpr int off_rb = off_ff + NC * Sh::NF;        // NC x NQ partial rows of split threads
+    static constexpr int off_x = off_rb + (T::SPLIT > 1 ? NC * Sh::NQ : 0);  // NC columns of r_q
+    static constexpr int off_woj = off_x + NC * Lines::NX;     // W / J
+    static constexpr int off_f1 = off_woj + Lines::NX;         // stage-1 tables of V
+    // The kept inverse mass matrix: a row of up to 20 entries per thread spares three short
+    // stages (20 RK stages of 2,058 Tet p = 3 elements 2,330 -> 2,160 us without it and with it);
+    // the 35 of Tet p = 4 cost more in registers and memory than the stages (569 against 621 us
+    // at 24,576 elements).
+    static constexpr bool KEPT = NC * Sh::NP <= T::TS && Sh::NP <= 20 && Sh::NP <= Sh::NF;
+    static_assert(off_f1 + Lines::LF::NT1 <= off_st, "tail of the kernel beside the accumulators");
 };
 
 
@@ -84,11 +90,9 @@ __global__ void __launch_bounds__((StructTune<ELEM, P>::TS * StructTune<ELEM, P>
 k_time_derivative_struct(TensorParams tp, StructTables st, double* __restrict__ dudt, RKStage rk, int n_teams) {
     using Sh = Shape<ELEM, P>;
     using T = StructTune<ELEM, P>;
-    using SF = SumFact<ELEM, P, T::TS>;
     using L = StructLayout<ELEM, P>;
     constexpr int D = Sh::D, NC = Sh::NC, NH = Sh::NH, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF, NPF = Sh::NPF;
     constexpr int N1 = Sh::N1, TS = T::TS, MAXITEM = L::MAXITEM, SPLIT = T::SPLIT, NT = TS / SPLIT;
-    constexpr int MAXR = TENSOR_MAXR;
     // volume pairs: on each line node a evaluates its pairs with the nodes at cyclic
     // offsets 1..DH from it, which covers every unordered pair of an odd-length line
     // once; on an even-length line the offset N1/2 pairs nodes both ways and only
@@ -419,23 +423,15 @@ k_time_derivative_struct(TensorParams tp, StructTables st, double* __restrict__ 
                 for (int e = 0; e < NC; ++e) atomicAdd(&sfac[e * NF + j], part[e]);
             }
         }
-        // the lift's rows of R' (all MAXR entries at once, padding as a zero weight on node 0)
-        // and this thread's share of the factors of V, requested here so that their latency
-        // passes during phases D and E
-        int rj[MAXR];
-        double rv[MAXR];
-        if (half == 0 && tl < NQ) {
+        // the node's weights of R' and this thread's share of the stage-1 tables, requested here
+        // so that their latency passes during phase D
+        using LN = typename L::Lines;
+        NodeLift<ELEM, P> lift;
+        if (half == 0 && tl < NQ) lift.request(tp.faces, tl);
+        constexpr int NT1 = LN::LF::NT1, IT1 = (NT1 + TS - 1) / TS;
+        double f1v[IT1];
 #pragma unroll
-            for (int w = 0; w < MAXR; ++w) {
-                rj[w] = w < tp.wrt ? tp.rt_idx[w * NQ + tl] : -1;
-                rv[w] = w < tp.wrt ? tp.rt_val[w * NQ + tl] : 0.0;
-            }
-        }
-        using VF = VFactors<ELEM, P>;
-        constexpr bool STAGE = VF::size <= NH * NQ;
-        constexpr int NVF = STAGE ? (VF::size + TS - 1) / TS : 1;
-        double vf[NVF];
-        if constexpr (STAGE) VF::fetch(tp, vf, tt, TS);
+        for (int q = 0; q < IT1; ++q) f1v[q] = tp.lines.F1[min(tt + q * TS, NT1 - 1)];
         __syncthreads();
         // ---- phase D: the C sums into r (volume nodes) and f_f (facet nodes); f_f to LDS
         double* sff = sm + L::off_ff;
@@ -467,63 +463,105 @@ k_time_derivative_struct(TensorParams tp, StructTables st, double* __restrict__ 
         }
         __syncthreads();
         // ---- phase E: lift r_q -= R' f_f
-        double* sr = sm + L::off_r;
+        double* sx = sm + L::off_x;
+        double* woj = sm + L::off_woj;
+        double* F1 = sm + L::off_f1;
+#pragma unroll
+        for (int q = 0; q < IT1; ++q)
+            if (tt + q * TS < NT1) F1[tt + q * TS] = f1v[q];
+        face_transpose<ELEM, P, NC, TS>(tp.faces, sff, tt);
+        __syncthreads();
         if (half == 0 && tl < NQ) {
+            using G = LineGrid<ELEM, P>;
             if (SPLIT > 1) {
 #pragma unroll
                 for (int e = 0; e < NC; ++e) r[e] += srb[e * NQ + tl];
             }
+            lift.template apply<NC>(tp.faces, tl, sff, r);
 #pragma unroll
-            for (int w = 0; w < MAXR; ++w) {
-                if (rj[w] < 0) continue;
-#pragma unroll
-                for (int e = 0; e < NC; ++e) r[e] -= rv[w] * sff[e * NF + rj[w]];
-            }
-#pragma unroll
-            for (int e = 0; e < NC; ++e) sr[e * NQ + tl] = r[e];
+            for (int e = 0; e < NC; ++e) sx[e * G::NX + G::position(tl)] = r[e];
+            woj[G::position(tl)] = Wi * rcp_refined(Ji);
         }
         __syncthreads();
-        // ---- phase F: dudt = V' r_q, weight-adjusted mass solve; the factors of V are
-        // copied into the (now dead) hoisted-state array when they fit there
-        double* sy = sm + L::off_y;
-        double* sZ = sm + L::off_z;
-        double* sW = sm + L::off_W;
-        TensorParams tq = tp;
-        if constexpr (STAGE) {
-            VF::put(vf, sm + L::off_h, tt, TS);
-            tq = VF::in_lds(tp, sm + L::off_h);
-            __syncthreads();
-        }
-        // the weight-adjusted inverse V' diag(W/J) V kept per element, requested before
-        // the transform and staged where r_q and the temporaries were
-        constexpr bool MW = NP * NP <= L::off_fn - L::off_hf;
-        MassPrefetch<NP, TS> pre;
-        if constexpr (MW) {
-            if (tp.Mw) mass_prefetch<NP, TS>(tp.Mw + (size_t)k * NP * NP, tt, pre);
-        }
-        SF::Vt(tq, tt, sr, sy, sZ, sW);
-        if (MW && tp.Mw) {
-            mass_apply_staged<NP, NC, TS>(pre, sm + L::off_hf, sy, tt);
-        } else {
-            SF::V(tq, tt, sy, sr, sZ, sW);
-            if (half == 0 && tl < NQ) {
-                const double jw = Wi / Ji;
+        // ---- phase F: dudt = M^{-1} V' r_q, line by line. M^{-1} = V' diag(W/J) V: the kept
+        // matrix where a thread can hold one of its rows (requested before the transform), else
+        // (and without kept matrices) V, W/J and V' again
+        const LN ln(tp, F1, tt);
+        constexpr bool KEPT = L::KEPT;
+        if (KEPT && tp.Mw) {
+            const bool out = tt < NC * NP;
+            const int e = out ? tt / NP : 0, j = tt % NP;
+            const size_t o = ((size_t)k * NC + e) * NP + j;
+            double m[NP], u0 = 0.0, k0 = 0.0;
+            const double* Mk = tp.Mw + (size_t)k * NP * NP + j;  // symmetric: row j as a column
 #pragma unroll
-                for (int e = 0; e < NC; ++e) sr[e * NQ + tl] *= jw;
+            for (int i = 0; i < NP; ++i) m[i] = Mk[(size_t)i * NP];
+            if (rk.active) {
+                u0 = rk.u[o];
+                if (rk.A != 0.0) k0 = rk.tmp[o];
+            }
+            ln.down3(sx);
+            ln.down2(sx);
+            double* sy = sm + L::off_ff;  // NC x NP (the facet fluxes are dead)
+            if (ln.on1) {
+                double x[N1], y[N1];
+                line_load<N1, 1>(ln.line1(sx), x);
+                LN::LF::down1(F1, ln.m1, x, y);
+#pragma unroll
+                for (int b = 0; b < N1; ++b)
+                    if (b <= ln.md1.lim) sy[ln.c1 * NP + ln.md1.off + b] = y[b];
             }
             __syncthreads();
-            SF::Vt(tq, tt, sr, sy, sZ, sW);
+            if (!valid || !out) return;  // no barrier follows
+            double y0 = 0.0, y1 = 0.0;
+#pragma unroll
+            for (int i = 0; i + 1 < NP; i += 2) {
+                y0 += m[i] * sy[e * NP + i];
+                y1 += m[i + 1] * sy[e * NP + i + 1];
+            }
+            if constexpr (NP % 2 == 1) y0 += m[NP - 1] * sy[e * NP + NP - 1];
+            const double y = y0 + y1;
+            if (!rk.active) {
+                dudt[o] = y;
+            } else {
+                const double kt = rk.A * k0 + rk.dt_of(k) * y;
+                rk.tmp[o] = kt;
+                if (rk.keep) rk.keep[o] = u0;
+                rk.u[o] = u0 + rk.B * kt;
+            }
+            return;
         }
-        const size_t base = (size_t)k * NP * NC;
-        if (!valid) {
-        } else if (!rk.active) {
-            for (int t = tt; t < NP * NC; t += TS) dudt[base + t] = sy[t];
-        } else {
-            for (int t = tt; t < NP * NC; t += TS) {
-                const double kt = (rk.A == 0.0 ? 0.0 : rk.A * rk.tmp[base + t]) + rk.dt_of(k) * sy[t];
-                rk.tmp[base + t] = kt;
-                if (rk.keep) rk.keep[base + t] = rk.u[base + t];
-                rk.u[base + t] += rk.B * kt;
+        const size_t base = ((size_t)k * NC + ln.c1) * NP + ln.md1.off;
+        double u0[N1], k0[N1];  // an RK stage's state and register, requested before the transforms
+        if (rk.active) {
+#pragma unroll
+            for (int b = 0; b < N1; ++b) {
+                const size_t t = base + min(b, ln.md1.lim);
+                u0[b] = rk.u[t];
+                k0[b] = rk.A == 0.0 ? 0.0 : rk.tmp[t];
+            }
+        }
+        ln.down3(sx);
+        ln.down2(sx);
+        ln.turn1(sx);
+        ln.up2(sx);
+        ln.scale3(sx, woj);
+        ln.down2(sx);
+        if (!valid || !ln.on1) return;  // no barrier follows
+        double x[N1], y[N1];
+        line_load<N1, 1>(ln.line1(sx), x);
+        LN::LF::down1(F1, ln.m1, x, y);
+#pragma unroll
+        for (int b = 0; b < N1; ++b) {
+            if (b > ln.md1.lim) continue;
+            const size_t t = base + b;
+            if (!rk.active) {
+                dudt[t] = y[b];
+            } else {
+                const double kt = rk.A * k0[b] + rk.dt_of(k) * y[b];
+                rk.tmp[t] = kt;
+                if (rk.keep) rk.keep[t] = u0[b];
+                rk.u[t] = u0[b] + rk.B * kt;
             }
         }
     }
@@ -593,6 +631,15 @@ int struct_occupancy(int elem, int P) {
 bool struct_config(int elem, int P, StructConfig* c) {
 #define SSE_CASE(E, PP) \
     if (elem == E && P == PP) { *c = struct_config_of<E, PP>(); return true; }
+    SSE_STRUCT_CASES
+#undef SSE_CASE
+    return false;
+}
+
+// the kernel uses each element's kept inverse mass matrix (TensorParams::Mw)
+bool struct_keeps_mass(int elem, int P) {
+#define SSE_CASE(E, PP) \
+    if (elem == E && P == PP) return StructLayout<E, PP>::KEPT;
     SSE_STRUCT_CASES
 #undef SSE_CASE
     return false;

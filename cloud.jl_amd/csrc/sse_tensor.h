@@ -101,47 +101,6 @@ __device__ __forceinline__ int element_of_block(int b, int nb, int remap) {
     return (b & 7) * (nb >> 3) + (b >> 3);
 }
 
-// ----------------------------------------------------------------------------- factors of V in LDS
-// The sum-factorisation factors A, B (and C on the Tet) of V are a few KB read by every
-// stage of every application; a kernel copies them to LDS once and hands SumFact a
-// TensorParams whose VA, VB, VC point there (LDS latency instead of cache latency in the
-// factor loops).
-template <int ELEM, int P>
-struct VFactors {
-    static constexpr int N1 = P + 1;
-    static constexpr int NA = N1 * (P + 1), NB = N1 * (P + 1) * (P + 1);
-    static constexpr int NCF = ELEM == ELEM_TET ? N1 * (P + 1) * (P + 1) * (P + 1) : 0;
-    static constexpr int size = NA + NB + NCF;
-    // all `nt` threads of the caller copy; a barrier must follow before use
-    __device__ static void stage(const TensorParams& tp, double* dst, int t, int nt) {
-        for (int i = t; i < NA; i += nt) dst[i] = tp.VA[i];
-        for (int i = t; i < NB; i += nt) dst[NA + i] = tp.VB[i];
-        if constexpr (NCF > 0)
-            for (int i = t; i < NCF; i += nt) dst[NA + NB + i] = tp.VC[i];
-    }
-    // the same copy in two steps: thread t's entries t, t + nt, ... (of the concatenated
-    // factors) into registers, then into LDS; v holds ceil(size / nt) values
-    __device__ static void fetch(const TensorParams& tp, double* v, int t, int nt) {
-#pragma unroll
-        for (int r = 0; r * nt < size; ++r) {
-            const int i = t + r * nt;
-            v[r] = i < NA ? tp.VA[i] : i < NA + NB ? tp.VB[i - NA] : i < size ? tp.VC[i - NA - NB] : 0.0;
-        }
-    }
-    __device__ static void put(const double* v, double* dst, int t, int nt) {
-#pragma unroll
-        for (int r = 0; r * nt < size; ++r)
-            if (t + r * nt < size) dst[t + r * nt] = v[r];
-    }
-    __device__ static TensorParams in_lds(const TensorParams& tp, const double* src) {
-        TensorParams r = tp;
-        r.VA = src;
-        r.VB = src + NA;
-        r.VC = NCF > 0 ? src + NA + NB : tp.VC;
-        return r;
-    }
-};
-
 // ----------------------------------------------------------------------------- sum factorisation
 // All arrays are component-major LDS arrays: x[e * stride + point]. NCV
 // components (conserved variables, or several elements or directions side by
@@ -355,62 +314,5 @@ struct SumFact<ELEM_TET, P, TS, NCV> {
         b3 = m;
     }
 };
-
-// The weight-adjusted mass solve with the element's kept inverse Mk = V' diag(W/J_k) V
-// (NP x NP column-major in global memory): mass_prefetch requests a team's share of Mk
-// into registers (issued before a transform, whose time hides the latency), then
-// mass_apply_staged writes it to LDS (sM, NP x NP, not aliasing x) and computes
-// x = Mk x in place for NC columns of NP modes in LDS: thread t of a team of TS takes
-// the items (e, j) = t, t + TS, ..., into registers, then writes them back. Ends with a
-// barrier.
-template <int NP, int TS>
-struct MassPrefetch {
-    static constexpr int MI = (NP * NP + TS - 1) / TS;
-    double v[MI];
-};
-
-template <int NP, int TS>
-__device__ __forceinline__ void mass_prefetch(const double* __restrict__ Mk, int t, MassPrefetch<NP, TS>& pre) {
-#pragma unroll
-    for (int r = 0; r < MassPrefetch<NP, TS>::MI; ++r) {
-        const int c = t + r * TS;
-        pre.v[r] = c < NP * NP ? Mk[c] : 0.0;
-    }
-}
-
-template <int NP, int NC, int TS>
-__device__ __forceinline__ void mass_apply_staged(const MassPrefetch<NP, TS>& pre, double* sM, double* x, int t) {
-#pragma unroll
-    for (int r = 0; r < MassPrefetch<NP, TS>::MI; ++r) {
-        const int c = t + r * TS;
-        if (c < NP * NP) sM[c] = pre.v[r];
-    }
-    __syncthreads();
-    constexpr int IT = (NP * NC + TS - 1) / TS;
-    double y[IT];
-#pragma unroll
-    for (int r = 0; r < IT; ++r) {
-        const int it = t + r * TS;
-        double s0 = 0.0, s1 = 0.0;
-        if (it < NP * NC) {
-            const int e = it / NP, j = it - e * NP;
-            const double* xe = x + e * NP;
-#pragma unroll 4
-            for (int i = 0; i + 1 < NP; i += 2) {
-                s0 += sM[j + NP * i] * xe[i];
-                s1 += sM[j + NP * (i + 1)] * xe[i + 1];
-            }
-            if constexpr (NP % 2 == 1) s0 += sM[j + NP * (NP - 1)] * xe[NP - 1];
-        }
-        y[r] = s0 + s1;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < IT; ++r) {
-        const int it = t + r * TS;
-        if (it < NP * NC) x[it] = y[r];
-    }
-    __syncthreads();
-}
 
 }  // namespace sse

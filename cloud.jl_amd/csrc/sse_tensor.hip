@@ -62,7 +62,7 @@ hipError_t launch_weight_adjusted_inverse(const DevParams& p, double* Mw, hipStr
 // took 669 us at 24,576 Tet p = 4 elements and 42.3 us at 8,192 Tri p = 3, now 595 and 27.9 us.
 template <int ELEM, int P>
 struct K1Layout {
-    using L = EulerLines<ELEM, P>;
+    using L = EulerGroup<ELEM, P>;
     using Sh = Shape<ELEM, P>;
     static constexpr int x = 0, woj = x + L::NCOL * L::NX, f1 = woj + L::E * L::NX, e = f1 + L::LF::NT1;
     static constexpr int size = e + L::NCOL * Sh::NF;
@@ -73,7 +73,7 @@ __global__ void __launch_bounds__((EulerTune<ELEM, P>::TS), (ELEM == ELEM_TET ? 
 k_nodal_values_tensor(TensorParams tp, const double* __restrict__ u) {
     using Sh = Shape<ELEM, P>;
     using G = LineGrid<ELEM, P>;
-    using EL = EulerLines<ELEM, P>;
+    using EL = EulerGroup<ELEM, P>;
     using L = K1Layout<ELEM, P>;
     constexpr int D = Sh::D, NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF, N1 = G::N1, NX = G::NX;
     constexpr int E = EL::E, TS = EL::TS, ITQ = (E * NQ + TS - 1) / TS;
@@ -84,7 +84,7 @@ k_nodal_values_tensor(TensorParams tp, const double* __restrict__ u) {
     auto element = [&](int s) { return min(k0 + s, last); };  // past the last: computed, not stored
     double *X = sm + L::x, *woj = sm + L::woj, *F1 = sm + L::f1, *es = sm + L::e;
     EL::LF::stage_tables(tp.lines, F1, tl, TS);
-    const EL el(tp, F1);
+    const EL el(tp, F1, tl);
     double J[ITQ], um[N1];
     {
         const int s = el.c1 / NC, e = el.c1 - s * NC;

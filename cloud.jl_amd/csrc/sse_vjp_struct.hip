@@ -69,7 +69,7 @@ struct VjpLayout {
 // LDS of V1 and of the reverse projection V3 (EulerLines)
 template <int ELEM, int P>
 struct VjpLinesLayout {
-    using L = EulerLines<ELEM, P>;
+    using L = EulerGroup<ELEM, P>;
     static constexpr int x = 0, woj = x + L::NCOL * L::NX, f1 = woj + L::E * L::NX, more = f1 + L::LF::NT1;
     static constexpr int size1 = more + L::NCOL * L::G::Sh::NF;  // V1: line ends
     static constexpr int size3 = more + L::NCOL * L::NX;         // V3: V u
@@ -100,7 +100,7 @@ k_vjp_v1_tensor(TensorParams tp, const double* ybar, double* __restrict__ rbar, 
                 double* __restrict__ fbar_ext, VjpIn in) {
     using Sh = Shape<ELEM, P>;
     using G = LineGrid<ELEM, P>;
-    using EL = EulerLines<ELEM, P>;
+    using EL = EulerGroup<ELEM, P>;
     using L = VjpLinesLayout<ELEM, P>;
     constexpr int E = EL::E, TS = EL::TS, NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, NF = Sh::NF, N1 = G::N1;
     extern __shared__ double sm[];
@@ -110,7 +110,7 @@ k_vjp_v1_tensor(TensorParams tp, const double* ybar, double* __restrict__ rbar, 
     auto element = [&](int s) { return min(k0 + s, last); };  // past the last: computed, not stored
     double *X = sm + L::x, *woj = sm + L::woj, *F1 = sm + L::f1, *es = sm + L::more;
     EL::LF::stage_tables(tp.lines, F1, tl, TS);
-    const EL el(tp, F1);
+    const EL el(tp, F1, tl);
     double y[N1];
     {
         const int s = el.c1 / NC, e = el.c1 - s * NC;
@@ -635,7 +635,7 @@ k_vjp_v3_tensor(TensorParams tp, const double* __restrict__ u, const double* __r
                 double* __restrict__ ubar, VjpOut out) {
     using Sh = Shape<ELEM, P>;
     using G = LineGrid<ELEM, P>;
-    using EL = EulerLines<ELEM, P>;
+    using EL = EulerGroup<ELEM, P>;
     using L = VjpLinesLayout<ELEM, P>;
     using A = EulerAdj<Sh::D>;
     constexpr int E = EL::E, TS = EL::TS, NC = Sh::NC, NP = Sh::NP, NQ = Sh::NQ, N1 = G::N1, NX = G::NX;
@@ -646,7 +646,7 @@ k_vjp_v3_tensor(TensorParams tp, const double* __restrict__ u, const double* __r
     auto element = [&](int s) { return min(k0 + s, last); };  // past the last: computed, not stored
     double *X = sm + L::x, *woj = sm + L::woj, *F1 = sm + L::f1, *U = sm + L::more;
     EL::LF::stage_tables(tp.lines, F1, tl, TS);
-    const EL el(tp, F1);
+    const EL el(tp, F1, tl);
     const int s1 = el.c1 / NC, s3 = el.col / NC;
     const size_t o1 = ((size_t)element(s1) * NC + (el.c1 - s1 * NC)) * NP + el.md1.off;
     double um[N1], w[N1];
