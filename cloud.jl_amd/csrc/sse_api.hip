@@ -56,6 +56,10 @@ int struct_occupancy(int elem, int P);
 bool struct_keeps_mass(int elem, int P);
 hipError_t launch_struct(const TensorParams& tp, const StructTables& st, double* dudt, const RKStage& rk,
                          hipStream_t s, int n_blocks);
+// triangles of several degrees in one launch
+int tri_nodal_blocks(int P, int N_e);
+hipError_t launch_nodal_values_tri_groups(const TriGroups& a, hipStream_t s);
+hipError_t launch_time_derivative_tri_groups(const TriGroups& a, hipStream_t s);
 bool std_tensor_config(int elem, int P);
 size_t vjp_tensor_config(int elem, int P);
 hipError_t launch_vjp_tensor(const TensorParams& tp, const StructTables& st, const double* u, const double* ybar,
@@ -2186,6 +2190,42 @@ int ensemble_chunk(const sse_desc* D, int R) {
     return (int)std::max<size_t>(cap, 2);
 }
 
+// The groups whose stages go into one launch each for all of them (sse::TriGroups): the first
+// group of each degree that has the line-structured triangle kernels, if there are two or more.
+// The order of atomic sums is theirs to choose, so deterministic groups keep their own launches;
+// SSE_BATCH_BRANCHES=0 (all groups in sequence) gives every group its own.
+std::vector<size_t> tri_groups(const sse_batch* b) {
+    std::vector<size_t> of;
+    const char* env = getenv("SSE_BATCH_BRANCHES");
+    if (env && env[0] == '0') return of;
+    bool taken[7] = {};
+    for (size_t g = 0; g < b->groups.size(); ++g) {
+        const sse_handle* h = b->groups[g];
+        const int P = h->TP.P;
+        if (b->chunk[g] || !h->use_struct || h->TP.elem != sse::ELEM_TRI || h->ST.det || P < 2 || P > 6 || taken[P])
+            continue;
+        taken[P] = true;
+        of.push_back(g);
+    }
+    if (of.size() < 2) of.clear();
+    return of;
+}
+
+int tri_stage(sse_batch* b, const std::vector<size_t>& of, int s, hipStream_t stream) {
+    sse::TriGroups a = {};
+    for (size_t g : of) {
+        const sse_handle* h = b->groups[g];
+        sse::TriGroup& t = a.g[h->TP.P - 2];
+        t.set(h->TP, h->ST, RKStage{1, CK_A[s], CK_B[s], 0.0, b->tmp[g], b->state[g], b->dt_e[g]});
+        t.blocks1 = sse::tri_nodal_blocks(h->TP.P, h->P.N_e);
+        t.blocks2 = h->struct_blocks;
+    }
+    hipError_t e = sse::launch_nodal_values_tri_groups(a, stream);
+    if (e == hipSuccess) e = sse::launch_time_derivative_tri_groups(a, stream);
+    if (e != hipSuccess) return bfail(b, SSE_ERR_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
+    return 0;
+}
+
 // RK stage of members [c0, c0 + n) of ensemble group g (tangent: lanes of the pair buffers)
 int ensemble_stage(sse_batch* b, size_t g, int s, bool tangent) {
     sse_handle* h = b->groups[g];
@@ -2379,19 +2419,24 @@ int sse_batch_rk_steps(sse_batch* b, double* const* u, const double* dt, int32_t
         // the host vector must outlive the copy
         if ((rc = hip_ok(hipStreamSynchronize(b->stream), "sync"))) return rc;
     }
+    // units of work that do not depend on each other: a group, or the triangle groups that share
+    // their launches (all of them under the first one's number)
+    const std::vector<size_t> tri = tri_groups(b);
+    std::vector<size_t> units;
+    for (size_t g = 0; g < b->groups.size(); ++g)
+        if (std::find(tri.begin() + (tri.empty() ? 0 : 1), tri.end(), g) == tri.end()) units.push_back(g);
+    auto stage = [&](size_t g, int s, hipStream_t stream) -> int {
+        if (!tri.empty() && g == tri[0]) return tri_stage(b, tri, s, stream);
+        if (b->chunk[g]) return ensemble_stage(b, g, s, false);
+        RKStage rk{1, CK_A[s], CK_B[s], 0.0, b->tmp[g], b->state[g], b->dt_e[g]};
+        const int r = launch(b->groups[g], b->state[g], nullptr, rk, 3);
+        return r ? bfail(b, r, b->groups[g]->err) : 0;
+    };
     auto one_step = [&]() -> int {
-        for (int s = 0; s < 5; ++s)
-            for (size_t g = 0; g < b->groups.size(); ++g) {
-                if (b->chunk[g]) {
-                    int r = ensemble_stage(b, g, s, false);
-                    if (r) return r;
-                    continue;
-                }
-                RKStage rk{1, CK_A[s], CK_B[s], 0.0, b->tmp[g], b->state[g], b->dt_e[g]};
-                int r = launch(b->groups[g], b->state[g], nullptr, rk, 3);
-                if (r) return bfail(b, r, b->groups[g]->err);
-            }
-        return 0;
+        int r = 0;
+        for (int s = 0; s < 5 && !r; ++s)
+            for (size_t t = 0; t < units.size() && !r; ++t) r = stage(units[t], s, b->stream);
+        return r;
     };
     int step = 0;
     if (nsteps > 0) {  // the first step runs eagerly (it also sets kernel attributes)
@@ -2400,14 +2445,14 @@ int sse_batch_rk_steps(sse_batch* b, double* const* u, const double* dt, int32_t
     }
     if (use_graph && step < nsteps) {
         if (!b->exec) {
-            // one branch per group (SSE_BATCH_BRANCHES=0: all groups in sequence on one stream)
+            // one branch per unit (SSE_BATCH_BRANCHES=0: all groups in sequence on one stream)
             const char* env = getenv("SSE_BATCH_BRANCHES");
-            const bool branches = !(env && env[0] == '0') && b->groups.size() > 1;
+            const bool branches = !(env && env[0] == '0') && units.size() > 1;
             if (branches && b->branch.empty()) {
                 b->branch.assign(b->groups.size(), nullptr);
                 b->join.assign(b->groups.size(), nullptr);
                 if ((rc = hip_ok(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming), "event create"))) return rc;
-                for (size_t g = 0; g < b->groups.size(); ++g)
+                for (size_t g : units)
                     if ((rc = hip_ok(hipStreamCreate(&b->branch[g]), "stream create")) ||
                         (rc = hip_ok(hipEventCreateWithFlags(&b->join[g], hipEventDisableTiming), "event create")))
                         return rc;
@@ -2418,21 +2463,13 @@ int sse_batch_rk_steps(sse_batch* b, double* const* u, const double* dt, int32_t
             hipError_t e = hipSuccess;
             if (branches) {
                 e = hipEventRecord(b->fork, b->stream);
-                for (size_t g = 0; g < b->groups.size() && e == hipSuccess; ++g) {
-                    e = hipStreamWaitEvent(b->branch[g], b->fork, 0);
+                for (size_t g : units) {
+                    if (e == hipSuccess) e = hipStreamWaitEvent(b->branch[g], b->fork, 0);
                     sse_set_stream(b->groups[g], b->branch[g]);
                 }
-                for (size_t g = 0; g < b->groups.size() && e == hipSuccess && !r; ++g)
-                    for (int s = 0; s < 5 && !r; ++s) {
-                        if (b->chunk[g]) {
-                            r = ensemble_stage(b, g, s, false);
-                            continue;
-                        }
-                        RKStage rk{1, CK_A[s], CK_B[s], 0.0, b->tmp[g], b->state[g], b->dt_e[g]};
-                        r = launch(b->groups[g], b->state[g], nullptr, rk, 3);
-                        if (r) r = bfail(b, r, b->groups[g]->err);
-                    }
-                for (size_t g = 0; g < b->groups.size(); ++g) {
+                for (size_t t = 0; t < units.size() && e == hipSuccess && !r; ++t)
+                    for (int s = 0; s < 5 && !r; ++s) r = stage(units[t], s, b->branch[units[t]]);
+                for (size_t g : units) {
                     if (e == hipSuccess) e = hipEventRecord(b->join[g], b->branch[g]);
                     if (e == hipSuccess) e = hipStreamWaitEvent(b->stream, b->join[g], 0);
                     sse_set_stream(b->groups[g], b->stream);

@@ -67,7 +67,7 @@ struct StructLayout {
     static constexpr int off_woj = off_x + NC * Lines::NX;     // W / J
     static constexpr int off_f1 = off_woj + Lines::NX;         // stage-1 tables of V
     // The kept inverse mass matrix: a row of up to 20 entries per thread spares three short
-    // stages (20 RK stages of 2,058 Tet p = 3 elements 2,330 -> 2,160 us without it and with it);
+    // stages (ten RK steps of 2,058 Tet p = 3 elements 2,330 -> 2,160 us without it and with it);
     // the 35 of Tet p = 4 cost more in registers and memory than the stages (569 against 621 us
     // at 24,576 elements).
     static constexpr bool KEPT = NC * Sh::NP <= T::TS && Sh::NP <= 20 && Sh::NP <= Sh::NF;
@@ -86,8 +86,9 @@ struct IntConst {
 // the column sums of C go through per-chunk slots summed in chunk order. The C pairs are
 // then evaluated twice (row and column), and no sum depends on the order of atomics.
 template <int ELEM, int P, bool DET>
-__global__ void __launch_bounds__((StructTune<ELEM, P>::TS * StructTune<ELEM, P>::EPB), (StructTune<ELEM, P>::WAVES))
-k_time_derivative_struct(TensorParams tp, StructTables st, double* __restrict__ dudt, RKStage rk, int n_teams) {
+__device__ __forceinline__ void time_derivative_body(const TensorParams& tp, const StructTables& st,
+                                                     double* __restrict__ dudt, const RKStage& rk, int block,
+                                                     int blocks) {
     using Sh = Shape<ELEM, P>;
     using T = StructTune<ELEM, P>;
     using L = StructLayout<ELEM, P>;
@@ -147,7 +148,7 @@ k_time_derivative_struct(TensorParams tp, StructTables st, double* __restrict__ 
     // one element per team; a team past the last element computes on a valid
     // element (block-wide barriers) and stores nothing
     const int last = p.N_e - 1;
-    const int kb = element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * T::EPB;
+    const int kb = element_of_block(block, blocks, tp.xcd_remap) * T::EPB;
     {
         const int k = min(kb + team, last);
         const bool valid = kb + team < p.N_e;
@@ -567,6 +568,30 @@ k_time_derivative_struct(TensorParams tp, StructTables st, double* __restrict__ 
     }
 }
 
+template <int ELEM, int P, bool DET>
+__global__ void __launch_bounds__((StructTune<ELEM, P>::TS * StructTune<ELEM, P>::EPB), (StructTune<ELEM, P>::WAVES))
+k_time_derivative_struct(TensorParams tp, StructTables st, double* __restrict__ dudt, RKStage rk) {
+    time_derivative_body<ELEM, P, DET>(tp, st, dudt, rk, blockIdx.x, gridDim.x);
+}
+
+// One RK stage of triangles of several degrees in one launch (see k_nodal_values_tri_groups).
+__global__ void __launch_bounds__(128) k_time_derivative_tri_groups(TriGroups a) {
+    static_assert(StructTune<ELEM_TRI, 2>::TS * StructTune<ELEM_TRI, 2>::EPB == 128, "the block of every degree");
+    static_assert(StructLayout<ELEM_TRI, 6>::size * 16 <= 65536, "LDS without an attribute");
+    int block = blockIdx.x;
+#define SSE_TRI_GROUP(PP)                                                                                     \
+    if (block < a.g[PP - 2].blocks2)                                                                          \
+        return time_derivative_body<ELEM_TRI, PP, false>(a.g[PP - 2].params(), a.g[PP - 2].st, nullptr, a.g[PP - 2].rk, \
+                                                         block, a.g[PP - 2].blocks2);                         \
+    block -= a.g[PP - 2].blocks2;
+    SSE_TRI_GROUP(6)
+    SSE_TRI_GROUP(5)
+    SSE_TRI_GROUP(4)
+    SSE_TRI_GROUP(3)
+    SSE_TRI_GROUP(2)
+#undef SSE_TRI_GROUP
+}
+
 struct StructConfig {
     int TS, EPB, lds, max_item;
 };
@@ -591,7 +616,7 @@ hipError_t launch_struct_v(const TensorParams& tp, const StructTables& st, doubl
         attr_set = true;
     }
     hipLaunchKernelGGL((k_time_derivative_struct<ELEM, P, DET>), dim3(n_blocks), dim3(T::TS * T::EPB), c.lds, s, tp,
-                       st, dudt, rk, n_blocks * T::EPB);
+                       st, dudt, rk);
     return hipGetLastError();
 }
 
@@ -652,6 +677,19 @@ hipError_t launch_struct(const TensorParams& tp, const StructTables& st, double*
     SSE_STRUCT_CASES
 #undef SSE_CASE
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_time_derivative_tri_groups(const TriGroups& a, hipStream_t s) {
+    int lds = 0, blocks = 0;
+    for (int P = 2; P <= 6; ++P) {
+        if (!a.g[P - 2].blocks2) continue;
+        StructConfig c;
+        if (!struct_config(ELEM_TRI, P, &c)) return hipErrorInvalidValue;
+        lds = c.lds > lds ? c.lds : lds;
+        blocks += a.g[P - 2].blocks2;
+    }
+    hipLaunchKernelGGL(k_time_derivative_tri_groups, dim3(blocks), dim3(128), lds, s, a);
+    return hipGetLastError();
 }
 
 }  // namespace sse

@@ -80,6 +80,47 @@ struct StructTables {
     int det;  // 1: every sum in a fixed order (no atomic accumulation)
 };
 
+// Triangles of several degrees in one launch (batched problems): entry P - 2 is the group of
+// degree P, if it has elements; the blocks of the higher degrees, whose elements take longer, go
+// first. By value, and only what these kernels read (at most 4 KiB of arguments): from a table
+// in memory they held every pointer in a spilled scalar register (2,000 register moves).
+struct TriGroup {
+    int N_e, xcd_remap, blocks1, blocks2;  // blocks of the nodal values and of the time derivative
+    LawParams law;
+    const double *Jq, *Lam, *nJf, *Jf, *W, *B, *fn;
+    const int* mapP;
+    double *uq, *uf, *uf_ext;
+    int* status;
+    const double *VA, *VB, *Mw;
+    LineTables lines;
+    FaceTables faces;
+    StructTables st;
+    RKStage rk;
+
+    __host__ void set(const TensorParams& tp, const StructTables& t, const RKStage& r) {
+        const DevParams& p = tp.base;
+        N_e = p.N_e, xcd_remap = tp.xcd_remap, law = p.law;
+        Jq = p.Jq, Lam = p.Lam, nJf = p.nJf, Jf = p.Jf, W = p.W, B = p.B, fn = p.fn, mapP = p.mapP;
+        uq = p.uq, uf = p.uf, uf_ext = tp.uf_ext, status = p.status;
+        VA = tp.VA, VB = tp.VB, Mw = tp.Mw, lines = tp.lines, faces = tp.faces, st = t, rk = r;
+    }
+    // the parameters as the kernels of one degree take them (what they do not read stays empty)
+    __device__ __forceinline__ TensorParams params() const {
+        TensorParams tp = {};
+        DevParams& p = tp.base;
+        p.N_e = N_e, tp.xcd_remap = xcd_remap, p.law = law;
+        p.Jq = Jq, p.Lam = Lam, p.nJf = nJf, p.Jf = Jf, p.W = W, p.B = B, p.fn = fn, p.mapP = mapP;
+        p.uq = uq, p.uf = uf, tp.uf_ext = uf_ext, p.status = status;
+        tp.VA = VA, tp.VB = VB, tp.Mw = Mw, tp.lines = lines, tp.faces = faces;
+        return tp;
+    }
+};
+
+struct TriGroups {
+    TriGroup g[5];
+};
+static_assert(sizeof(TriGroups) <= 4096, "kernel arguments");
+
 // q index of (b1, b2), b1 + b2 <= P, enumerated with b1 outer: also the mode
 // number of (b1, b2) in 2D.
 template <int P>

@@ -69,8 +69,8 @@ struct K1Layout {
 };
 
 template <int ELEM, int P>
-__global__ void __launch_bounds__((EulerTune<ELEM, P>::TS), (ELEM == ELEM_TET ? 6 : 1))
-k_nodal_values_tensor(TensorParams tp, const double* __restrict__ u) {
+__device__ __forceinline__ void nodal_values_body(const TensorParams& tp, const double* __restrict__ u, int block,
+                                                  int blocks) {
     using Sh = Shape<ELEM, P>;
     using G = LineGrid<ELEM, P>;
     using EL = EulerGroup<ELEM, P>;
@@ -80,7 +80,7 @@ k_nodal_values_tensor(TensorParams tp, const double* __restrict__ u) {
     extern __shared__ double sm[];
     const DevParams& p = tp.base;
     const int tl = threadIdx.x;
-    const int k0 = element_of_block(blockIdx.x, gridDim.x, tp.xcd_remap) * E, last = p.N_e - 1;
+    const int k0 = element_of_block(block, blocks, tp.xcd_remap) * E, last = p.N_e - 1;
     auto element = [&](int s) { return min(k0 + s, last); };  // past the last: computed, not stored
     double *X = sm + L::x, *woj = sm + L::woj, *F1 = sm + L::f1, *es = sm + L::e;
     EL::LF::stage_tables(tp.lines, F1, tl, TS);
@@ -163,6 +163,69 @@ k_nodal_values_tensor(TensorParams tp, const double* __restrict__ u) {
         }
     }
     if (!ok) atomicOr(p.status, 1);
+}
+
+template <int ELEM, int P>
+__global__ void __launch_bounds__((EulerTune<ELEM, P>::TS), (ELEM == ELEM_TET ? 6 : 1))
+k_nodal_values_tensor(TensorParams tp, const double* __restrict__ u) {
+    nodal_values_body<ELEM, P>(tp, u, blockIdx.x, gridDim.x);
+}
+
+// Triangles of several degrees in one launch: each degree alone leaves most of the chip idle,
+// and branches of a graph overlap only in part (24 problems of degrees 2 to 6, 7,468 triangles:
+// 133 us per RK stage one after the other, 72 us in five branches, 55 us in one launch of each
+// kernel: 17 us here and 38 us for the time derivative, 1.5 rounds of its 5 wavefronts per SIMD).
+__global__ void __launch_bounds__(64) k_nodal_values_tri_groups(TriGroups a) {
+    static_assert(K1Layout<ELEM_TRI, 2>::size * 8 <= 65536 && K1Layout<ELEM_TRI, 6>::size * 8 <= 65536,
+                  "LDS without an attribute");
+    int block = blockIdx.x;
+#define SSE_TRI_GROUP(PP)                                                                           \
+    if (block < a.g[PP - 2].blocks1)                                                                \
+        return nodal_values_body<ELEM_TRI, PP>(a.g[PP - 2].params(), a.g[PP - 2].rk.u, block, a.g[PP - 2].blocks1); \
+    block -= a.g[PP - 2].blocks1;
+    SSE_TRI_GROUP(6)
+    SSE_TRI_GROUP(5)
+    SSE_TRI_GROUP(4)
+    SSE_TRI_GROUP(3)
+    SSE_TRI_GROUP(2)
+#undef SSE_TRI_GROUP
+}
+
+template <int P>
+void tri_k1_config(int N_e, int* blocks, int* lds) {
+    using T = EulerTune<ELEM_TRI, P>;
+    static_assert(T::TS == 64, "one block size");
+    *blocks = (N_e + T::E - 1) / T::E;
+    *lds = (int)sizeof(double) * K1Layout<ELEM_TRI, P>::size;
+}
+
+void tri_k1_config(int P, int N_e, int* blocks, int* lds) {
+    switch (P) {
+        case 2: return tri_k1_config<2>(N_e, blocks, lds);
+        case 3: return tri_k1_config<3>(N_e, blocks, lds);
+        case 4: return tri_k1_config<4>(N_e, blocks, lds);
+        case 5: return tri_k1_config<5>(N_e, blocks, lds);
+        default: return tri_k1_config<6>(N_e, blocks, lds);
+    }
+}
+
+int tri_nodal_blocks(int P, int N_e) {
+    int blocks, lds;
+    tri_k1_config(P, N_e, &blocks, &lds);
+    return blocks;
+}
+
+hipError_t launch_nodal_values_tri_groups(const TriGroups& a, hipStream_t s) {
+    int most = 0, blocks = 0;
+    for (int P = 2; P <= 6; ++P) {
+        if (!a.g[P - 2].blocks1) continue;
+        int b, lds;
+        tri_k1_config(P, a.g[P - 2].N_e, &b, &lds);
+        most = lds > most ? lds : most;
+        blocks += a.g[P - 2].blocks1;
+    }
+    hipLaunchKernelGGL(k_nodal_values_tri_groups, dim3(blocks), dim3(64), most, s, a);
+    return hipGetLastError();
 }
 
 // ----------------------------------------------------------------------------- time_derivative
