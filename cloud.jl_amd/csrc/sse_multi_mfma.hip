@@ -10,9 +10,15 @@
 // chains interleave. The operator (A) fragments are read from global memory (the same
 // small operator for every workgroup, so they stay in L2), a group of four K steps ahead;
 // the element data (B) and the results live in LDS (the facet rows reuse the space of the
-// modal coefficients, a chunk at a time, so that two workgroups fit a compute unit). The
-// entropy-variable maps run per (element, node) between the products, as in
-// k_nodal_values_generic.
+// modal coefficients, a chunk at a time, and no row of a tile's padding is kept, so that three
+// workgroups fit a compute unit at 20 modes and 64 nodes). The entropy-variable maps run per
+// (element, node) between the products, as in k_nodal_values_generic.
+//
+// Bound by latency (operator fragments, the maps' logarithms, barriers) at three wavefronts per
+// SIMD. 10,368 Tet elements of p = 3: 133 us, with the permuted columns and the third workgroup
+// 125. Eight wavefronts per workgroup were slower (by 10 us, and by 40 with registers for six per
+// SIMD). The products of the mass solve stay: one with a kept inverse mass matrix took 104 us, but
+// its rounding goes through e2c and raised the residual's error by up to 30 %.
 //
 // Lane layout of v_mfma_f64_16x16x4f64 (checked on the device): lane l supplies
 // A[l % 16][l / 16] and B[l / 16][l % 16], and receives D[4 r + l / 16][l % 16], r = 0..3.
@@ -31,16 +37,26 @@ constexpr int MF_E = 16;  // elements per workgroup
 
 __host__ __device__ constexpr int round16(int n) { return (n + 15) / 16 * 16; }
 __host__ __device__ constexpr int round4(int n) { return (n + 3) / 4 * 4; }
+__host__ __device__ constexpr int rows_x(int N_p) { return N_p < 16 ? 16 : round4(N_p); }
 
-// C[0, Mp) x [0, NCOL) = A B, A (M x K) through the accessor a(i, k) (zero outside the
-// operator), B (Kp x NCOL) and C row-major in LDS with leading dimension NCOL; Mp a
-// multiple of 16, Kp of 4. Wave w takes the tiles w, w + nw, ... in pairs; the K steps go
-// in groups of four, the operator fragments of the next group requested before the
-// MFMAs of the current one.
+// Element data in LDS: row-major, each row's columns permuted within their sixteens. Rows are 160
+// or 128 words apart, so unpermuted the lanes of the (element, node) loops, one row each, met in
+// two banks.
+template <int NCOL>
+__device__ __forceinline__ int at(int row, int col) {
+    return row * NCOL + (col ^ (row & 15));
+}
+
+// C[0, M) x [0, NCOL) = A B, A (M x K) through the accessor a(i, k) (zero outside the
+// operator), B (Kp x NCOL) and C in LDS; Kp a multiple of 4. Wave w takes the tiles w, w + nw, ...
+// in pairs (the count from another wave in each workgroup, as the waves of one number share a
+// SIMD); the K steps go in groups of four, the operator fragments of the next group requested
+// before the MFMAs of the current one.
 template <int NCOL, class AFn>
-__device__ __forceinline__ void mm_tiles(const AFn& a, int Mp, int Kp, const double* B, double* C) {
+__device__ __forceinline__ void mm_tiles(const AFn& a, int M, int Kp, const double* B, double* C) {
     constexpr int NT = NCOL / 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int Mp = round16(M);
+    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6, wave = ((threadIdx.x >> 6) + blockIdx.x) & (nw - 1);
     const int li = lane & 15, lk = lane >> 4;
     const int units = (Mp / 16) * NT, steps = Kp / 4, groups = (steps + 3) / 4;
     for (int u0 = wave; u0 < units; u0 += 2 * nw) {
@@ -67,7 +83,7 @@ __device__ __forceinline__ void mm_tiles(const AFn& a, int Mp, int Kp, const dou
                 const int st = 4 * g + q;
                 if (st < steps) {
                     const int k = 4 * st + lk;
-                    const double b0 = B[k * NCOL + 16 * ct0 + li], b1 = B[k * NCOL + 16 * ct1 + li];
+                    const double b0 = B[at<NCOL>(k, 16 * ct0 + li)], b1 = B[at<NCOL>(k, 16 * ct1 + li)];
                     acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(c0[q], b0, acc0, 0, 0, 0);
                     acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(c1[q], b1, acc1, 0, 0, 0);
                 }
@@ -78,12 +94,15 @@ __device__ __forceinline__ void mm_tiles(const AFn& a, int Mp, int Kp, const dou
                 c1[q] = n1[q];
             }
         }
+        auto store = [&](int rt, int ct, const dvec4& acc) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) C[(16 * rt0 + 4 * r + lk) * NCOL + 16 * ct0 + li] = acc0[r];
-        if (two) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) C[(16 * rt1 + 4 * r + lk) * NCOL + 16 * ct1 + li] = acc1[r];
-        }
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * rt + 4 * r + lk;
+                if (row < M) C[at<NCOL>(row, 16 * ct + li)] = acc[r];
+            }
+        };
+        store(rt0, ct0, acc0);
+        if (two) store(rt1, ct1, acc1);
     }
 }
 
@@ -94,9 +113,9 @@ __global__ void __launch_bounds__(256) k_nodal_values_mfma(DevParams p, const do
     static_assert(NCOL % 16 == 0, "16 elements of NC components fill whole column tiles");
     extern __shared__ double sm[];
     const int N_p = p.N_p, N_q = p.N_q, N_f = p.N_f, N_e = p.N_e;
-    const int NPp = round16(N_p), NQp = round16(N_q);
-    double* X = sm;                // NPp x NCOL: modal coefficients, then NPp facet rows at a time
-    double* Y = X + NPp * NCOL;    // NQp x NCOL: volume nodes
+    const int NPp = round4(N_p), NQp = round4(N_q), XR = rows_x(N_p);
+    double* X = sm;               // XR x NCOL: modal coefficients, then facet rows, a chunk at a time
+    double* Y = X + XR * NCOL;    // NQp x NCOL: volume nodes
     const int k0 = blockIdx.x * MF_E;
     const int tid = threadIdx.x, nt = blockDim.x;
 
@@ -106,7 +125,7 @@ __global__ void __launch_bounds__(256) k_nodal_values_mfma(DevParams p, const do
     __syncthreads();
     for (int t = tid; t < MF_E * NC * N_p; t += nt) {
         const int e = t / (NC * N_p), r = t - e * NC * N_p, c = r / N_p, j = r - c * N_p;
-        if (k0 + e < N_e) X[j * NCOL + e * NC + c] = u[(size_t)(k0 + e) * NC * N_p + r];
+        if (k0 + e < N_e) X[at<NCOL>(j, e * NC + c)] = u[(size_t)(k0 + e) * NC * N_p + r];
     }
     __syncthreads();
 
@@ -115,61 +134,61 @@ __global__ void __launch_bounds__(256) k_nodal_values_mfma(DevParams p, const do
 
     bool ok = true;
 
-    mm_tiles<NCOL>(aV, NQp, round4(N_p), X, Y);  // u_q = V u
+    mm_tiles<NCOL>(aV, NQp, NPp, X, Y);  // u_q = V u
     __syncthreads();
     for (int t = tid; t < MF_E * N_q; t += nt) {  // WJ c2e(u_q)
         const int e = t / N_q, i = t - e * N_q, k = k0 + e;
         double ub[NC], wb[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) ub[c] = Y[i * NCOL + e * NC + c];
+        for (int c = 0; c < NC; ++c) ub[c] = Y[at<NCOL>(i, e * NC + c)];
         const bool good = Ph::c2e(p.law, ub, wb);
         if (k < N_e) ok &= good;
         const double wj = k < N_e ? p.W[i] * p.Jq[(size_t)k * N_q + i] : 0.0;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) Y[i * NCOL + e * NC + c] = k < N_e ? wb[c] * wj : 0.0;
+        for (int c = 0; c < NC; ++c) Y[at<NCOL>(i, e * NC + c)] = k < N_e ? wb[c] * wj : 0.0;
     }
     __syncthreads();
-    mm_tiles<NCOL>(aVt, NPp, round4(N_q), Y, X);  // w = V' (WJ w_q)
+    mm_tiles<NCOL>(aVt, NPp, NQp, Y, X);  // w = V' (WJ w_q)
     __syncthreads();
-    mm_tiles<NCOL>(aV, NQp, round4(N_p), X, Y);  // V w
+    mm_tiles<NCOL>(aV, NQp, NPp, X, Y);  // V w
     __syncthreads();
     for (int t = tid; t < MF_E * N_q; t += nt) {  // J^{-1} W (V w)
         const int e = t / N_q, i = t - e * N_q, k = k0 + e;
         const double jw = k < N_e ? p.W[i] / p.Jq[(size_t)k * N_q + i] : 0.0;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) Y[i * NCOL + e * NC + c] *= jw;
+        for (int c = 0; c < NC; ++c) Y[at<NCOL>(i, e * NC + c)] *= jw;
     }
     __syncthreads();
-    mm_tiles<NCOL>(aVt, NPp, round4(N_q), Y, X);  // w = V' (...)
+    mm_tiles<NCOL>(aVt, NPp, NQp, Y, X);  // w = V' (...)
     __syncthreads();
-    mm_tiles<NCOL>(aV, NQp, round4(N_p), X, Y);  // w_q = V w
+    mm_tiles<NCOL>(aV, NQp, NPp, X, Y);  // w_q = V w
     __syncthreads();
-    // u_q = e2c(w_q); then w_f = R w_q, NPp facet rows at a time in the space of X
+    // u_q = e2c(w_q); then w_f = R w_q, a chunk of facet rows at a time in the space of X
     for (int t = tid; t < MF_E * N_q; t += nt) {
         const int e = t / N_q, i = t - e * N_q, k = k0 + e;
         if (k >= N_e) continue;
         double ub[NC], wb[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) wb[c] = Y[i * NCOL + e * NC + c];
+        for (int c = 0; c < NC; ++c) wb[c] = Y[at<NCOL>(i, e * NC + c)];
         ok &= Ph::e2c(p.law, wb, ub);
         double* uqk = p.uq + (size_t)k * N_q * NC;
 #pragma unroll
         for (int c = 0; c < NC; ++c) uqk[i + N_q * c] = ub[c];
     }
-    for (int f0 = 0; f0 < N_f; f0 += NPp) {
-        const int rows = min(NPp, round16(N_f - f0));
+    const int chunk = XR / 16 * 16;
+    for (int f0 = 0; f0 < N_f; f0 += chunk) {
+        const int nf = min(chunk, N_f - f0);
         auto aR = [&](int i, int k) {
             return (f0 + i < N_f && k < N_q) ? p.Rd[f0 + i + (size_t)N_f * k] : 0.0;
         };
-        mm_tiles<NCOL>(aR, rows, round4(N_q), Y, X);
+        mm_tiles<NCOL>(aR, nf, NQp, Y, X);
         __syncthreads();
-        const int nf = min(NPp, N_f - f0);
         for (int t = tid; t < MF_E * nf; t += nt) {  // u_f = e2c(w_f)
             const int e = t / nf, jl = t - e * nf, k = k0 + e;
             if (k >= N_e) continue;
             double ub[NC], wb[NC];
 #pragma unroll
-            for (int c = 0; c < NC; ++c) wb[c] = X[jl * NCOL + e * NC + c];
+            for (int c = 0; c < NC; ++c) wb[c] = X[at<NCOL>(jl, e * NC + c)];
             ok &= Ph::e2c(p.law, wb, ub);
             double* ufk = p.uf + (size_t)k * N_f * NC;
 #pragma unroll
@@ -183,7 +202,7 @@ __global__ void __launch_bounds__(256) k_nodal_values_mfma(DevParams p, const do
 }  // namespace
 
 size_t lds_nodal_values_mfma(const DevParams& p) {
-    return sizeof(double) * (size_t)(round16(p.N_p) + round16(p.N_q)) * MF_E * p.N_c;
+    return sizeof(double) * (size_t)(rows_x(p.N_p) + round4(p.N_q)) * MF_E * p.N_c;
 }
 
 // Euler in 2D or 3D with the entropy projection and a modal V only
