@@ -550,19 +550,14 @@ k_vjp_v2_tensor(TensorParams tp, StructTables st, double* __restrict__ rbar, con
         }
     }
     __syncthreads();
-    // ---- phase D: cotangents of the entropy variables, w = c2e(u): volume and facet
-    if (half == 0 && tl < NQ) {
-        if (SPLIT > 1 && !EARLY) {
+    // ---- phase D: cotangents of the entropy variables, w = c2e(u): the volume nodes on the first
+    // half-team, the facet nodes beside them on the last (one after the other on the first, and a
+    // tree of barriers for λ, took 7 us of the pull-back's 286 at 10,368 Tet p = 3 elements)
+    double wb[NC];
 #pragma unroll
-            for (int e = 0; e < NC; ++e) ubq[e] += sub[e * NQ + tl];
-        }
-        if constexpr (!DET) {
-#pragma unroll
-            for (int e = 0; e < NC; ++e) ubq[e] += srow[e * NQ + tl];
-        }
-    }
-    if (half == 0 && tl < NF) {
-        double ubf[NC], hf[NH];
+    for (int e = 0; e < NC; ++e) wb[e] = 0.0;
+    if (half == SPLIT - 1 && tl < NF) {
+        double ubf[NC], hf[NH], wf[NC];
         if constexpr (DET) {  // the node's chunk slots, in chunk order
 #pragma unroll
             for (int e = 0; e < NC; ++e) ubf[e] = 0.0;
@@ -580,30 +575,37 @@ k_vjp_v2_tensor(TensorParams tp, StructTables st, double* __restrict__ rbar, con
         // the C-pair sums are (rho, v, p) cotangents: to conservative, beside the interface part
         double ubc[NC];
 #pragma unroll
-        for (int e = 0; e < NC; ++e) ubc[e] = swf[e * NF + tl];
+        for (int e = 0; e < NC; ++e) {
+            ubc[e] = swf[e * NF + tl];
+            wf[e] = 0.0;
+        }
         A::prim_cot_to_cons(p.law, hf, ubf, ubc);
-        double wb[NC];
+        A::e2c_adj_prim(p.law, hf[A::H_RHO], hf + A::H_V, hf[A::H_P], ubc, wf);
 #pragma unroll
-        for (int e = 0; e < NC; ++e) wb[e] = 0.0;
-        A::e2c_adj_prim(p.law, hf[A::H_RHO], hf + A::H_V, hf[A::H_P], ubc, wb);
-#pragma unroll
-        for (int e = 0; e < NC; ++e) swf[e * NF + tl] = wb[e];
+        for (int e = 0; e < NC; ++e) swf[e * NF + tl] = wf[e];
     }
-    __syncthreads();  // the w_f cotangents are complete
     if (half == 0 && tl < NQ) {
-        double wb[NC];
+        if (SPLIT > 1 && !EARLY) {
+#pragma unroll
+            for (int e = 0; e < NC; ++e) ubq[e] += sub[e * NQ + tl];
+        }
+        if constexpr (!DET) {
+#pragma unroll
+            for (int e = 0; e < NC; ++e) ubq[e] += srow[e * NQ + tl];
+        }
 #pragma unroll
         for (int v = 0; v < NH; ++v) hi[v] = sh[v * NQ + tl];
         // the pair sums are (rho, v, p) cotangents: to conservative once per node
         double ubc[NC];
 #pragma unroll
-        for (int e = 0; e < NC; ++e) {
-            ubc[e] = 0.0;
-            wb[e] = 0.0;
-        }
+        for (int e = 0; e < NC; ++e) ubc[e] = 0.0;
         A::prim_cot_to_cons(p.law, hi, ubq, ubc);
         A::e2c_adj_prim(p.law, hi[A::H_RHO], hi + A::H_V, hi[A::H_P], ubc, wb);
-        // w_q' cotangent += R' (w_f cotangent)
+    }
+    __syncthreads();  // the w_f cotangents are complete
+    if (half == 0 && tl < NQ) {
+        // w_q' cotangent += R' (w_f cotangent), into the element's slice of rbar
+        double* wk = rbar + (size_t)k * NQ * NC;
 #pragma unroll
         for (int w = 0; w < MAXR; ++w) {
             if (rj[w] < 0) continue;
@@ -611,19 +613,27 @@ k_vjp_v2_tensor(TensorParams tp, StructTables st, double* __restrict__ rbar, con
             for (int e = 0; e < NC; ++e) wb[e] += rv[w] * swf[e * NF + rj[w]];
         }
 #pragma unroll
-        for (int e = 0; e < NC; ++e) sub[e * NQ + tl] = wb[e];
+        for (int e = 0; e < NC; ++e) wk[e * NQ + tl] = wb[e];
     }
-    __syncthreads();  // the w_q' cotangent is complete
-    double* wk = rbar + (size_t)k * NQ * NC;
-    for (int t = tt; t < NQ * NC; t += TS) wk[t] = sub[t];
-    // λ cotangent of this element, summed in a fixed order
-    red[tt] = lam;
-    __syncthreads();
-    for (int s = TS / 2; s > 0; s >>= 1) {
-        if (tt < s) red[tt] += red[tt + s];
+    // λ cotangent of this element, held by the last half-team, summed in a fixed order: its
+    // wavefronts' shares by halves (in the C sums' array, free after the barrier above), then
+    // within the first of them
+    if constexpr (NT > 64) {
+        if (half == SPLIT - 1) red[tl] = lam;
         __syncthreads();
+        if (half == SPLIT - 1 && tl < 64) {
+#pragma unroll
+            for (int w = NT / 2; w >= 64; w >>= 1) {
+                for (int t = tl; t < w; t += 64) red[t] += red[t + w];
+            }
+            lam = red[tl];
+        }
     }
-    if (tt == 0) lam_partial[k] = (out.accumulate ? lam_partial[k] : 0.0) + out.scale * red[0];
+    if (half == SPLIT - 1 && tl < 64) {
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) lam += __shfl_down(lam, w, 64);
+        if (tl == 0) lam_partial[k] = (out.accumulate ? lam_partial[k] : 0.0) + out.scale * lam;
+    }
 }
 
 // V3: the reverse of w_q' = V M^{-1} V' (WJ c2e(V u)): ubar (+)= scale *
