@@ -2109,6 +2109,7 @@ struct sse_batch {
     std::vector<hipStream_t> branch;
     std::vector<hipEvent_t> join;
     hipEvent_t fork = nullptr;
+    int* any_status = nullptr;  // the groups' status words, combined
     std::string err;
 };
 
@@ -2188,6 +2189,80 @@ int ensemble_chunk(const sse_desc* D, int R) {
     cap = std::min<size_t>(cap, 2 * (size_t)R);
     cap &= ~(size_t)1;
     return (int)std::max<size_t>(cap, 2);
+}
+
+// The members' states into the group buffers with each element's time step, or back: one launch
+// per MOVES problems. With a copy per problem, an upload of the time steps and a wait for it per
+// group and a status read per group, ten steps of 24 triangle problems took 3,218 us, five of 16
+// diffusivities (1,296 tetrahedra) 2,832; now 2,946 and 2,733.
+constexpr int MOVES = 32, MOVE_CHUNK = 2048;
+
+struct Moves {
+    int n, back;
+    int first[MOVES + 1];  // blocks: MOVE_CHUNK values each
+    double* user[MOVES];   // null: time steps only (the states are copied by the runtime)
+    double* group[MOVES];
+    size_t len[MOVES];
+    double* dt_e[MOVES];
+    size_t elems[MOVES];
+    double dt[MOVES];
+};
+
+__global__ void __launch_bounds__(256) k_batch_move(Moves m, int* any_status) {
+    if (any_status && blockIdx.x == 0 && threadIdx.x == 0) *any_status = 0;
+    int i = 0;
+    while (i + 1 < m.n && (int)blockIdx.x >= m.first[i + 1]) ++i;
+    const size_t t0 = (size_t)(blockIdx.x - m.first[i]) * MOVE_CHUNK + threadIdx.x;
+    const double dt = m.dt[i];
+#pragma unroll
+    for (int q = 0; q < MOVE_CHUNK / 256; ++q) {
+        const size_t t = t0 + q * 256;
+        if (t >= m.len[i]) break;
+        if (m.back) {
+            m.user[i][t] = m.group[i][t];
+        } else {
+            if (m.user[i]) m.group[i][t] = m.user[i][t];
+            if (t < m.elems[i]) m.dt_e[i][t] = dt;
+        }
+    }
+}
+
+struct StatusWords {
+    int n;
+    const int* word[64];
+};
+
+__global__ void __launch_bounds__(64) k_any_status(StatusWords w, int* any) {
+    const int t = threadIdx.x;
+    if (t < w.n && *w.word[t]) atomicOr(any, 1);
+}
+
+hipError_t batch_move(sse_batch* b, double* const* u, const double* dt, bool states, bool back) {
+    Moves m = {};
+    hipError_t e = hipSuccess;
+    int* any = b->any_status;  // cleared by the first launch
+    auto flush = [&]() {
+        if (!m.n || e != hipSuccess) return;
+        hipLaunchKernelGGL(k_batch_move, dim3(m.first[m.n]), dim3(256), 0, b->stream, m, back ? nullptr : any);
+        e = hipGetLastError();
+        any = nullptr;
+        m.n = 0;
+    };
+    m.back = back ? 1 : 0;
+    for (size_t g = 0; g < b->groups.size(); ++g)
+        for (size_t t = 0; t < b->members[g].size(); ++t) {
+            const int i = b->members[g][t], q = m.n;
+            m.user[q] = states ? u[i] : nullptr;
+            m.group[q] = b->state[g] + b->per_elem[i] * b->offsets[g][t];
+            m.len[q] = b->per_elem[i] * b->elems[i];
+            m.dt_e[q] = b->dt_e[g] + b->offsets[g][t];
+            m.elems[q] = b->elems[i];
+            m.dt[q] = dt[i];
+            m.first[q + 1] = m.first[q] + (int)((m.len[q] + MOVE_CHUNK - 1) / MOVE_CHUNK);
+            if (++m.n == MOVES) flush();
+        }
+    flush();
+    return e;
 }
 
 // The groups whose stages go into one launch each for all of them (sse::TriGroups): the first
@@ -2272,6 +2347,7 @@ int sse_batch_create(const sse_desc* const* descs, int32_t n, sse_batch** out) {
         b->per_elem[i] = (size_t)descs[i]->N_p * descs[i]->N_c;
     }
     if (hipStreamCreate(&b->stream) != hipSuccess) return cleanup(SSE_ERR_HIP, "hipStreamCreate failed");
+    if (hipMalloc(&b->any_status, sizeof(int)) != hipSuccess) return cleanup(SSE_ERR_OUT_OF_MEMORY, "hipMalloc failed");
     // ensembles first: StandardForm scalar problems on one mesh that differ at most in b
     std::vector<std::vector<int>> ens;
     for (int i = 0; i < n; ++i) {
@@ -2394,31 +2470,24 @@ int sse_batch_rk_steps(sse_batch* b, double* const* u, const double* dt, int32_t
     if (!b) return SSE_ERR_INVALID_ARGUMENT;
     if (!u || !dt || nsteps < 0) return bfail(b, SSE_ERR_INVALID_ARGUMENT, "u or dt is NULL, or nsteps < 0");
     if (where != SSE_DEVICE && where != SSE_HOST) return bfail(b, SSE_ERR_INVALID_ARGUMENT, "bad `where`");
-    const hipMemcpyKind in = where == SSE_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-    const hipMemcpyKind outk = where == SSE_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     auto hip_ok = [&](hipError_t e, const char* what) {
         if (e == hipSuccess) return 0;
         return bfail(b, SSE_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
     };
     int rc;
     // gather states and per-element time steps into the group buffers
-    for (size_t g = 0; g < b->groups.size(); ++g) {
-        std::vector<double> de;
+    const bool device = where == SSE_DEVICE;
+    for (size_t g = 0; g < b->groups.size(); ++g)
         for (size_t t = 0; t < b->members[g].size(); ++t) {
             const int i = b->members[g][t];
             if (!u[i]) return bfail(b, SSE_ERR_INVALID_ARGUMENT, "u[" + std::to_string(i) + "] is NULL");
+            if (device) continue;
             const size_t n_i = b->per_elem[i] * b->elems[i];
             if ((rc = hip_ok(hipMemcpyAsync(b->state[g] + b->per_elem[i] * b->offsets[g][t], u[i],
-                                            n_i * sizeof(double), in, b->stream), "state gather")))
+                                            n_i * sizeof(double), hipMemcpyHostToDevice, b->stream), "state gather")))
                 return rc;
-            de.insert(de.end(), b->elems[i], dt[i]);
         }
-        if ((rc = hip_ok(hipMemcpyAsync(b->dt_e[g], de.data(), de.size() * sizeof(double), hipMemcpyHostToDevice,
-                                        b->stream), "dt upload")))
-            return rc;
-        // the host vector must outlive the copy
-        if ((rc = hip_ok(hipStreamSynchronize(b->stream), "sync"))) return rc;
-    }
+    if ((rc = hip_ok(batch_move(b, u, dt, device, false), "state gather"))) return rc;
     // units of work that do not depend on each other: a group, or the triangle groups that share
     // their launches (all of them under the first one's number)
     const std::vector<size_t> tri = tri_groups(b);
@@ -2491,17 +2560,33 @@ int sse_batch_rk_steps(sse_batch* b, double* const* u, const double* dt, int32_t
     for (; step < nsteps; ++step)
         if ((rc = one_step())) return rc;
     // scatter back
-    for (size_t g = 0; g < b->groups.size(); ++g)
-        for (size_t t = 0; t < b->members[g].size(); ++t) {
-            const int i = b->members[g][t];
-            const size_t n_i = b->per_elem[i] * b->elems[i];
-            if ((rc = hip_ok(hipMemcpyAsync(u[i], b->state[g] + b->per_elem[i] * b->offsets[g][t],
-                                            n_i * sizeof(double), outk, b->stream), "state scatter")))
-                return rc;
-        }
-    if ((rc = hip_ok(hipStreamSynchronize(b->stream), "sync"))) return rc;
-    for (sse_handle* h : b->groups)
-        if ((rc = check_status(h))) return bfail(b, rc, h->err);
+    if (device) {
+        if ((rc = hip_ok(batch_move(b, u, dt, true, true), "state scatter"))) return rc;
+    } else {
+        for (size_t g = 0; g < b->groups.size(); ++g)
+            for (size_t t = 0; t < b->members[g].size(); ++t) {
+                const int i = b->members[g][t];
+                const size_t n_i = b->per_elem[i] * b->elems[i];
+                if ((rc = hip_ok(hipMemcpyAsync(u[i], b->state[g] + b->per_elem[i] * b->offsets[g][t],
+                                                n_i * sizeof(double), hipMemcpyDeviceToHost, b->stream),
+                                 "state scatter")))
+                    return rc;
+            }
+    }
+    // a non-physical state in any group: then each group's own check names it
+    for (size_t g0 = 0; g0 < b->groups.size(); g0 += 64) {
+        StatusWords w = {};
+        for (size_t g = g0; g < std::min(g0 + 64, b->groups.size()); ++g) w.word[w.n++] = b->groups[g]->P.status;
+        hipLaunchKernelGGL(k_any_status, dim3(1), dim3(64), 0, b->stream, w, b->any_status);
+        if ((rc = hip_ok(hipGetLastError(), "kernel launch"))) return rc;
+    }
+    int any = 0;
+    if ((rc = hip_ok(hipMemcpyAsync(&any, b->any_status, sizeof(int), hipMemcpyDeviceToHost, b->stream), "status")) ||
+        (rc = hip_ok(hipStreamSynchronize(b->stream), "sync")))
+        return rc;
+    if (any)
+        for (sse_handle* h : b->groups)
+            if ((rc = check_status(h))) return bfail(b, rc, h->err);
     return 0;
 }
 
@@ -2612,6 +2697,7 @@ void sse_batch_destroy(sse_batch* b) {
     for (hipEvent_t ev : b->join)
         if (ev) (void)hipEventDestroy(ev);
     if (b->fork) (void)hipEventDestroy(b->fork);
+    if (b->any_status) (void)hipFree(b->any_status);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }

@@ -60,3 +60,24 @@ def test_rk_steps(name, graph):
     for c, (s, u0, dt), u in zip(BATCHES[name], probs, states):
         want = O.rk_steps(s.arrays, u0, dt, 6)
         assert np.abs(to_host(u) - want).max() <= 1e-10 * np.abs(want).max(), (c, batch.describe())
+
+
+@pytest.mark.parametrize("host", [False, True], ids=["device", "host"])
+def test_more_problems_than_one_move(host):
+    """33 problems (one more than the states moved by a launch), and a state that is not physical
+    in the last of them: reported, and gone with the next call."""
+    from sse.batch import BatchError, BatchedSolver
+    from sse.time_integration import to_device, to_host
+    probs = [_problem("tri", 2 + i % 3, 1 + i % 2) for i in range(33)]
+    batch = BatchedSolver([s for s, _, _ in probs])
+    fresh = lambda: [np.array(u0, order="F") if host else to_device(u0) for _, u0, _ in probs]
+    dts = [dt for _, _, dt in probs]
+    bad = fresh()
+    bad[-1][...] = -1.0
+    with pytest.raises(BatchError, match="non-physical"):
+        batch.rk_steps(bad, dts, 1)
+    states = fresh()
+    batch.rk_steps(states, dts, 3)
+    for (s, u0, dt), u in zip(probs, states):
+        want = O.rk_steps(s.arrays, u0, dt, 3)
+        assert np.abs((u if host else to_host(u)) - want).max() <= 1e-10 * np.abs(want).max()
