@@ -2104,8 +2104,9 @@ struct sse_batch {
     hipStream_t stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    // the captured RK step runs each group's five stages on a stream of its own (a branch
-    // of the graph, forked from and joined to `stream`), so that groups overlap
+    // the captured RK step runs the five stages of each group, or of the triangle groups that
+    // share launches, on a stream of its own (a branch of the graph, forked from and joined to
+    // `stream`), so that they overlap
     std::vector<hipStream_t> branch;
     std::vector<hipEvent_t> join;
     hipEvent_t fork = nullptr;
