@@ -101,6 +101,7 @@ struct sse_handle {
     int erk_stages = 0;
     double* stage_u = nullptr;
     double* stage_dudt = nullptr;
+    double* u_copy = nullptr;    // StandardForm scalar kernels: u of a residual whose dudt covers u in part
     double* fpartial = nullptr;  // functionals: per-element partial sums and the result
     double* fout = nullptr;
     double* ferr = nullptr;      // staging of u_exact for sse_l2_error with host arrays
@@ -995,6 +996,8 @@ int build_pairs(sse_handle* h, const sse_desc* D) {
     return 0;
 }
 
+size_t state_size(const sse_handle* h) { return (size_t)h->P.N_p * h->P.N_c * h->P.N_e; }
+
 int launch(sse_handle* h, const double* u, double* dudt, const RKStage& rk, int which,
            const sse::ErkTail& tail = sse::ErkTail{}) {
     if (h->use_struct) {
@@ -1006,6 +1009,15 @@ int launch(sse_handle* h, const double* u, double* dudt, const RKStage& rk, int 
     }
     hipError_t e;
     if (h->use_std_tensor) {
+        // the time derivative reads u of its own element again: dudt may be u, but where it
+        // covers u in part it would overwrite other elements first
+        const size_t n = state_size(h);
+        if (which == 3 && !rk.active && u != dudt && sse::overlap(u, dudt, n)) {
+            int rc;
+            if (!h->u_copy && (rc = alloc(h, n, &h->u_copy))) return rc;
+            SSE_HIP_TRY(h, hipMemcpyAsync(h->u_copy, u, n * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+            u = h->u_copy;
+        }
         e = sse::launch_std_tensor(h->TP, 1, nullptr, 0, u, dudt, rk, h->stream, which);
     } else if (h->P.standard) {  // phase 1 without entropy projection, then the StandardForm kernels
         e = (which & 1) ? sse::launch_generic_dispatch(h->P, u, dudt, rk, h->stream, 1, tail) : hipSuccess;
@@ -1039,8 +1051,6 @@ int check_status(sse_handle* h) {
     }
     return 0;
 }
-
-size_t state_size(const sse_handle* h) { return (size_t)h->P.N_p * h->P.N_c * h->P.N_e; }
 
 }  // namespace
 

@@ -420,9 +420,11 @@ hipError_t launch_generic(const DevParams& p, const double* u, double* dudt, con
                           int which /* bit 0: phase 1, bit 1: phase 2 */, const ErkTail& tail) {
     dim3 grid(p.N_e), block(256);
     // nodal diagonal-E schemes: u_q = u and u_f selects from it, so a whole residual reads u
-    // directly and needs no phase 1. Not inside an RK stage, whose epilogue updates u while
-    // other workgroups still read their neighbours' states.
-    const bool direct = which == 3 && !rk.active && p.ec && p.sel && !p.has_V;
+    // directly and needs no phase 1. Not where u is written while other workgroups still read
+    // their neighbours' states: inside an RK stage, whose epilogue updates u, and with dudt in
+    // the memory of u.
+    const bool direct = which == 3 && !rk.active && p.ec && p.sel && !p.has_V &&
+                        !overlap(u, dudt, (size_t)p.N_p * p.N_c * p.N_e);
     if (direct) {
         which = 2;
     } else if ((which & 1) && p.mfma) {

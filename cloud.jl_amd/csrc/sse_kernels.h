@@ -178,4 +178,10 @@ struct ErkTail {
     double* out;
 };
 
+// The n values at a and the n at b share memory (a == b included).
+inline bool overlap(const double* a, const double* b, size_t n) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + n * sizeof(double) && y < x + n * sizeof(double);
+}
+
 }  // namespace sse

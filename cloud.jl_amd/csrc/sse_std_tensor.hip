@@ -465,6 +465,8 @@ __global__ void __launch_bounds__((StdTune<ELEM, P>::TS), std_waves(P))
 // ----------------------------------------------------------------------------- time derivative
 // dudt = M^{-1} V' [ sum_n VT_n(f_n) - R' (B J_f f*) ],  f_n = a_n u - b q_n,
 // f* = a.n {u} + halfl |a.n| [u] - b {q}.n (LF; BR1 when second order).
+// dudt may be u, and an RK stage updates u: a workgroup reads u of its own slots only, all of it
+// before the barriers that precede its stores.
 template <int ELEM, int P>
 struct StdTdLayout {
     using G = LineGrid<ELEM, P>;
@@ -475,7 +477,7 @@ struct StdTdLayout {
 
 template <int ELEM, int P, bool SKEW, bool SECOND>
 __global__ void __launch_bounds__((StdTune<ELEM, P>::TS), std_waves(P))
-    k_std_td_tensor(TensorParams tp, Ensemble en, const double* __restrict__ u, double* __restrict__ dudt, RKStage rk) {
+    k_std_td_tensor(TensorParams tp, Ensemble en, const double* u, double* dudt, RKStage rk) {
     using G = LineGrid<ELEM, P>;
     using LF = LineFact<ELEM, P>;
     using T = StdTune<ELEM, P>;

@@ -160,7 +160,8 @@ int sse_create(const sse_desc* desc, sse_handle** out);
 
 /* Replaces semi_discrete_residual!(dudt, u, solver, t)
  * (src/Solvers/Solvers.jl:474-514). u and dudt are (N_p, N_c, N_e) column-major;
- * `where` says whether they are device or host pointers. dudt is overwritten.
+ * `where` says whether they are device or host pointers. dudt is overwritten. It may be u
+ * itself or share memory with it: the result is then that of u before the call.
  * The call is asynchronous on the handle's stream for SSE_DEVICE. */
 int sse_residual(sse_handle* h, const double* u, double* dudt, double t, int32_t where);
 
