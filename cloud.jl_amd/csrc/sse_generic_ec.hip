@@ -83,6 +83,23 @@ __global__ void __launch_bounds__(EC_NT)
     double* sff = srq + NC * N_q;     // NC x N_f
     const double* uqk = (direct ? u : p.uq) + (size_t)k * N_q * NC;
     const double* Lk = p.Lam + (size_t)k * N_q * D * D;
+    // All states of this element and its facets in units in which node 0 is near one; the row
+    // sums are converted back as they are read. Node 0 is requested here and used once a node's
+    // own loads are on their way (opaque: else the compiler waits for it before the loop).
+    double u0[NC];
+#pragma unroll
+    for (int e = 0; e < NC; ++e) u0[e] = uqk[N_q * e];
+    ElementUnits<D> units;
+    auto set_units = [&]() {
+        double x[NC];
+#pragma unroll
+        for (int e = 0; e < NC; ++e) {
+            x[e] = u0[e];
+            asm volatile("" : "+v"(x[e]));
+        }
+        units.set(p.law, x);
+    };
+    if (tid >= N_q + N_f) set_units();
 
     // hoisted volume states, metric terms; facet nodes: hoisted states and the interface flux
     for (int t = tid; t < N_q + N_f; t += EC_NT) {
@@ -90,17 +107,18 @@ __global__ void __launch_bounds__(EC_NT)
             double us[NC], h[NH];
 #pragma unroll
             for (int e = 0; e < NC; ++e) us[e] = uqk[t + N_q * e];
+            double Li[D * D];
+#pragma unroll
+            for (int mn = 0; mn < D * D; ++mn) Li[mn] = Lk[t + N_q * mn];
+            set_units();
+            units.in(us);
             hoist<D>(p.law, us, h);
 #pragma unroll
             for (int v = 0; v < NH; ++v) sh[v * N_q + t] = h[v];
 #pragma unroll
             for (int e = 0; e < NC; ++e) srq[e * N_q + t] = 0.0;
-            double Li[D * D];
 #pragma unroll
-            for (int mn = 0; mn < D * D; ++mn) {
-                Li[mn] = Lk[t + N_q * mn];
-                sL[mn * N_q + t] = Li[mn];
-            }
+            for (int mn = 0; mn < D * D; ++mn) sL[mn * N_q + t] = Li[mn];
             if (corr) {
                 for (int f = 0; f < p.N_fac; ++f) {
 #pragma unroll
@@ -134,6 +152,9 @@ __global__ void __launch_bounds__(EC_NT)
                     uout[e] = ufn[jn + N_f * e];
                 }
             }
+            set_units();
+            units.in(uin);
+            units.in(uout);
             hoist<D>(p.law, uin, hin);
             hoist<D>(p.law, uout, hout);
             const double jf = p.Jf[j + (size_t)N_f * k], inv_jf = 1.0 / jf;
@@ -316,7 +337,7 @@ __global__ void __launch_bounds__(EC_NT)
                 for (int e = 0; e < NC; ++e) a[e] += q * x[e * stride];
             }
 #pragma unroll
-            for (int e = 0; e < NC; ++e) sp[(part * NC + e) * N_p + j] = a[e];
+            for (int e = 0; e < NC; ++e) sp[(part * NC + e) * N_p + j] = units.out(e, a[e]);
         }
         __syncthreads();
         for (int t = tid; t < N_p * NC; t += EC_NT) {
@@ -358,7 +379,7 @@ __global__ void __launch_bounds__(EC_NT)
             double s = srq[t];
 #pragma unroll 4
             for (int c = p.Rt_ptr[i]; c < p.Rt_ptr[i + 1]; ++c) s -= p.Rt_val[c] * sff[p.Rt_idx[c] + N_f * e];
-            so[t] = s / (p.W[i] * Jk[i]);
+            so[t] = units.out(e, s / (p.W[i] * Jk[i]));
         }
     }
     __syncthreads();

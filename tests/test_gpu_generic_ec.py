@@ -93,3 +93,36 @@ def test_stage_combination_in_the_epilogue(stages):
     erk_steps(solver, u, 1e-3, 3, alg)
     ref = O.erk_steps(solver.arrays, ode.u0, 1e-3, 3, alg.A, alg.b)
     assert _rel(to_host(u), ref) <= 1e-10
+
+
+UNITS = [(17, 8), (-20, 8), (0, -9), (-300, 150), (300, -90)]  # powers of two of density and of velocity
+
+
+@pytest.mark.parametrize("a,c", UNITS)
+@pytest.mark.parametrize("name", ["hex_p2", "hex_p4", "line"])
+def test_residual_does_not_depend_on_the_units(name, a, c):
+    """A state in units of 2^a for density and 2^c for velocity (pressures from 2^-63 to 2^316; the
+    first ones are near those of air in kg, m and s, p / rho = 6e4): such a change of units is exact, so
+    the deterministic residual of a nodal scheme is that of the state near one, bit by bit. (The tests
+    above compare states near one with the oracle.)"""
+    import torch
+    from sse import semi_discrete_residual
+    from sse.time_integration import to_device, to_host
+    law, sd, _, _, ode = _line(NodalTensor(5), 7) if name == "line" else CASES[name]()
+    form = FluxDifferencingForm(inviscid_numerical_flux=LaxFriedrichsNumericalFlux())
+    solver = Solver(law, sd, form, parallelism=MI355X(deterministic=True))
+    d = law.d
+    state = np.ldexp(1.0, [a] + [a + c] * d + [a + 2 * c]).reshape(1, -1, 1)
+    flux = np.ldexp(1.0, [a + c] + [a + 2 * c] * d + [a + 3 * c]).reshape(1, -1, 1)
+
+    def residual(u0):
+        u = to_device(np.asfortranarray(u0))
+        du = torch.empty_like(u)
+        semi_discrete_residual(du, u, solver)
+        torch.cuda.synchronize()
+        return to_host(du)
+
+    got = residual(ode.u0)
+    assert solver.describe().startswith("generic"), solver.describe()
+    assert np.isfinite(got).all() and np.abs(got).max() > 0.0
+    assert np.array_equal(residual(ode.u0 * state), got * flux)
