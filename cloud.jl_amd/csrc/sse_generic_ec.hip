@@ -27,16 +27,24 @@
 // node its column of C), the S partial sums of a node added in turn; pairs are evaluated twice.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "sse_kernels.h"
 
 namespace sse {
 
 namespace {
 
-// Threads of a workgroup: 512 when an element has more than 256 nodes, volume and facet (one
-// node per thread in the first phase, at least two threads per volume node in the second),
-// else 256.
-__host__ __device__ constexpr int ec_threads(int nodes) { return nodes > 256 ? 512 : 256; }
+// Threads of a workgroup by the element's nodes, volume and facet: 512 above 256 (one node per
+// thread in the first phase, at least two threads per volume node in the second), else 256, and
+// fewer where most of 256 have nothing to do and only hold a place on the chip. ModalMulti,
+// 256 threads -> as here: Tri p = 2, 18 nodes, 800 elements 12.2 -> 10.1 us and 3,200 elements
+// 44.4 -> 31.3; Tri p = 4, 40 nodes, 3,200 elements 63.1 -> 49.2 (with 128 51.8); Tet p = 2, 63
+// nodes, 10,368 elements 174.8 -> 147.2; but Tet p = 3, 128 nodes, with 128 threads 18.2 -> 23.6
+// at 162 elements (223 -> 218 at 3,072).
+__host__ __device__ constexpr int ec_threads(int nodes) {
+    return nodes <= 40 ? 64 : nodes <= 64 ? 128 : nodes <= 256 ? 256 : 512;
+}
 
 // LDS of one element (doubles). The state area is dead after the flux phase and then holds
 // the partial sums and the transforms of the mass solve.
@@ -425,11 +433,17 @@ hipError_t launch_ec(const DevParams& p, const double* u, double* dudt, const RK
 template <int D>
 hipError_t launch_ec_d(const DevParams& p, const double* u, double* dudt, const RKStage& rk, const ErkTail& tail,
                        hipStream_t s) {
-    if (ec_threads(p.N_q + p.N_f) == 512)
-        return p.det ? launch_ec<D, 512, true>(p, u, dudt, rk, tail, s)
-                     : launch_ec<D, 512, false>(p, u, dudt, rk, tail, s);
-    return p.det ? launch_ec<D, 256, true>(p, u, dudt, rk, tail, s)
-                 : launch_ec<D, 256, false>(p, u, dudt, rk, tail, s);
+    auto run = [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
+        return p.det ? launch_ec<D, NT, true>(p, u, dudt, rk, tail, s)
+                     : launch_ec<D, NT, false>(p, u, dudt, rk, tail, s);
+    };
+    switch (ec_threads(p.N_q + p.N_f)) {
+        case 64: return run(std::integral_constant<int, 64>{});
+        case 128: return run(std::integral_constant<int, 128>{});
+        case 256: return run(std::integral_constant<int, 256>{});
+        default: return run(std::integral_constant<int, 512>{});
+    }
 }
 
 hipError_t launch_time_derivative_ec(const DevParams& p, const double* u, double* dudt, const RKStage& rk,

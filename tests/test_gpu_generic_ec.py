@@ -1,6 +1,6 @@
 """The general entropy-conservative time derivative (runtime-sized elements) at the edges of its
 work split, against the CPU oracle: more nodes than a 256-thread workgroup has threads (one
-thread per node, 512 threads), few nodes (many threads per node), even and odd counts (the
+thread per node, 512 threads), few nodes (workgroups of 64 and 128, many threads per node), even and odd counts (the
 half-way cyclic offset), sparse and dense operators, the atomic and the deterministic variant,
 and the Runge-Kutta stage combination in its epilogue for one, two and three stages.
 
@@ -42,7 +42,8 @@ CASES = {
     "line_257_nodes": lambda: _line(NodalTensor(256), 2),       # one thread per node, 512 threads
     "line_modal_p2": lambda: _line(ModalMulti(2), 5),           # 3 modes: 85 threads per node
     "tri_modal_p2": lambda: euler_vortex_2d_modal(M=3, p=2, approx=ModalMulti)[:5],
-    "tri_nodal_p5": lambda: euler_vortex_2d_modal(M=2, p=5, approx=NodalMulti)[:5],
+    "tri_nodal_p4": lambda: euler_vortex_2d_modal(M=2, p=4, approx=NodalMulti)[:5],  # 40 nodes: 64 threads
+    "tri_nodal_p5": lambda: euler_vortex_2d_modal(M=2, p=5, approx=NodalMulti)[:5],  # 54 nodes: 128
     "tet_modal_p2": lambda: density_wave_3d_config(M=1, p=2, approx=ModalMulti, ic_strength=0.2)[:5],
     "tet_modal_p4": lambda: density_wave_3d_config(M=1, p=4, approx=ModalMulti, ic_strength=0.2)[:5],
     "hex_p2": lambda: euler_3d_hex(M=2, p=2)[:5],
