@@ -380,7 +380,7 @@ struct EulerLines {
         constexpr int NQ = G::NQ;
         for (int t = threadIdx.x; t < E * NQ; t += TS) {
             const int s = t / NQ, i = t - s * NQ;
-            woj[s * NX + G::position(i)] = p.W[i] * rcp_refined(p.Jq[(size_t)element(s) * NQ + i]);
+            woj[s * NX + G::position(i)] = p.W[i] / p.Jq[(size_t)element(s) * NQ + i];
         }
     }
     __device__ double* line1(double* X) const { return X + c1 * NX + md1.base; }

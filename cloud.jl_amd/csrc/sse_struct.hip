@@ -481,7 +481,7 @@ __device__ __forceinline__ void time_derivative_body(const TensorParams& tp, con
             lift.template apply<NC>(tp.faces, tl, sff, r);
 #pragma unroll
             for (int e = 0; e < NC; ++e) sx[e * G::NX + G::position(tl)] = r[e];
-            woj[G::position(tl)] = Wi * rcp_refined(Ji);
+            woj[G::position(tl)] = Wi / Ji;
         }
         __syncthreads();
         // ---- phase F: dudt = M^{-1} V' r_q, line by line. M^{-1} = V' diag(W/J) V: the kept

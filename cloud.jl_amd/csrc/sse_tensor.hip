@@ -113,7 +113,7 @@ __device__ __forceinline__ void nodal_values_body(const TensorParams& tp, const 
         for (int e = 0; e < NC; ++e) ub[e] = x[e * NX];
         ok &= c2e_fast<D>(p.law, ub, wb);
         const double W = p.W[i], wj = W * J[q];
-        woj[s * NX + G::position(i)] = W * rcp_refined(J[q]);
+        woj[s * NX + G::position(i)] = W / J[q];
 #pragma unroll
         for (int e = 0; e < NC; ++e) x[e * NX] = wb[e] * wj;
     }
