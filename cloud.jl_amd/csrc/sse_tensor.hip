@@ -55,9 +55,13 @@ hipError_t launch_weight_adjusted_inverse(const DevParams& p, double* Mw, hipStr
 
 // ----------------------------------------------------------------------------- nodal_values
 // u_q = V u -> w = V' (WJ c2e(u_q)) -> M^{-1} w -> w_q = V w -> u_q = e2c(w_q), u_f = e2c(R w_q),
-// line by line (EulerLines), M^{-1} = V' (W/J V .) by the same transforms: a kept matrix per
-// element would be 38 % of this kernel's memory traffic at Tet p = 4, and a line's transform is
-// cheap. R is the ends of the lines and the interpolation on the faces (FaceTables).
+// line by line (EulerLines), M^{-1} = V' (W/J V .) by the same transforms from p = 4 on: a kept
+// matrix per element would be 38 % of this kernel's memory traffic at Tet p = 4, and a line's
+// transform is cheap. Up to p = 3 M^{-1} is the kept matrix where there is one: fewer roundings go
+// through e2c (error of the residual against 80-bit arithmetic, rms over 24 perturbed states, with
+// the transforms and with the matrix: Tet p = 2 4.4e-14 and 3.1e-14, Tet p = 3 4.4e-14 and 3.8e-14,
+// Tri p = 2 3.6e-14 and 2.9e-14; Tri p = 4 8.0e-14 with either form of the earlier kernels) at 2 % of
+// the residual's time on 16,464 Tet p = 3 elements (183 and 186 us). R is the ends of the lines and the interpolation on the faces (FaceTables).
 // With a node per thread (every multiply-add reading LDS, R in table rows) the whole residual
 // took 669 us at 24,576 Tet p = 4 elements and 42.3 us at 8,192 Tri p = 3, now 595 and 27.9 us.
 template <int ELEM, int P>
@@ -118,10 +122,52 @@ __device__ __forceinline__ void nodal_values_body(const TensorParams& tp, const 
         for (int e = 0; e < NC; ++e) x[e * NX] = wb[e] * wj;
     }
     __syncthreads();
+    // the kept matrix up to p = 3: a row of one element per PARTS neighbouring threads, requested early
+    constexpr bool KEPT = P <= 3;
+    constexpr int PARTS = E * NP * 4 <= TS ? 4 : E * NP * 2 <= TS ? 2 : 1, LEN = KEPT ? (NP + PARTS - 1) / PARTS : 1;
+    static_assert(!KEPT || E * NP <= TS, "a row per thread");
+    const int row = tl / PARTS, part = tl % PARTS, sm_ = min(row / NP, E - 1), jm = row % NP;
+    double mk[LEN];
+    if (KEPT && tp.Mw) {
+        const double* Mk = tp.Mw + (size_t)element(sm_) * NP * NP + jm;  // symmetric: row j as a column
+#pragma unroll
+        for (int q = 0; q < LEN; ++q) mk[q] = part + q * PARTS < NP ? Mk[(size_t)(part + q * PARTS) * NP] : 0.0;
+    }
     el.down3(X);
     el.down2(X);
-    el.turn1(X);
-    el.mass(X, woj);
+    if (KEPT && tp.Mw) {
+        double* y = es;  // NCOL x NP modal values
+        if (el.on1) {
+            double x[N1], m[N1];
+            line_load<N1, 1>(el.line1(X), x);
+            EL::LF::down1(F1, el.m1, x, m);
+#pragma unroll
+            for (int b = 0; b < N1; ++b)
+                if (b <= el.md1.lim) y[el.c1 * NP + el.md1.off + b] = m[b];
+        }
+        __syncthreads();
+        double s[NC];
+#pragma unroll
+        for (int e = 0; e < NC; ++e) {
+            s[e] = 0.0;
+#pragma unroll
+            for (int q = 0; q < LEN; ++q) s[e] += mk[q] * y[(sm_ * NC + e) * NP + min(part + q * PARTS, NP - 1)];
+#pragma unroll
+            for (int w = 1; w < PARTS; w <<= 1) s[e] += __shfl_xor(s[e], w, 64);
+        }
+        if (part == 0 && row < E * NP) {
+#pragma unroll
+            for (int e = 0; e < NC; ++e) X[(sm_ * NC + e) * NX + jm] = s[e];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < N1; ++b) um[b] = b <= el.md1.lim ? X[el.c1 * NX + el.md1.off + b] : 0.0;
+        __syncthreads();
+        el.up1(X, um);
+    } else {
+        el.turn1(X);
+        el.mass(X, woj);
+    }
     el.up2(X);
     double* ec = es + el.col * NF;
     el.up3(X, [&](const double* y) { line_ends<ELEM, P, 0>(tp.faces, y, el.line, ec); });  // w_q = V w
