@@ -425,13 +425,18 @@ int upload_lines(sse_handle* h, const sse_desc* D, sse::LineTables* lt) {
 }
 
 // R as line ends and an interpolation on each face (FaceTables). For each face the direction
-// along which its rows of R factorise, R_f[j, (t, a)] = M[j, t] w[a]; structured = false when a
-// face has none (to 1e-12 of its largest entry).
+// along which its rows of R factorise, R_f[j, (t, a)] = M[j, t] w[a], by least squares in extended
+// precision; structured = false when a face has none. The kernels then use the product, so it has
+// to be the caller's R to the rounding of its entries, FACE_TOL of the largest one: the factors of
+// the package's rules (Gauss and LGL facets, Tri p = 2..6, Tet p = 2..5) give their R exactly where
+// M = I and within 2e-16 elsewhere.
+constexpr double FACE_TOL = 8 * 2.220446049250313e-16;
+
 int upload_faces(sse_handle* h, const sse_desc* D, sse::FaceTables* ft, bool& structured) {
+    using real = long double;
     const int n1 = D->V_p + 1, d = D->d, nq = D->N_q, nf = D->N_f, nfac = D->N_fac, n2 = nq / n1;
     structured = false;
     if (nf != nfac * n2 || nfac > 4) return 0;
-    auto R = [&](int j, int i) { return D->R[j + (size_t)nf * i]; };
     std::vector<double> w((size_t)nfac * n1, 0.0), Pf((size_t)nfac * n1 * n1, 0.0);
     ft->general = 0;
     std::vector<std::vector<std::pair<int, double>>> mrows(nf), mtrows(nf);
@@ -440,58 +445,91 @@ int upload_faces(sse_handle* h, const sse_desc* D, sse::FaceTables* ft, bool& st
         for (int l = 0; l < d && !found; ++l) {
             int st = 1;
             for (int t = l + 1; t < d; ++t) st *= n1;
-            auto node = [&](int t, int a) { return (t / st) * st * n1 + a * st + t % st; };  // line t of direction l
-            int jm = 0, tm = 0;
-            double big = 0.0;  // the line with the largest entry gives w, scaled to sum 1
+            auto Rf = [&](int j, int t, int a) {  // at node a of line t of direction l
+                return D->R[f * n2 + j + (size_t)nf * ((t / st) * st * n1 + a * st + t % st)];
+            };
+            double big = 0.0;
+            int jm = 0, tm = 0;  // the line with the largest entry gives the first w
             for (int j = 0; j < n2; ++j)
                 for (int t = 0; t < n2; ++t)
                     for (int a = 0; a < n1; ++a)
-                        if (std::fabs(R(f * n2 + j, node(t, a))) > big) {
-                            big = std::fabs(R(f * n2 + j, node(t, a)));
+                        if (std::fabs(Rf(j, t, a)) > big) {
+                            big = std::fabs(Rf(j, t, a));
                             jm = j;
                             tm = t;
                         }
-            double sum = 0.0, sq = 0.0;
-            for (int a = 0; a < n1; ++a) sum += R(f * n2 + jm, node(tm, a));
-            if (big == 0.0 || std::fabs(sum) < 1e-8 * big) continue;
-            for (int a = 0; a < n1; ++a) {
-                w[(size_t)f * n1 + a] = R(f * n2 + jm, node(tm, a)) / sum;
-                sq += w[(size_t)f * n1 + a] * w[(size_t)f * n1 + a];
-            }
-            std::vector<double> M((size_t)n2 * n2, 0.0);
-            double worst = 0.0;
-            for (int j = 0; j < n2; ++j)
-                for (int t = 0; t < n2; ++t) {
-                    double m = 0.0;
-                    for (int a = 0; a < n1; ++a) m += R(f * n2 + j, node(t, a)) * w[(size_t)f * n1 + a];
-                    m /= sq;
-                    for (int a = 0; a < n1; ++a)
-                        worst = std::max(worst, std::fabs(R(f * n2 + j, node(t, a)) - m * w[(size_t)f * n1 + a]));
-                    M[(size_t)j * n2 + t] = m;
+            std::vector<real> v(n1), M((size_t)n2 * n2);
+            for (int a = 0; a < n1; ++a) v[a] = Rf(jm, tm, a);
+            auto solve_M = [&]() {
+                real sq = 0.0L;
+                for (int a = 0; a < n1; ++a) sq += v[a] * v[a];
+                for (int j = 0; j < n2; ++j)
+                    for (int t = 0; t < n2; ++t) {
+                        real m = 0.0L;
+                        for (int a = 0; a < n1; ++a) m += Rf(j, t, a) * v[a];
+                        M[(size_t)j * n2 + t] = m / sq;
+                    }
+            };
+            bool ok = big > 0.0;
+            for (int it = 0; it < 4 && ok; ++it) {  // v of sum 1, M for it, v for M
+                real sum = 0.0L;
+                for (int a = 0; a < n1; ++a) sum += v[a];
+                if (!(std::fabs(sum) > 1e-8L * big)) ok = false;
+                for (int a = 0; a < n1; ++a) v[a] /= sum;
+                if (!ok || it == 3) break;
+                solve_M();
+                real mm = 0.0L;
+                for (const real m : M) mm += m * m;
+                for (int a = 0; a < n1; ++a) {
+                    v[a] = 0.0L;
+                    for (int j = 0; j < n2; ++j)
+                        for (int t = 0; t < n2; ++t) v[a] += Rf(j, t, a) * M[(size_t)j * n2 + t] / mm;
                 }
-            if (worst > 1e-12 * big) continue;
+            }
+            if (!ok) continue;
+            for (int a = 0; a < n1; ++a) v[a] = (double)v[a];
+            solve_M();  // for the rounded w
+            // the rows as the product of u and the matrix m(j, t)?
+            auto fits = [&](const std::vector<double>& u, auto&& m) {
+                for (int j = 0; j < n2; ++j)
+                    for (int t = 0; t < n2; ++t)
+                        for (int a = 0; a < n1; ++a)
+                            if (!(std::fabs(Rf(j, t, a) - m(j, t) * u[a]) <= FACE_TOL * big)) return false;
+                return true;
+            };
+            std::vector<double> u(n1), P((size_t)n1 * n1, 0.0);
+            for (int a = 0; a < n1; ++a) {  // M = I: w is the mean row
+                real s = 0.0L;
+                for (int j = 0; j < n2; ++j) s += Rf(j, j, a);
+                u[a] = (double)(s / n2);
+            }
+            auto ident = [&](int j, int t) { return j == t ? 1.0 : 0.0; };
+            auto kron = [&](int j, int t) { return j / n1 == t / n1 ? P[(size_t)(j % n1) * n1 + t % n1] : 0.0; };
+            auto dense = [&](int j, int t) { return (double)M[(size_t)j * n2 + t]; };
+            int kind = fits(u, ident) ? 0 : -1;
+            if (kind < 0) {
+                for (int a = 0; a < n1; ++a) u[a] = (double)v[a];
+                for (int a = 0; a < n1; ++a)  // I x P: the mean of the diagonal blocks
+                    for (int b = 0; b < n1; ++b) {
+                        real s = 0.0L;
+                        for (int i = 0; i < n2; i += n1) s += M[(size_t)(i + a) * n2 + i + b];
+                        P[(size_t)a * n1 + b] = (double)(s * n1 / n2);
+                    }
+                kind = d == 3 && fits(u, kron) ? 1 : fits(u, dense) ? 2 : -1;
+            }
+            if (kind < 0) continue;
             found = true;
             ft->dir[f] = l;
-            // I, I x P or neither (to rounding: 1e-13 of the largest entry, which is about 1)
-            bool ident = true, kron = true;
+            ft->kind[f] = kind == 0 ? 0 : 1;
+            if (kind == 2) ft->general = 1;
+            std::copy(u.begin(), u.end(), w.begin() + (size_t)f * n1);
+            std::copy(P.begin(), P.end(), Pf.begin() + (size_t)f * n1 * n1);
             for (int j = 0; j < n2; ++j)
                 for (int t = 0; t < n2; ++t) {
-                    const double m = M[(size_t)j * n2 + t];
-                    const double p = j / n1 == t / n1 ? M[(size_t)(j % n1) * n2 + t % n1] : 0.0;
-                    if (std::fabs(m - (j == t ? 1.0 : 0.0)) > 1e-13) ident = false;
-                    if (std::fabs(m - p) > 1e-13) kron = false;
-                }
-            ft->kind[f] = ident ? 0 : 1;
-            if (!ident && (!kron || d == 2)) ft->general = 1;
-            for (int a = 0; a < n1; ++a)
-                for (int b = 0; b < n1; ++b) Pf[((size_t)f * n1 + a) * n1 + b] = M[(size_t)a * n2 + b];
-            for (int j = 0; j < n2; ++j)
-                for (int t = 0; t < n2; ++t) {
-                    double m = M[(size_t)j * n2 + t];
                     bool any = false;  // a zero block of R is no entry
-                    for (int a = 0; a < n1; ++a) any |= R(f * n2 + j, node(t, a)) != 0.0;
+                    for (int a = 0; a < n1; ++a) any |= Rf(j, t, a) != 0.0;
                     if (!any) continue;
-                    if (std::fabs(m - 1.0) < 4e-16) m = 1.0;
+                    const double m = kind == 0 ? ident(j, t) : kind == 1 ? kron(j, t) : dense(j, t);
                     mrows[f * n2 + j].push_back({f * n2 + t, m});
                     mtrows[f * n2 + t].push_back({f * n2 + j, m});
                 }
@@ -1353,18 +1391,19 @@ int sse_create(const sse_desc* D, sse_handle** out) { return create_handle(D, 1,
 int sse_describe(const sse_handle* h, char* buf, int32_t len) {
     if (!h || !buf || len <= 0) return SSE_ERR_INVALID_ARGUMENT;
     const DevParams& P = h->P;
+    auto faces = [](const sse::TensorParams& T) { return T.faces.general ? "general" : "lines"; };
     if (h->use_struct) {
         const sse::TensorParams& T = h->TP;
         const sse::StructTables& S = h->ST;
-        snprintf(buf, len, "struct elem=%d P=%d variant=%d blocks=%d items=%d ch=%d wrt=%d%s", T.elem, T.P, T.variant,
-                 h->struct_blocks, S.n_items, S.ch, T.wrt, S.det ? " deterministic" : "");
+        snprintf(buf, len, "struct elem=%d P=%d variant=%d blocks=%d items=%d ch=%d wrt=%d faces=%s%s", T.elem, T.P, T.variant,
+                 h->struct_blocks, S.n_items, S.ch, T.wrt, faces(T), S.det ? " deterministic" : "");
     } else if (h->use_tensor) {
         const sse::TensorParams& T = h->TP;
         snprintf(buf, len, "tensor elem=%d P=%d variant=%d pairs=%d vol_pairs=%d passes=%d pass_size=%d wv=%d wf=%d wrt=%d",
                  T.elem, T.P, T.variant, T.n_pairs, T.n_vol_pairs, T.n_pass, T.pass_size, T.wv, T.wf, T.wrt);
     } else if (h->use_std_tensor) {
-        snprintf(buf, len, "standard tensor elem=%d P=%d N_e=%d members=%d mapping=%s%s", h->TP.elem,
-                 h->TP.P, P.N_e, h->members, P.skew ? "skew" : "standard", P.second_order ? " br1" : "");
+        snprintf(buf, len, "standard tensor elem=%d P=%d N_e=%d members=%d mapping=%s%s faces=%s", h->TP.elem,
+                 h->TP.P, P.N_e, h->members, P.skew ? "skew" : "standard", P.second_order ? " br1" : "", faces(h->TP));
     } else if (P.standard) {
         snprintf(buf, len, "standard d=%d N_p=%d N_q=%d N_f=%d N_c=%d N_e=%d mapping=%s%s", P.d, P.N_p, P.N_q, P.N_f,
                  P.N_c, P.N_e, P.skew ? "skew" : "standard", P.second_order ? " br1" : "");

@@ -103,7 +103,10 @@ typedef struct sse_desc {
 
     /* reference-element operators, column-major */
     const double* V;            /* N_q x N_p Vandermonde; NULL = identity (nodal) */
-    const double* R;            /* N_f x N_q extrapolation */
+    const double* R;            /* N_f x N_q extrapolation. The line kernels of ModalTensor
+                                   Tri/Tet take an R that factorises along the lines of the
+                                   tensor grid to the rounding of its entries (Gauss, LGL and
+                                   similar facet rules); any other runs the general kernels */
     const int64_t* R_selection; /* N_f, 1-based volume node of each facet node for
                                    diagonal-E operators (SelectionMap), else NULL */
     const double* W;            /* N_q volume weights */
