@@ -83,9 +83,11 @@ SSE_STD_TUNE(ELEM_TET, 4, 256, 10, 256, 3)
 SSE_STD_TUNE(ELEM_TET, 5, 256, 7, 256, 2)
 #undef SSE_STD_TUNE
 
-// Waves per SIMD the registers must allow (one more spills at either size: Tet p = 5 at
-// 24,576 elements 395 us with 5, 438 us with 6).
-constexpr int std_waves(int P) { return P == 5 ? 5 : 6; }
+// Waves per SIMD the registers must allow. Lines of six and seven values take 81 to 94 registers,
+// which allow 5, on either element; with 6 (80 registers) those kernels spill: Tet p = 5 at 24,576
+// elements 395 us with 5, 438 with 6, Tri p = 6 at 28,800 elements 59 us with 5, 74 with 6. Up to
+// p = 4 the kernels fit 6.
+constexpr int std_waves(int P) { return P >= 5 ? 5 : 6; }
 
 namespace {
 
