@@ -51,7 +51,7 @@ def _citations():
                             (int(a), int(b) if b else int(a)) for a, b in ranges]
 
 
-@pytest.mark.skipif(not os.path.isdir(REFERENCE), reason="reference sources not mounted")
+@pytest.mark.skipif(not os.path.isdir(REFERENCE) or not os.listdir(REFERENCE), reason="reference sources not mounted")
 def test_every_reference_citation_resolves_inside_its_file():
     by_path, by_name = _reference_files()
     bad, count = [], 0
