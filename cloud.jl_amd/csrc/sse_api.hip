@@ -1346,15 +1346,23 @@ int create_handle(const sse_desc* D, int members, sse_handle** out) {
     }
     if (only_generic) h->use_tensor = false;
     if (!h->use_tensor) h->use_struct = false;
-    // the weight-adjusted mass solve with a kept matrix per element (N_p^2 doubles each; up to
-    // 16 GiB) in place of V, W/J and V' (SSE_MASS_MATRICES=0: off): the line-structured time
-    // derivative of small elements and the general entropy-conservative one
+    if (P.ec && !h->use_tensor && (rc = build_pairs(h, D))) return cleanup_fail(rc);
+    // The weight-adjusted mass solve with a kept matrix per element (N_p^2 doubles each) in place of
+    // V, W/J and V' (SSE_MASS_MATRICES=0: off): the line-structured kernels of small elements and the
+    // general entropy-conservative one. The kernels do without, so the matrices take at most 16 GiB
+    // and an eighth of the memory that is free (work buffers come later), and none if there is no
+    // such block.
     const bool keeps = h->use_tensor ? h->use_struct && sse::struct_keeps_mass(D->element, D->V_p) : P.ec != 0;
-    if (keeps && P.has_V && (size_t)N_p * N_p * N_e * sizeof(double) <= ((size_t)16 << 30)) {
-        const char* menv = getenv("SSE_MASS_MATRICES");
-        if (!(menv && menv[0] == '0')) {
-            double* Mw = nullptr;
-            if ((rc = alloc(h, (size_t)N_p * N_p * N_e, &Mw))) return cleanup_fail(rc);
+    const char* menv = getenv("SSE_MASS_MATRICES");
+    if (keeps && P.has_V && !(menv && menv[0] == '0')) {
+        const size_t bytes = (size_t)N_p * N_p * N_e * sizeof(double);
+        size_t room = 0, total = 0;
+        double* Mw = nullptr;
+        if (hipMemGetInfo(&room, &total) != hipSuccess || bytes > std::min(room / 8, (size_t)16 << 30) ||
+            alloc(h, (size_t)N_p * N_p * N_e, &Mw)) {
+            (void)hipGetLastError();  // clear the failure
+            h->err.clear();
+        } else {
             hipError_t e = sse::launch_weight_adjusted_inverse(P, Mw, nullptr);
             if (e == hipSuccess) e = hipDeviceSynchronize();
             if (e != hipSuccess) {
@@ -1365,7 +1373,6 @@ int create_handle(const sse_desc* D, int members, sse_handle** out) {
             else P.Mw = Mw;
         }
     }
-    if (P.ec && !h->use_tensor && (rc = build_pairs(h, D))) return cleanup_fail(rc);
     if (members > 1 && !h->use_std_tensor) {
         h->err = "an ensemble of problems needs the compiled StandardForm shapes of scalar laws";
         return cleanup_fail(SSE_ERR_UNSUPPORTED);
@@ -1395,8 +1402,8 @@ int sse_describe(const sse_handle* h, char* buf, int32_t len) {
     if (h->use_struct) {
         const sse::TensorParams& T = h->TP;
         const sse::StructTables& S = h->ST;
-        snprintf(buf, len, "struct elem=%d P=%d variant=%d blocks=%d items=%d ch=%d wrt=%d faces=%s%s", T.elem, T.P, T.variant,
-                 h->struct_blocks, S.n_items, S.ch, T.wrt, faces(T), S.det ? " deterministic" : "");
+        snprintf(buf, len, "struct elem=%d P=%d variant=%d blocks=%d items=%d ch=%d wrt=%d faces=%s mass=%s%s", T.elem, T.P, T.variant,
+                 h->struct_blocks, S.n_items, S.ch, T.wrt, faces(T), T.Mw ? "kept" : "transforms", S.det ? " deterministic" : "");
     } else if (h->use_tensor) {
         const sse::TensorParams& T = h->TP;
         snprintf(buf, len, "tensor elem=%d P=%d variant=%d pairs=%d vol_pairs=%d passes=%d pass_size=%d wv=%d wf=%d wrt=%d",
@@ -1408,8 +1415,9 @@ int sse_describe(const sse_handle* h, char* buf, int32_t len) {
         snprintf(buf, len, "standard d=%d N_p=%d N_q=%d N_f=%d N_c=%d N_e=%d mapping=%s%s", P.d, P.N_p, P.N_q, P.N_f,
                  P.N_c, P.N_e, P.skew ? "skew" : "standard", P.second_order ? " br1" : "");
     } else {
-        snprintf(buf, len, "generic d=%d N_p=%d N_q=%d N_f=%d N_c=%d N_e=%d%s%s", P.d, P.N_p, P.N_q, P.N_f, P.N_c,
-                 P.N_e, P.mfma ? " nodal_values=mfma" : "", P.det ? " deterministic" : "");
+        snprintf(buf, len, "generic d=%d N_p=%d N_q=%d N_f=%d N_c=%d N_e=%d%s%s%s", P.d, P.N_p, P.N_q, P.N_f, P.N_c,
+                 P.N_e, P.mfma ? " nodal_values=mfma" : "", !P.ec || !P.has_V ? "" : P.Mw ? " mass=kept" : " mass=transforms",
+                 P.det ? " deterministic" : "");
     }
     return 0;
 }
@@ -1680,7 +1688,9 @@ int sse_rk_adjoint(sse_handle* h, const double* u0, double dt, int32_t nsteps, i
            *stages = nullptr, *p1 = nullptr;
     {  // the block to keep: what this call needs with both segment buffer sets, if within ADJ_KEEP
         const size_t q = (size_t)h->P.N_q * h->P.N_c * h->P.N_e, f = (size_t)h->P.N_f * h->P.N_c * h->P.N_e;
-        const size_t stage = (h->vjp_tensor ? q + 2 * f : 0) + n, sets = h->vjp_tensor && nseg > 1 ? 2 : 1;
+        const char* env = getenv("SSE_ADJ_OVERLAP");
+        const bool two = h->vjp_tensor && nseg > 1 && !(env && env[0] == '0');
+        const size_t stage = (h->vjp_tensor ? q + 2 * f : 0) + n, sets = two ? 2 : 1;
         const size_t need = (n * (7 + (size_t)nseg) + stage * 5 * (size_t)seglen * sets) * sizeof(double) + 16 * 256;
         if (need <= ADJ_KEEP && need > h->adj_ws_bytes) {
             if (h->adj_ws) (void)hipFree(h->adj_ws);  // waits for earlier work that reads it
@@ -2021,8 +2031,10 @@ int sse_erk_steps(sse_handle* h, double* u, double t0, double dt, int32_t nsteps
                 return fail(h, SSE_ERR_INVALID_ARGUMENT, "A must be strictly lower triangular (an explicit method)");
     const size_t n = state_size(h);
     int rc;
-    if (h->erk_stages < stages) {  // stage derivatives and two stage states (kept for later calls)
-        if ((rc = alloc(h, (size_t)(stages + 2) * n, &h->erk_k))) return rc;
+    // nodal diagonal-E schemes: see `fused` below
+    const bool direct = h->P.ec && !h->use_tensor && h->P.sel && !h->P.has_V;
+    if (h->erk_stages < stages) {  // stage derivatives and one or two stage states (kept for later calls)
+        if ((rc = alloc(h, (size_t)(stages + (direct ? 2 : 1)) * n, &h->erk_k))) return rc;
         h->erk_stages = stages;
     }
     double* K = h->erk_k;
@@ -2053,7 +2065,7 @@ int sse_erk_steps(sse_handle* h, double* u, double t0, double dt, int32_t nsteps
     // residual also forms the next stage's state, in its epilogue. Two stage states take turns,
     // because other workgroups still read the current one; a single-stage method would update
     // u while it is read.
-    const bool fused = h->P.ec && !h->use_tensor && h->P.sel && !h->P.has_V && stages > 1;
+    const bool fused = direct && stages > 1;
     for (int step = 0; step < nsteps; ++step) {
         if (fused) {
             for (int i = 0; i < stages; ++i) {

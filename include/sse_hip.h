@@ -184,7 +184,8 @@ int sse_rk_steps(sse_handle* h, double* u, double t0, double dt, int32_t nsteps,
  * With the Dormand-Prince 8(5,3) tableau this replaces solve(ode, DP8(),
  * adaptive=false, dt=dt) of the reference's 3D Euler test (test/euler_3d.jl:45-53).
  * The stage states are combined on the device (one kernel per stage); the library
- * keeps stages + 1 state-sized buffers on the handle. A and b are host arrays. */
+ * keeps stages + 1 state-sized buffers on the handle (one more for nodal diagonal-E
+ * schemes). A and b are host arrays. */
 int sse_erk_steps(sse_handle* h, double* u, double t0, double dt, int32_t nsteps, int32_t stages,
                   const double* A, const double* b, int32_t where);
 
@@ -219,7 +220,8 @@ int sse_residual_vjp(sse_handle* h, const double* u, const double* ybar, double*
  * kernels, the recomputation runs on a second stream of the library's beside the
  * reverse sweep, and the forward sweep keeps its last two segments (environment
  * SSE_ADJ_OVERLAP=0: one stream, the last segment kept). No counterpart in the
- * reference. u0 and grad_u0 are device or host per `where`. Blocks. */
+ * reference. u0 and grad_u0 are device or host per `where`. Blocks. The handle keeps up
+ * to 1 GiB of the call's work memory for the next call, until sse_destroy. */
 int sse_rk_adjoint(sse_handle* h, const double* u0, double dt, int32_t nsteps, int32_t checkpoint_every,
                    int32_t objective, double* J, double* grad_u0, double* grad_lambda, int32_t where);
 
