@@ -2172,6 +2172,7 @@ struct sse_batch {
     std::vector<hipEvent_t> join;
     hipEvent_t fork = nullptr;
     int* any_status = nullptr;  // the groups' status words, combined
+    int device = 0;             // the one that was current when the batch was created
     std::string err;
 };
 
@@ -2299,7 +2300,19 @@ __global__ void __launch_bounds__(64) k_any_status(StatusWords w, int* any) {
     if (t < w.n && *w.word[t]) atomicOr(any, 1);
 }
 
-hipError_t batch_move(sse_batch* b, double* const* u, const double* dt, bool states, bool back) {
+// Memory that a kernel of the batch may read and write: the batch's own device's. Other states that
+// a caller passes as device memory (another device's, the host's) are copied by the runtime.
+bool movable(const sse_batch* b, const void* p) {
+    hipPointerAttribute_t a = {};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();  // memory that the runtime does not know
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == b->device && !a.isManaged;
+}
+
+// moved[i]: problem i's state too, else its time steps only
+hipError_t batch_move(sse_batch* b, double* const* u, const double* dt, const std::vector<char>& moved, bool back) {
     Moves m = {};
     hipError_t e = hipSuccess;
     int* any = b->any_status;  // cleared by the first launch
@@ -2314,7 +2327,8 @@ hipError_t batch_move(sse_batch* b, double* const* u, const double* dt, bool sta
     for (size_t g = 0; g < b->groups.size(); ++g)
         for (size_t t = 0; t < b->members[g].size(); ++t) {
             const int i = b->members[g][t], q = m.n;
-            m.user[q] = states ? u[i] : nullptr;
+            if (back && !moved[i]) continue;
+            m.user[q] = moved[i] ? u[i] : nullptr;
             m.group[q] = b->state[g] + b->per_elem[i] * b->offsets[g][t];
             m.len[q] = b->per_elem[i] * b->elems[i];
             m.dt_e[q] = b->dt_e[g] + b->offsets[g][t];
@@ -2408,7 +2422,8 @@ int sse_batch_create(const sse_desc* const* descs, int32_t n, sse_batch** out) {
         b->elems[i] = descs[i]->N_e;
         b->per_elem[i] = (size_t)descs[i]->N_p * descs[i]->N_c;
     }
-    if (hipStreamCreate(&b->stream) != hipSuccess) return cleanup(SSE_ERR_HIP, "hipStreamCreate failed");
+    if (hipGetDevice(&b->device) != hipSuccess || hipStreamCreate(&b->stream) != hipSuccess)
+        return cleanup(SSE_ERR_HIP, "hipStreamCreate failed");
     if (hipMalloc(&b->any_status, sizeof(int)) != hipSuccess) return cleanup(SSE_ERR_OUT_OF_MEMORY, "hipMalloc failed");
     // ensembles first: StandardForm scalar problems on one mesh that differ at most in b
     std::vector<std::vector<int>> ens;
@@ -2539,17 +2554,20 @@ int sse_batch_rk_steps(sse_batch* b, double* const* u, const double* dt, int32_t
     int rc;
     // gather states and per-element time steps into the group buffers
     const bool device = where == SSE_DEVICE;
+    std::vector<char> moved(b->elems.size(), 0);
     for (size_t g = 0; g < b->groups.size(); ++g)
         for (size_t t = 0; t < b->members[g].size(); ++t) {
             const int i = b->members[g][t];
             if (!u[i]) return bfail(b, SSE_ERR_INVALID_ARGUMENT, "u[" + std::to_string(i) + "] is NULL");
-            if (device) continue;
+            moved[i] = device && movable(b, u[i]);
+            if (moved[i]) continue;
             const size_t n_i = b->per_elem[i] * b->elems[i];
             if ((rc = hip_ok(hipMemcpyAsync(b->state[g] + b->per_elem[i] * b->offsets[g][t], u[i],
-                                            n_i * sizeof(double), hipMemcpyHostToDevice, b->stream), "state gather")))
+                                            n_i * sizeof(double), device ? hipMemcpyDefault : hipMemcpyHostToDevice,
+                                            b->stream), "state gather")))
                 return rc;
         }
-    if ((rc = hip_ok(batch_move(b, u, dt, device, false), "state gather"))) return rc;
+    if ((rc = hip_ok(batch_move(b, u, dt, moved, false), "state gather"))) return rc;
     // units of work that do not depend on each other: a group, or the triangle groups that share
     // their launches (all of them under the first one's number)
     const std::vector<size_t> tri = tri_groups(b);
@@ -2622,19 +2640,17 @@ int sse_batch_rk_steps(sse_batch* b, double* const* u, const double* dt, int32_t
     for (; step < nsteps; ++step)
         if ((rc = one_step())) return rc;
     // scatter back
-    if (device) {
-        if ((rc = hip_ok(batch_move(b, u, dt, true, true), "state scatter"))) return rc;
-    } else {
-        for (size_t g = 0; g < b->groups.size(); ++g)
-            for (size_t t = 0; t < b->members[g].size(); ++t) {
-                const int i = b->members[g][t];
-                const size_t n_i = b->per_elem[i] * b->elems[i];
-                if ((rc = hip_ok(hipMemcpyAsync(u[i], b->state[g] + b->per_elem[i] * b->offsets[g][t],
-                                                n_i * sizeof(double), hipMemcpyDeviceToHost, b->stream),
-                                 "state scatter")))
-                    return rc;
-            }
-    }
+    if ((rc = hip_ok(batch_move(b, u, dt, moved, true), "state scatter"))) return rc;
+    for (size_t g = 0; g < b->groups.size(); ++g)
+        for (size_t t = 0; t < b->members[g].size(); ++t) {
+            const int i = b->members[g][t];
+            if (moved[i]) continue;
+            const size_t n_i = b->per_elem[i] * b->elems[i];
+            if ((rc = hip_ok(hipMemcpyAsync(u[i], b->state[g] + b->per_elem[i] * b->offsets[g][t],
+                                            n_i * sizeof(double), device ? hipMemcpyDefault : hipMemcpyDeviceToHost,
+                                            b->stream), "state scatter")))
+                return rc;
+        }
     // a non-physical state in any group: then each group's own check names it
     for (size_t g0 = 0; g0 < b->groups.size(); g0 += 64) {
         StatusWords w = {};

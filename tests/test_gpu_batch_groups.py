@@ -81,3 +81,30 @@ def test_more_problems_than_one_move(host):
     for (s, u0, dt), u in zip(probs, states):
         want = O.rk_steps(s.arrays, u0, dt, 3)
         assert np.abs((u if host else to_host(u)) - want).max() <= 1e-10 * np.abs(want).max()
+
+
+def test_states_in_memory_of_other_kinds():
+    """States passed as device memory that the batch's kernels do not move: pinned and pageable host
+    memory (as a copy by the runtime takes it), beside states on the device."""
+    import ctypes as C
+
+    import torch
+    from sse import abi
+    from sse.batch import BatchedSolver
+    from sse.time_integration import to_device, to_host
+    probs = [_problem("tri", 2 + i % 3, 1 + i % 2) for i in range(5)]
+    batch = BatchedSolver([s for s, _, _ in probs])
+    on_device = [to_device(u0) for _, u0, _ in probs]
+    states = list(on_device)
+    states[1] = torch.empty(on_device[1].shape, dtype=torch.float64, pin_memory=True).copy_(on_device[1])
+    states[2] = on_device[2].cpu()
+    torch.cuda.synchronize()
+    ptrs = (C.c_void_p * 5)(*[x.data_ptr() for x in states])
+    dt = np.array([dt for _, _, dt in probs])
+    for n in (1, 2):
+        code = batch.lib.sse_batch_rk_steps(batch.handle, ptrs, dt.ctypes.data_as(C.POINTER(C.c_double)), n,
+                                            abi.SSE_DEVICE, 1)
+        assert code == 0, batch.lib.sse_batch_last_error(batch.handle)
+    for (s, u0, dt_), x in zip(probs, states):
+        want = O.rk_steps(s.arrays, u0, dt_, 3)
+        assert np.abs(to_host(x.cuda()) - want).max() <= 1e-10 * np.abs(want).max()
