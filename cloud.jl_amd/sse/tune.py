@@ -2,11 +2,12 @@
 
 libsse_hip compiles, per (element type, degree), a few kernel configurations:
 the kernel family of the time derivative (line-structured, table-driven pairs,
-runtime-shaped generic) and, for the tensor kernels, launch-shape variants
-(threads per element, elements per workgroup, pairs per thread of the
-projection and pair kernels). A configuration is chosen when a handle is
-created, from ``SSE_KERNELS`` (``tensor`` or ``generic``; unset = the fastest
-family the shape has) and ``SSE_TENSOR_VARIANT``.
+runtime-shaped generic) and, for the table-driven pair kernel, launch-shape
+variants (threads per element, elements per workgroup, pairs per thread). The
+projection and the line-structured kernels have one launch shape each. A
+configuration is chosen when a handle is created, from ``SSE_KERNELS``
+(``tensor`` or ``generic``; unset = the fastest family the shape has) and
+``SSE_TENSOR_VARIANT``.
 
 ``autotune(solver, u)`` creates one handle per configuration on the solver's
 arrays (``Solver.with_law`` shares them), times the residual with HIP events on
@@ -28,9 +29,10 @@ from typing import List, Optional
 
 from .solvers import Solver
 
-# launch-shape variants compiled for some (element, degree) shapes; a variant that
-# a shape lacks falls back to variant 0, and duplicates are dropped by description
-MAX_VARIANT = 5
+# launch-shape variants of the table-driven pair kernel compiled for some (element, degree)
+# shapes; a variant that a shape lacks falls back to variant 0, and duplicates are dropped by
+# description
+MAX_VARIANT = 3
 FAMILIES = ("struct", "tensor", "generic")
 
 
@@ -86,7 +88,7 @@ def autotune(solver: Solver, u, nrep: int = 20, check_tol: float = 1e-12) -> Lis
     seen = set()
     ref = None
     for family in FAMILIES:
-        variants = [None] if family == "generic" else list(range(MAX_VARIANT))
+        variants = list(range(MAX_VARIANT)) if family == "tensor" else [None]
         for v in variants:
             with _selection(family, v):
                 s = solver.with_law(solver.conservation_law)

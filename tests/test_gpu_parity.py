@@ -828,6 +828,9 @@ def test_autotune_times_every_configuration_and_selects_one(make, monkeypatch):
     timings = tune.autotune(ode.p, u, nrep=3)
     assert len(timings) >= 2 and all(t.total_ms > 0 for t in timings)
     assert len({t.describe for t in timings}) == len(timings)
+    # only the table-driven pair kernel has launch shapes to choose from
+    assert all(t.variant is None for t in timings if t.family != "tensor")
+    assert [t.family for t in timings].count("struct") == 1
     tune.select(timings[0])
     fresh = ode.p.with_law(ode.p.conservation_law)
     assert fresh.describe() == timings[0].describe
