@@ -2747,11 +2747,13 @@ int sse_batch_rk_tangent(sse_batch* b, double* const* u, double* const* v, const
 int sse_batch_describe(const sse_batch* b, char* buf, int32_t len) {
     if (!b || !buf || len <= 0) return SSE_ERR_INVALID_ARGUMENT;
     std::string out = "batch groups=" + std::to_string(b->groups.size());
+    const std::vector<size_t> tri = tri_groups(b);
     for (size_t g = 0; g < b->groups.size(); ++g) {
         char one[256];
         sse_describe(b->groups[g], one, sizeof(one));
         out += " | " + std::to_string(b->members[g].size()) + (b->chunk[g] ? " problems on one mesh" : " problems") +
                ", N_e=" + std::to_string(b->groups[g]->P.N_e) + ": " + one;
+        if (std::find(tri.begin(), tri.end(), g) != tri.end()) out += " shared launches";
     }
     snprintf(buf, len, "%s", out.c_str());
     return 0;

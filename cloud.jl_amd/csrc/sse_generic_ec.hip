@@ -18,8 +18,9 @@
 //   * every volume pair belongs to one of its two nodes (host-balanced; consecutive nodes have
 //     partners at the same cyclic offset, so that the atomic adds of a wavefront go to
 //     different rows); the S threads of a node take every S-th entry of its lists;
-//   * 1/2 nJq (the reference normal of each face in the metric of each volume node) is formed
-//     once per node and face, not once per pair;
+//   * nJq (the reference normal of each face in the metric of each volume node) is formed once
+//     per node and face, not once per pair (the mean of the two normals and the halved
+//     contraction vector are the factor of the table's C_ij / 4);
 //   * V' r - V' R' f_f is one product with the stacked operator [V; -R V]' over the volume and
 //     facet nodes, and the weight-adjusted mass solve one product with the element's kept
 //     V' diag(W/J) V (V, W/J, V' where it is not kept).
@@ -56,7 +57,7 @@ struct EcLayout {
         h = 0;                                            // NH x N_q hoisted volume states
         hf = h + NH * p.N_q;                              // NH x N_f hoisted facet states and
         L = hf + (corr ? (NH + p.d) * p.N_f : 0);         // d x N_f scaled normals (facet correction)
-        nq = L + p.d * p.d * p.N_q;                       // N_fac x d x N_q: nJq / 2 (facet correction)
+        nq = L + p.d * p.d * p.N_q;                       // N_fac x d x N_q: nJq (facet correction)
         const int states = nq + (corr ? p.N_fac * p.d * p.N_q : 0);
         part = 0;                                         // partial sums [part][c][mode] of the products,
         const int n_part = nt / p.N_p > 1 ? nt / p.N_p : 1;
@@ -198,7 +199,8 @@ __global__ void __launch_bounds__(EC_NT)
         }
         ec_dot_h<D>(p.law, hi, hj, av, c);
     };
-    // a/2 of a facet pair, a = C_ij (nJ_f,j + nJq_i of j's face) / 2; cq = C_ij / 4
+    // a/2 of a facet pair, a = C_ij (nJ_f,j + nJq_i of j's face) / 2; cq = C_ij / 4, so the sum
+    // of the two normals comes in unscaled
     auto facet_flux = [&](const double* hi, int i, int j, double cq, double* c) {
         double hj[NH], av[D];
         const int f = j / npf;

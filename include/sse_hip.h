@@ -334,7 +334,8 @@ int sse_batch_rk_steps(sse_batch* b, double* const* u, const double* dt, int32_t
 int sse_batch_rk_tangent(sse_batch* b, double* const* u, double* const* v, const double* dt, int32_t nsteps,
                          int32_t where);
 
-/* One-line description of the groups (count, elements, kernel family). */
+/* One-line description of the groups (count, elements, kernel family, and which of them share
+ * the launches of their Runge-Kutta stages). */
 int sse_batch_describe(const sse_batch* b, char* buf, int32_t len);
 
 /* Message of the last failure on b (or of the last failed sse_batch_create when b is NULL). */

@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(autouse=True)
 def _default_kernels(monkeypatch):
     monkeypatch.delenv("SSE_KERNELS", raising=False)  # another test's choice of kernels
+    monkeypatch.delenv("SSE_BATCH_BRANCHES", raising=False)
 
 
 def _problem(elem, p, M, flux="lf", det=False):
@@ -36,6 +37,8 @@ def _problem(elem, p, M, flux="lf", det=False):
     return s, u0, 0.05 * (2.0 / M) / ((2 * p + 1) * 3.0)
 
 
+# problems, and how many groups of them share their launches
+SHARED = {"every degree": 5, "two degrees": 2, "one degree": 0, "with others": 3}
 BATCHES = {
     "every degree": [("tri", p, M) for p, M in ((2, 3), (3, 1), (4, 3), (5, 1), (6, 3), (3, 5))],
     "two degrees": [("tri", 6, 1), ("tri", 2, 1)],
@@ -53,6 +56,7 @@ def test_rk_steps(name, graph):
     from sse.time_integration import to_device, to_host
     probs = [_problem(*c) for c in BATCHES[name]]
     batch = BatchedSolver([s for s, _, _ in probs])
+    assert batch.describe().count("shared launches") == SHARED[name], batch.describe()
     states = [to_device(u0) for _, u0, _ in probs]
     for n in (3, 1, 2):  # captured in the first call and replayed in the third
         batch.rk_steps(states, [dt for _, _, dt in probs], n, use_graph=graph)

@@ -44,8 +44,19 @@ def _problem(elem, p, M, lgl=False):
 
 
 CASES = [("tri", 2, 3, False), ("tri", 3, 3, False), ("tri", 4, 2, False), ("tri", 5, 3, False), ("tri", 6, 1, False),
-         ("tri", 4, 2, True), ("tet", 2, 1, False), ("tet", 3, 1, False), ("tet", 4, 1, False), ("tet", 5, 1, False),
+         ("tri", 2, 3, True), ("tri", 4, 2, True), ("tet", 2, 1, False), ("tet", 3, 1, False), ("tet", 4, 1, False), ("tet", 5, 1, False),
          ("tet", 3, 1, True)]
+
+
+def _check_family(s, elem, p, lgl):
+    """The line kernels, with general face rows for LGL facets of Tri p = 2. Where a volume node meets
+    more than ten facet nodes (LGL from p = 3 on) the general kernels run."""
+    if not lgl:
+        assert s.describe().startswith("struct") and "faces=lines" in s.describe(), s.describe()
+    elif (elem, p) == ("tri", 2):
+        assert s.describe().startswith("struct") and "faces=general" in s.describe(), s.describe()
+    else:
+        assert s.describe().startswith("generic"), s.describe()
 
 
 @pytest.mark.parametrize("elem,p,M,lgl", CASES)
@@ -58,6 +69,7 @@ def test_residual(elem, p, M, lgl):
     du = torch.empty_like(u)
     semi_discrete_residual(du, u, s)
     torch.cuda.synchronize()
+    _check_family(s, elem, p, lgl)
     sd = s.spatial_discretization
     rows = max(np.abs(np.asarray(Dm)).sum(1).max() for Dm in sd.reference_approximation.D)
     bar = 4 * np.finfo(float).eps / 2e-2 * rows / sd.geometric_factors.J_q.min() * np.abs(u0).max()
@@ -71,6 +83,7 @@ def test_pull_back(elem, p, M, lgl):
     rng = np.random.default_rng(6)
     du, y = (np.asfortranarray(rng.standard_normal(u0.shape)) for _ in range(2))
     ubar, lam = residual_vjp(s, u0, y)
+    _check_family(s, elem, p, lgl)
     _, jv = O.residual_jvp(s.arrays, u0, du, 0.7)
     a, b = float((ubar * du).sum()) + 0.7 * lam, float((y * jv).sum())
     assert abs(a - b) <= 1e-11 * float(np.abs(y * jv).sum())

@@ -72,6 +72,7 @@ def test_residual(elem, p, M, b, skew, lgl):
     semi_discrete_residual(du, u, s)
     torch.cuda.synchronize()
     assert s.describe().startswith("standard tensor"), s.describe()
+    assert s.describe().endswith("faces=general" if lgl else "faces=lines"), s.describe()
     assert _rel(to_host(du), O.residual(s.arrays, u0)) <= 1e-12
 
 
