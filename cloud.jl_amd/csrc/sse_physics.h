@@ -190,7 +190,7 @@ template <int D>
 struct ElementUnits {
     int a, c;
     __device__ __forceinline__ void set(const LawParams& P, const double* u) {
-        const double rho = u[0], irho = rcp_refined(rho);
+        const double rho = u[0], irho = __builtin_amdgcn_rcp(rho);  // only the exponents count
         double s = 0.0;
 #pragma unroll
         for (int m = 0; m < D; ++m) {
