@@ -220,7 +220,7 @@ k_nodal_values_tensor(TensorParams tp, const double* __restrict__ u) {
 // Triangles of several degrees in one launch: each degree alone leaves most of the chip idle,
 // and branches of a graph overlap only in part (24 problems of degrees 2 to 6, 7,468 triangles:
 // 133 us per RK stage one after the other, 72 us in five branches, 55 us in one launch of each
-// kernel: 17 us here and 38 us for the time derivative, 1.5 rounds of its 5 wavefronts per SIMD).
+// kernel: 17 us here and 38 us for the time derivative, 1.8 rounds of its 4 wavefronts per SIMD).
 __global__ void __launch_bounds__(64) k_nodal_values_tri_groups(TriGroups a) {
     static_assert(K1Layout<ELEM_TRI, 2>::size * 8 <= 65536 && K1Layout<ELEM_TRI, 6>::size * 8 <= 65536,
                   "LDS without an attribute");
