@@ -423,9 +423,9 @@ template <int D, int NT, bool DET>
 hipError_t launch_ec(const DevParams& p, const double* u, double* dudt, const RKStage& rk, const ErkTail& tail,
                      hipStream_t s) {
     const size_t lds = lds_time_derivative_ec(p);
-    if (lds > 64 * 1024) {
+    if (lds > 64 * 1024) {  // the same limit from every handle and thread
         const hipError_t e = hipFuncSetAttribute((const void*)k_time_derivative_ec<D, NT, DET>,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL((k_time_derivative_ec<D, NT, DET>), dim3(p.N_e), dim3(NT), lds, s, p, u, dudt, rk, tail);

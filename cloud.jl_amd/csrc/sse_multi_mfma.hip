@@ -213,14 +213,14 @@ hipError_t launch_nodal_values_mfma(const DevParams& p, const double* u, hipStre
     switch (p.d) {
         case 2: {
             const hipError_t e = hipFuncSetAttribute((const void*)k_nodal_values_mfma<2, LAW_EULER>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL((k_nodal_values_mfma<2, LAW_EULER>), grid, block, lds, s, p, u);
             break;
         }
         case 3: {
             const hipError_t e = hipFuncSetAttribute((const void*)k_nodal_values_mfma<3, LAW_EULER>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL((k_nodal_values_mfma<3, LAW_EULER>), grid, block, lds, s, p, u);
             break;
