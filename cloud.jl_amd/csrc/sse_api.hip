@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <cstddef>
@@ -1636,8 +1637,29 @@ int sse_residual_vjp(sse_handle* h, const double* u, const double* ybar, double*
     return check_status(h);
 }
 
-// work memory of sse_rk_adjoint that a handle keeps between calls
-static constexpr size_t ADJ_KEEP = (size_t)1 << 30;
+// work memory of sse_rk_adjoint that a handle keeps between calls, and that all handles of the
+// process keep together: a program with many handles holds no more than that
+static constexpr size_t ADJ_KEEP = (size_t)1 << 30, ADJ_KEEP_ALL = (size_t)4 << 30;
+static std::atomic<size_t> adj_kept_all{0};
+
+// h's block grown to `bytes` (its contents are lost), or none if the limits or the memory do not allow it
+static void keep_adjoint_block(sse_handle* h, size_t bytes) {
+    if (bytes > ADJ_KEEP || bytes <= h->adj_ws_bytes) return;
+    const size_t more = bytes - h->adj_ws_bytes;
+    if (adj_kept_all.fetch_add(more) + more > ADJ_KEEP_ALL) {
+        adj_kept_all.fetch_sub(more);
+        return;
+    }
+    if (h->adj_ws) (void)hipFree(h->adj_ws);  // waits for earlier work that reads it
+    h->adj_ws = nullptr;
+    h->adj_ws_bytes = bytes;
+    if (hipMalloc(&h->adj_ws, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        h->adj_ws = nullptr;
+        h->adj_ws_bytes = 0;
+        adj_kept_all.fetch_sub(bytes);
+    }
+}
 
 int sse_rk_adjoint(sse_handle* h, const double* u0, double dt, int32_t nsteps, int32_t checkpoint_every,
                    int32_t objective, double* J, double* grad_u0, double* grad_lambda, int32_t where) {
@@ -1652,7 +1674,7 @@ int sse_rk_adjoint(sse_handle* h, const double* u0, double dt, int32_t nsteps, i
     const int nseg = (nsteps + checkpoint_every - 1) / checkpoint_every;
     const int seglen = nsteps < checkpoint_every ? nsteps : checkpoint_every;
     // Work buffers: allocated for the call and freed at its end, except that up to ADJ_KEEP bytes
-    // stay with the handle for the next call (allocating and freeing 600 MB took 1.3 of the 10.4 ms
+    // (ADJ_KEEP_ALL over all handles) stay with the handle for the next call (allocating and freeing 600 MB took 1.3 of the 10.4 ms
     // of a 20-step gradient on 1,296 Tet p = 3 elements). They are carved from that block in turn.
     std::vector<void*> mine;
     size_t ws_used = 0;
@@ -1693,17 +1715,7 @@ int sse_rk_adjoint(sse_handle* h, const double* u0, double dt, int32_t nsteps, i
         const bool two = h->vjp_tensor && nseg > 1 && !(env && env[0] == '0');
         const size_t stage = (h->vjp_tensor ? q + 2 * f : 0) + n, sets = two ? 2 : 1;
         const size_t need = (n * (7 + (size_t)nseg) + stage * 5 * (size_t)seglen * sets) * sizeof(double) + 16 * 256;
-        if (need <= ADJ_KEEP && need > h->adj_ws_bytes) {
-            if (h->adj_ws) (void)hipFree(h->adj_ws);  // waits for earlier work that reads it
-            h->adj_ws = nullptr;
-            h->adj_ws_bytes = 0;
-            if (hipMalloc(&h->adj_ws, need) == hipSuccess) {
-                h->adj_ws_bytes = need;
-            } else {  // the call then allocates piece by piece
-                (void)hipGetLastError();
-                h->adj_ws = nullptr;
-            }
-        }
+        keep_adjoint_block(h, need);  // without one, the call allocates piece by piece
     }
     if ((rc = dalloc(n, &u)) || (rc = dalloc(n, &ktmp)) || (rc = dalloc(n, &ub)) || (rc = dalloc(n, &kb)) ||
         (rc = dalloc(n, &vb)) || (rc = dalloc(n * (size_t)(nseg > 0 ? nseg : 1), &ckpt)) ||
@@ -2142,6 +2154,7 @@ void sse_destroy(sse_handle* h) {
     if (h->rk_graph) (void)hipGraphDestroy(h->rk_graph);
     for (void* p : h->allocations) (void)hipFree(p);
     if (h->adj_ws) (void)hipFree(h->adj_ws);
+    adj_kept_all.fetch_sub(h->adj_ws_bytes);
     if (h->own_stream) (void)hipStreamDestroy(h->own_stream);
     if (h->adj_stream) (void)hipStreamDestroy(h->adj_stream);
     delete h;

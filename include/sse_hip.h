@@ -221,7 +221,8 @@ int sse_residual_vjp(sse_handle* h, const double* u, const double* ybar, double*
  * reverse sweep, and the forward sweep keeps its last two segments (environment
  * SSE_ADJ_OVERLAP=0: one stream, the last segment kept). No counterpart in the
  * reference. u0 and grad_u0 are device or host per `where`. Blocks. The handle keeps up
- * to 1 GiB of the call's work memory for the next call, until sse_destroy. */
+ * to 1 GiB of the call's work memory for the next call, until sse_destroy (all handles of a
+ * process together up to 4 GiB; further ones keep none). */
 int sse_rk_adjoint(sse_handle* h, const double* u0, double dt, int32_t nsteps, int32_t checkpoint_every,
                    int32_t objective, double* J, double* grad_u0, double* grad_lambda, int32_t where);
 

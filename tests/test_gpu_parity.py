@@ -631,6 +631,32 @@ def test_kept_mass_matrices_leave_memory_to_the_rest(monkeypatch):
     assert float((a - b).abs().max()) <= RES_TOL * float(a.abs().max())
 
 
+def test_adjoint_work_memory_kept_by_many_handles_is_bounded():
+    # each gradient below takes 0.8 GiB of work memory, of which its handle keeps a block for the next
+    # call: seven handles keep at most 4 GiB together (with 0.5 GiB for the handles themselves), give
+    # the same gradients from a kept block and without one, and give it back when they are closed
+    from sse.adjoint import rk_adjoint
+    from sse.solvers import MI355X, Solver
+    torch = _gpu()
+    law, sd, ic, form, ode = density_wave_3d_config(M=4, p=3, ic_strength=0.2)[:5]
+    free = lambda: torch.cuda.mem_get_info()[0]  # noqa: E731
+    handles, grads = [], []
+    before = None
+    for _ in range(8):
+        s = Solver(law, sd, form, parallelism=MI355X(deterministic=True))
+        grads.append(rk_adjoint(s, ode.u0, 1e-3, 50, checkpoint_every=25)[1])
+        if before is None:  # the first one also loads the kernels
+            s.close()
+            before = free()
+        else:
+            handles.append(s)
+    assert before - free() <= int(4.5 * (1 << 30))
+    assert all(np.array_equal(g, grads[0]) for g in grads)
+    for s in handles:
+        s.close()
+    assert before - free() <= 1 << 29
+
+
 def test_rk_steps_graph_replay_matches_eager_and_oracle(monkeypatch):
     # sse_rk_steps replays one captured step; a new state pointer or a new dt recaptures
     from sse.time_integration import rk_steps, to_device, to_host
