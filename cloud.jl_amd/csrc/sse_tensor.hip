@@ -125,7 +125,7 @@ __device__ __forceinline__ void nodal_values_body(const TensorParams& tp, const 
     // the kept matrix up to p = 3: a row of one element per PARTS neighbouring threads, requested early
     constexpr bool KEPT = P <= 3;
     constexpr int PARTS = E * NP * 4 <= TS ? 4 : E * NP * 2 <= TS ? 2 : 1, LEN = KEPT ? (NP + PARTS - 1) / PARTS : 1;
-    static_assert(!KEPT || E * NP <= TS, "a row per thread");
+    static_assert(!KEPT || (E * NP <= TS && NP <= NF), "a row per thread, the modal values in place of the line ends");
     const int row = tl / PARTS, part = tl % PARTS, sm_ = min(row / NP, E - 1), jm = row % NP;
     double mk[LEN];
     if (KEPT && tp.Mw) {
