@@ -37,14 +37,23 @@ namespace sse {
 namespace {
 
 // Threads of a workgroup by the element's nodes, volume and facet: 512 above 256 (one node per
-// thread in the first phase, at least two threads per volume node in the second), else 256, and
-// fewer where most of 256 have nothing to do and only hold a place on the chip. ModalMulti,
-// 256 threads -> as here: Tri p = 2, 18 nodes, 800 elements 12.2 -> 10.1 us and 3,200 elements
-// 44.4 -> 31.3; Tri p = 4, 40 nodes, 3,200 elements 63.1 -> 49.2 (with 128 51.8); Tet p = 2, 63
-// nodes, 10,368 elements 174.8 -> 147.2; but Tet p = 3, 128 nodes, with 128 threads 18.2 -> 23.6
-// at 162 elements (223 -> 218 at 3,072).
-__host__ __device__ constexpr int ec_threads(int nodes) {
-    return nodes <= 40 ? 64 : nodes <= 64 ? 128 : nodes <= 256 ? 256 : 512;
+// thread in the first phase, at least two threads per volume node in the second), else 256. With
+// fewer nodes most of 256 threads have nothing to do; that only matters once the elements are more
+// than a round of such workgroups, and with fewer threads a node's lists take longer. ModalMulti, us
+// per residual with 256 | 128 | 64 threads:
+//   Tri p = 2, 18 nodes:    242 elements 19.9 | 19.6 | 19.8    1,568 35.9 | 32.9 | 32.5   3,200 54.1 | 47.9 | 44.5
+//   Tri p = 3, 28 nodes:    450 elements 21.6 | 22.0 | 22.7    1,568 35.6 | 34.3 | 34.7   3,200 53.8 | 49.6 | 47.4
+//   Tri p = 4, 40 nodes:    450 elements 24.4 | 25.5 | 28.5      800 25.7 | 25.3 | 30.5   3,200 70.2 | 64.7 | 66.7
+//   Tri p = 5, 54 nodes:    450 elements 27.1 | 31.2 | 41.3    1,800 61.3 | 63.9 | 77.7
+//   Tet p = 2, 63 nodes:  1,296 elements 48.3 | 49.8 | 52.4    4,374 108  | 101  | 110
+//   Tet p = 3, 128 nodes:   162 elements 18.2 | 23.6
+// (of residuals that overlap on several streams 800 Tri p = 2 elements 12.2 | 10.1 | 10.1, 3,200 Tri
+// p = 4 elements 63.1 | 51.8 | 49.2).
+__host__ __device__ constexpr int ec_threads(int nodes, int N_e) {
+    if (nodes <= 20) return 64;
+    if (nodes <= 40) return N_e > 3 * 256 ? 128 : 256;   // three workgroups per compute unit
+    if (nodes <= 64) return N_e > 12 * 256 ? 128 : 256;  // twelve
+    return nodes <= 256 ? 256 : 512;
 }
 
 // LDS of one element (doubles). The state area is dead after the flux phase and then holds
@@ -52,7 +61,7 @@ __host__ __device__ constexpr int ec_threads(int nodes) {
 struct EcLayout {
     int h, hf, L, nq, acc, part, o, size;
     __host__ __device__ EcLayout(const DevParams& p) {
-        const int NH = p.d + 5, NC = p.d + 2, nt = ec_threads(p.N_q + p.N_f);
+        const int NH = p.d + 5, NC = p.d + 2, nt = ec_threads(p.N_q + p.N_f, p.N_e);
         const bool corr = p.C_kind != 0;
         h = 0;                                            // NH x N_q hoisted volume states
         hf = h + NH * p.N_q;                              // NH x N_f hoisted facet states and
@@ -440,7 +449,7 @@ hipError_t launch_ec_d(const DevParams& p, const double* u, double* dudt, const 
         return p.det ? launch_ec<D, NT, true>(p, u, dudt, rk, tail, s)
                      : launch_ec<D, NT, false>(p, u, dudt, rk, tail, s);
     };
-    switch (ec_threads(p.N_q + p.N_f)) {
+    switch (ec_threads(p.N_q + p.N_f, p.N_e)) {
         case 64: return run(std::integral_constant<int, 64>{});
         case 128: return run(std::integral_constant<int, 128>{});
         case 256: return run(std::integral_constant<int, 256>{});

@@ -1,6 +1,6 @@
 """The general entropy-conservative time derivative (runtime-sized elements) at the edges of its
 work split, against the CPU oracle: more nodes than a 256-thread workgroup has threads (one
-thread per node, 512 threads), few nodes (workgroups of 64 and 128, many threads per node), even and odd counts (the
+thread per node, 512 threads), few nodes (workgroups of 64, and of 128 on many elements), even and odd counts (the
 half-way cyclic offset), sparse and dense operators, the atomic and the deterministic variant,
 and the Runge-Kutta stage combination in its epilogue for one, two and three stages.
 
@@ -42,8 +42,8 @@ CASES = {
     "line_257_nodes": lambda: _line(NodalTensor(256), 2),       # one thread per node, 512 threads
     "line_modal_p2": lambda: _line(ModalMulti(2), 5),           # 3 modes: 85 threads per node
     "tri_modal_p2": lambda: euler_vortex_2d_modal(M=3, p=2, approx=ModalMulti)[:5],
-    "tri_nodal_p4": lambda: euler_vortex_2d_modal(M=2, p=4, approx=NodalMulti)[:5],  # 40 nodes: 64 threads
-    "tri_nodal_p5": lambda: euler_vortex_2d_modal(M=2, p=5, approx=NodalMulti)[:5],  # 54 nodes: 128
+    "tri_nodal_p4": lambda: euler_vortex_2d_modal(M=2, p=4, approx=NodalMulti)[:5],  # 40 nodes: 256 threads
+    "tri_nodal_p5": lambda: euler_vortex_2d_modal(M=2, p=5, approx=NodalMulti)[:5],
     "tet_modal_p2": lambda: density_wave_3d_config(M=1, p=2, approx=ModalMulti, ic_strength=0.2)[:5],
     "tet_modal_p4": lambda: density_wave_3d_config(M=1, p=4, approx=ModalMulti, ic_strength=0.2)[:5],
     "hex_p2": lambda: euler_3d_hex(M=2, p=2)[:5],
@@ -127,3 +127,25 @@ def test_residual_does_not_depend_on_the_units(name, a, c):
     assert solver.describe().startswith("generic"), solver.describe()
     assert np.isfinite(got).all() and np.abs(got).max() > 0.0
     assert np.array_equal(residual(ode.u0 * state), got * flux)
+
+
+@pytest.mark.parametrize("det", [False, True], ids=["atomic", "deterministic"])
+@pytest.mark.parametrize("make,problems", [
+    (lambda: euler_vortex_2d_modal(M=4, p=4, approx=ModalMulti), 25),                      # 40 nodes, 800 elements
+    (lambda: density_wave_3d_config(M=2, p=2, approx=ModalMulti, ic_strength=0.2), 65),    # 63 nodes, 3,120
+], ids=["tri_p4", "tet_p2"])
+def test_workgroups_of_128_on_many_elements(make, problems, det):
+    """Many small problems in one batch are one mesh of enough elements for smaller workgroups."""
+    from sse.batch import BatchedSolver
+    from sse.time_integration import to_device, to_host
+    law, sd, _, form, ode = make()[:5]
+    solver = Solver(law, sd, form, parallelism=MI355X(deterministic=det))
+    batch = BatchedSolver([solver] * problems)
+    assert f"N_e={problems * sd.N_e}" in batch.describe(), batch.describe()
+    starts = [np.asfortranarray(ode.u0 * (1.0 + 1e-3 * np.random.default_rng(r).standard_normal(ode.u0.shape)))
+              for r in range(3)]
+    u = [to_device(starts[i % 3]) for i in range(problems)]
+    batch.rk_steps(u, [1e-3] * problems, 2)
+    refs = [O.rk_steps(solver.arrays, x, 1e-3, 2) for x in starts]
+    worst = max(_rel(to_host(x), refs[i % 3]) for i, x in enumerate(u))
+    assert worst <= 1e-10
