@@ -151,6 +151,10 @@ __global__ void __launch_bounds__(EC_NT)
         } else {
             const int j = t - N_q;
             const int g = p.mapP[j + (size_t)N_f * k];
+            const double jf = p.Jf[j + (size_t)N_f * k], bj = p.B[j] * jf;
+            double nJ[D];
+#pragma unroll
+            for (int m = 0; m < D; ++m) nJ[m] = p.nJf[D * (j + (size_t)N_f * k) + m];
             const int kn = g / N_f, jn = g - kn * N_f;
             double uin[NC], uout[NC], hin[NH], hout[NH], nrm[D], c[NC];
             if (direct) {
@@ -175,8 +179,7 @@ __global__ void __launch_bounds__(EC_NT)
             units.in(uout);
             hoist<D>(p.law, uin, hin);
             hoist<D>(p.law, uout, hout);
-            const double jf = p.Jf[j + (size_t)N_f * k], inv_jf = 1.0 / jf;
-            const double* nJ = p.nJf + D * (j + (size_t)N_f * k);
+            const double inv_jf = 1.0 / jf;
 #pragma unroll
             for (int m = 0; m < D; ++m) nrm[m] = nJ[m] * inv_jf;
             if (corr) {
@@ -186,7 +189,6 @@ __global__ void __launch_bounds__(EC_NT)
                 for (int m = 0; m < D; ++m) snJ[m * N_f + j] = nJ[m];
             }
             ec_dot<D>(p.law, hin, hout, nrm, c);
-            const double bj = p.B[j] * jf;
             const double al =
                 p.law.inviscid_flux == 1 ? p.law.half_lambda * wave_speed_h<D>(p.law, hin, hout, nrm) : 0.0;
 #pragma unroll
